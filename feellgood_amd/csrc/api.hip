@@ -476,7 +476,10 @@ void build_plan(Ctx &c, const fg_mesh *m)
     c.corr = dalloc<double2>(N);
     c.src_pos = dalloc<double4>(c.S);
     upload(c.src_pos, spos, st);
-    c.src_q = dalloc<double2>(c.S);
+    // the direct sum's partial potentials follow the charges in one allocation
+    const bool direct = c.opt.demag_method != FG_DEMAG_FMM;
+    c.src_q = dalloc<double2>(c.S + (direct ? (size_t)p2p_shares(c) * N : 0));
+    if (direct) c.p2p_part = c.src_q + c.S;
     std::vector<int64_t> rank(c.S);
     for (int64_t k = 0; k < c.S; k++) rank[k] = k;
     c.src_rank = dalloc<int64_t>(c.S);

@@ -124,6 +124,7 @@ struct Ctx {
     double4 *src_pos = nullptr;  // [S] in tree order when the FMM is used
     int64_t *src_rank = nullptr; // [S] source index (5 per magnetic tet, 4 per charged tri) -> slot
     double2 *src_q = nullptr;    // [S] (q from u, q from v)
+    double2 *p2p_part = nullptr; // FG_DEMAG_DIRECT: [shares][N] partial potentials (u, v) of the direct sum
     float4 *src_pos_f = nullptr; // FP32 copies for the mixed-precision P2P
     double2 *qe = nullptr;       // [Tm + 3 Fm] element charge values for the FMM near-field operator:
                                  // -Ms div u per tetrahedron, u_a . n per triangle vertex (u, v)
@@ -193,6 +194,7 @@ void launch_update(Ctx &c, double dt, bool gated = false);
 void launch_spmv_debug(Ctx &c, double c_stencil, const double2 *xin, double2 *yout);
 void launch_charges(Ctx &c);
 void launch_direct_p2p(Ctx &c);
+int p2p_shares(const Ctx &c);  // shares of the sources of the direct sum
 void launch_energy(Ctx &c, const double Hext[3], const double *hsp = nullptr, double amp = 0);
 // c.hst from the node spin accumulation c.spin_s and the per-region prefactors c.spin_pref
 void launch_spin_field(Ctx &c);

@@ -18,6 +18,7 @@
 // it and projects back, reading 12 bytes per stored entry instead of a 2x2 FP64 block.
 #include "ctx.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace fg {
@@ -1417,70 +1418,142 @@ __global__ __launch_bounds__(BLOCK) void k_corr_gather(int N, const int32_t *__r
     }
 }
 
+// 1/sqrt(x) in FP64: the hardware approximation (about 24 correct bits) and one third-order step
+// y (1 + e/2 + 3 e^2 / 8), e = 1 - x y^2, whose error 5 e^3 / 16 is below the rounding: five
+// operations against the IEEE square root and division sequences (about 30). x > 0.
+__device__ inline double rsqrt_f64(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // Exact potentials phi_i = (sum_s q_s / |x_i - y_s| + corr_i) / (4 pi) (src/fmm_demag.h:211-223),
-// FP64, sources staged through LDS in tiles of BLOCK. In a batch (node_inst != nullptr) a node
-// sees only its own instance's sources: tetrahedron sources [r.x, r.y), triangle sources [r.z, r.w)
-// with r = inst_src[instance].
-__global__ __launch_bounds__(BLOCK) void k_p2p_direct(int N, int64_t S, const int32_t *__restrict__ mag,
-                                                      const double4 *__restrict__ pos4,
+// FP64. Bound by FP64 VALU issue: 13 operations and one quarter-rate rsq per pair. A block holds
+// P2P_TPT targets per thread and one of nsplit shares of the sources (staged through LDS, read by
+// broadcast: two targets per thread halve the LDS reads per pair), so that a mesh of a few thousand
+// nodes still fills the 256 CUs; the shares' partial sums go to part[share][node] and
+// k_p2p_finish adds them in a fixed order (deterministic). For 6,468 targets x 1.5e5 sources a step
+// takes 1.0 ms, 0.5 ms of it this sum; with a block of 256 targets running all sources alone (26
+// blocks on the chip) and 1.0 / sqrt, the sum took 15.5 ms.
+// In a batch (node_inst != nullptr) a node sees only its own instance's sources: tetrahedron sources
+// [r.x, r.y), triangle sources [r.z, r.w) with r = inst_src[instance]; a block runs the two ranges
+// that its nodes' instances (consecutive) span and tests each source only where they are several.
+template <int TPT>
+__global__ __launch_bounds__(BLOCK) void k_p2p_direct(int N, int64_t S, int nsplit, const double4 *__restrict__ pos4,
                                                       const double4 *__restrict__ spos,
-                                                      const double2 *__restrict__ q,
-                                                      const double2 *__restrict__ corr, NodeRec *__restrict__ nxt,
+                                                      const double2 *__restrict__ q, double2 *__restrict__ part,
                                                       const int32_t *__restrict__ node_inst,
                                                       const longlong4 *__restrict__ inst_src)
 {
-    __shared__ double4 ts[BLOCK];
-    __shared__ double2 tq[BLOCK];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool act = i < N && mag[i];
-    double4 xi = make_double4(0, 0, 0, 0);
-    if (i < N) xi = pos4[i];
-    longlong4 r = make_longlong4(0, S, 0, 0);
-    if (node_inst && i < N) r = inst_src[node_inst[i]];
-    double pu = 0, pv = 0;
-    for (int64_t base = 0; base < S; base += BLOCK) {
-        const int64_t k = base + threadIdx.x;
-        if (k < S) {
-            ts[threadIdx.x] = spos[k];
-            tq[threadIdx.x] = q[k];
-        } else {
-            ts[threadIdx.x] = make_double4(1e30, 1e30, 1e30, 0);
-            tq[threadIdx.x] = make_double2(0, 0);
+    __shared__ double4 ts[BLOCK];  // x, y, z, q of u
+    __shared__ double tv[BLOCK];   // q of v
+    const int tb = blockIdx.x / nsplit, sp = blockIdx.x - tb * nsplit;
+    const int n0 = tb * BLOCK * TPT;
+    // the block's source ranges [a0, a1) and [b0, b1), addressed as one list of len indices
+    int64_t a0 = 0, a1 = S, b0 = 0, b1 = 0;
+    bool mixed = false;
+    if (node_inst) {
+        const int i0 = node_inst[n0], i1 = node_inst[min(n0 + BLOCK * TPT, N) - 1];
+        a0 = inst_src[i0].x;
+        a1 = inst_src[i1].y;
+        b0 = inst_src[i0].z;
+        b1 = inst_src[i1].w;
+        mixed = i0 != i1;
+    }
+    const int64_t la = a1 - a0, len = la + (b1 - b0);
+    // shares in whole chunks of 64 sources
+    const int64_t units = (len + 63) / 64;
+    const int64_t k0 = units * sp / nsplit * 64, k1 = min(len, units * (sp + 1) / nsplit * 64);
+    double4 xi[TPT];
+    longlong4 r[TPT];
+    double pu[TPT], pv[TPT];
+#pragma unroll
+    for (int h = 0; h < TPT; h++) {
+        const int i = min(n0 + h * BLOCK + (int)threadIdx.x, N - 1);
+        xi[h] = pos4[i];
+        if (mixed) r[h] = inst_src[node_inst[i]];
+        pu[h] = pv[h] = 0;
+    }
+    for (int64_t base = k0; base < k1; base += BLOCK) {
+        const int cnt = (int)min((int64_t)BLOCK, k1 - base), cnt4 = (cnt + 3) & ~3;
+        const int t = threadIdx.x;
+        if (t < cnt) {
+            const int64_t k = base + t, s = k < la ? a0 + k : b0 + (k - la);
+            const double4 y = spos[s];
+            const double2 qq = q[s];
+            ts[t] = make_double4(y.x, y.y, y.z, qq.x);
+            tv[t] = qq.y;
+        } else if (t < cnt4) {  // padding: far away, no charge
+            ts[t] = make_double4(1e30, 1e30, 1e30, 0);
+            tv[t] = 0;
         }
         __syncthreads();
-        if (act) {
-            const bool all = (base >= r.x && base + BLOCK <= r.y) || (base >= r.z && base + BLOCK <= r.w);
-            if (all) {
-#pragma unroll 8
-                for (int j = 0; j < BLOCK; j++) {
-                    const double4 y = ts[j];
-                    const double dx = xi.x - y.x, dy = xi.y - y.y, dz = xi.z - y.z;
-                    const double ir = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
-                    const double2 qq = tq[j];
-                    pu += qq.x * ir;
-                    pv += qq.y * ir;
+        if (!mixed) {
+#pragma unroll 4
+            for (int j = 0; j < cnt4; j++) {
+                const double4 y = ts[j];
+                const double qv = tv[j];
+#pragma unroll
+                for (int h = 0; h < TPT; h++) {
+                    const double dx = xi[h].x - y.x, dy = xi[h].y - y.y, dz = xi[h].z - y.z;
+                    const double ir = rsqrt_f64(dx * dx + dy * dy + dz * dz);
+                    pu[h] += y.w * ir;
+                    pv[h] += qv * ir;
                 }
-            } else {
-                for (int j = 0; j < BLOCK; j++) {
-                    const int64_t s = base + j;
-                    if (!((s >= r.x && s < r.y) || (s >= r.z && s < r.w))) continue;
-                    const double4 y = ts[j];
-                    const double dx = xi.x - y.x, dy = xi.y - y.y, dz = xi.z - y.z;
-                    const double ir = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
-                    const double2 qq = tq[j];
-                    pu += qq.x * ir;
-                    pv += qq.y * ir;
+            }
+        } else {
+            for (int j = 0; j < cnt; j++) {
+                const int64_t k = base + j, s = k < la ? a0 + k : b0 + (k - la);
+                const double4 y = ts[j];
+                const double qv = tv[j];
+#pragma unroll
+                for (int h = 0; h < TPT; h++) {
+                    if (!((s >= r[h].x && s < r[h].y) || (s >= r[h].z && s < r[h].w))) continue;
+                    const double dx = xi[h].x - y.x, dy = xi[h].y - y.y, dz = xi[h].z - y.z;
+                    const double ir = rsqrt_f64(dx * dx + dy * dy + dz * dz);
+                    pu[h] += y.w * ir;
+                    pv[h] += qv * ir;
                 }
             }
         }
         __syncthreads();
     }
-    if (act) {
+#pragma unroll
+    for (int h = 0; h < TPT; h++) {
+        const int i = n0 + h * BLOCK + (int)threadIdx.x;
+        if (i < N) part[(size_t)sp * N + i] = make_double2(pu[h], pv[h]);
+    }
+}
+
+// The shares' sums of each magnetic node, 32 nodes per block with eight threads each (a strided
+// share of the partials, then in a fixed order through LDS), plus the vertex corrections.
+constexpr int P2P_FIN = 32;
+__global__ __launch_bounds__(BLOCK) void k_p2p_finish(int N, int nsplit, const int32_t *__restrict__ mag,
+                                                      const double2 *__restrict__ part,
+                                                      const double2 *__restrict__ corr, NodeRec *__restrict__ nxt)
+{
+    __shared__ double2 sh[BLOCK / P2P_FIN][P2P_FIN];
+    const int l = threadIdx.x % P2P_FIN, g = threadIdx.x / P2P_FIN;
+    const int i = blockIdx.x * P2P_FIN + l;
+    double pu = 0, pv = 0;
+    if (i < N)
+#pragma unroll 4
+        for (int s = g; s < nsplit; s += BLOCK / P2P_FIN) {
+            const double2 p = part[(size_t)s * N + i];
+            pu += p.x;
+            pv += p.y;
+        }
+    sh[g][l] = make_double2(pu, pv);
+    __syncthreads();
+    if (g == 0 && i < N && mag[i]) {
+        for (int k = 1; k < BLOCK / P2P_FIN; k++) {
+            pu += sh[k][l].x;
+            pv += sh[k][l].y;
+        }
         const double2 c = corr[i];
-        NodeRec r = nxt[i];
-        r.phi = (pu + c.x) / (4 * M_PI);
-        r.phiv = (pv + c.y) / (4 * M_PI);
-        nxt[i] = r;
+        nxt[i].phi = (pu + c.x) / (4 * M_PI);
+        nxt[i].phiv = (pv + c.y) / (4 * M_PI);
     }
 }
 
@@ -1880,11 +1953,27 @@ void launch_charges(Ctx &c)
     k_corr_gather<<<c.blocks_for(c.N), BLOCK, 0, c.stream>>>(c.N, c.cinc_ptr, c.cinc_idx, c.tri_corr, c.corr);
 }
 
+// Targets per thread and shares of the sources of the direct sum: about 2,048 blocks (eight per CU)
+// and at least 64 sources per share. Two targets per thread once a block of 512 is full.
+static int p2p_tpt(const Ctx &c) { return c.N > 2 * BLOCK ? 2 : 1; }
+int p2p_shares(const Ctx &c)
+{
+    const int64_t nt = (c.N + BLOCK * p2p_tpt(c) - 1) / (BLOCK * p2p_tpt(c));
+    return (int)std::max<int64_t>(1, std::min<int64_t>((2048 + nt - 1) / nt, (c.S + 63) / 64));
+}
+
 void launch_direct_p2p(Ctx &c)
 {
     Prof pr(c, "p2p_direct");
-    k_p2p_direct<<<grid1(c.N), BLOCK, 0, c.stream>>>(c.N, c.S, c.mag, c.pos4, c.src_pos, c.src_q, c.corr,
-                                                     c.rec[1 - c.cur], c.d_node_inst, c.d_inst_src);
+    const int ns = p2p_shares(c), tpt = p2p_tpt(c), nb = (c.N + BLOCK * tpt - 1) / (BLOCK * tpt) * ns;
+    if (tpt == 2)
+        k_p2p_direct<2><<<nb, BLOCK, 0, c.stream>>>(c.N, c.S, ns, c.pos4, c.src_pos, c.src_q, c.p2p_part, c.d_node_inst,
+                                                    c.d_inst_src);
+    else
+        k_p2p_direct<1><<<nb, BLOCK, 0, c.stream>>>(c.N, c.S, ns, c.pos4, c.src_pos, c.src_q, c.p2p_part, c.d_node_inst,
+                                                    c.d_inst_src);
+    k_p2p_finish<<<(c.N + P2P_FIN - 1) / P2P_FIN, BLOCK, 0, c.stream>>>(c.N, ns, c.mag, c.p2p_part, c.corr,
+                                                                        c.rec[1 - c.cur]);
 }
 
 void launch_energy(Ctx &c, const double Hext[3], const double *hsp, double amp)
