@@ -90,18 +90,15 @@ struct FmmPlan {
     int64_t *d_lc_ptr = nullptr;  // [ntl+1] shared column list of each such leaf
     int32_t *d_lc_col = nullptr;
     double2 *d_pot = nullptr;  // [T] near-field + correction potential
-    double2 *d_far = nullptr;  // [T] multipole (far) part of the potential, M2P's output
+    double2 *d_far = nullptr;  // M2P's partial sums of the multipole (far) part of the potentials
     int32_t *d_tgt_lc = nullptr;  // [T] local-expansion cell of each target's group (-1: none)
     float *d_nf_valf = nullptr;  // FP32 coefficients (mixed precision; d_nf_val is then released)
     bool mixed = false;
     double mscale = 1.0;         // expansions times mscale (a power of two) in the FP32 mode
     int64_t m2p_pairs = 0, m2l_pairs = 0, lc_cols = 0;
     int64_t m2p_slots = 0, m2p_far_pairs = 0;  // lane slots the M2P launch mapping executes (useful pairs / slots = SIMD efficiency)
-    // M2P launches: the groups of more than M2P_HALF_MAX targets (one cell per row), then the
-    // smaller ones (one cell per half row)
-    std::vector<int32_t> m2p_gid;
-    int m2p_n1 = 0;
-    int32_t *d_m2p_gid = nullptr;
+    int m2p_ntask = 0;  // M2P tasks (m2p_tasks) and the partial sums of every target
+    int4 *d_m2p_task = nullptr, *d_tgt_far = nullptr;
     int64_t nf_nnz = 0;
     int32_t *d_tgt_node = nullptr;
     double4 *d_tgt_pos = nullptr;
@@ -858,7 +855,7 @@ __global__ __launch_bounds__(64) void k_fmm_p2m(int nleaf, int Tm, const int32_t
             const int o = p2m_col_off<P>(MASK, m);
 #pragma unroll
             for (int n = m; n <= P; n++) {
-                const F sc = (F)p2m_scale(n, m);
+                const F sc = (F)(p2m_scale(n, m) * fmm_stored(n));
                 const int i = 2 * (o + n - m);
                 du[2 * fidx(n, m)] = au[i] * sc;
                 du[2 * fidx(n, m) + 1] = au[i + 1] * sc;
@@ -939,7 +936,7 @@ template <> struct Mfma<float> {
 template <int P> struct XL {
     static constexpr int NCo = fcount(P), NR = 2 * NCo, NT = (NR + 15) / 16, NKS = (NR + 3) / 4;
     static constexpr int frag_len() { return 8 * NT * NKS * 64; }
-    static constexpr int deg(int j)
+    __host__ __device__ static constexpr int deg(int j)
     {
         int n = 0;
         while (fidx(n + 1, 0) <= (j >> 1)) n++;
@@ -1362,54 +1359,27 @@ __global__ __launch_bounds__(256) void k_nf_apply(int ntl, const int32_t *__rest
     }
 }
 
-// Far field: multipole-to-target evaluation (M2P) per evaluation group, one wavefront per group.
-// The wavefront's four rows of 16 lanes are (target row, cell slot) pairs: with nt targets in the
-// current chunk of at most 64, nr = ceil(nt / 16) rows cover the targets and cps = 4 / nr cells
-// of the group's list are evaluated at once, one per slot. A row holds its cell's two expansions
-// in VGPRs (row-broadcast layout below), loaded at each step; every product with a coefficient is
-// a DPP row-broadcast fused multiply-add, so no lane re-reads the coefficients from memory or LDS.
-// Entries from u_far[g] on are evaluated to degree PF. The cell slots of each target are summed in
-// slot order, then the L2P of the group's level-(L-2) ancestor is added and phi, phi_v are
-// written.
-
-// Row-broadcast fused multiply-add: acc += c[lane L of this lane's row of 16] * x, through DPP
-// row_newbcast on src0 of v_fmac_f64 / v_fmac_f32 (gfx950), written only in the lanes of the banks
-// (groups of 4 lanes of a row) set in BM. Rules for the callers: EXEC is full wherever these run
-// (the broadcasting lane must be active), and a VALU write of a coefficient register is separated
-// from its first DPP read by row_fence (two wait states).
-template <int L, int BM = 15>
-__device__ __forceinline__ void fmac_row(double &acc, double c, double x)
-{
-    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:%4"
-        : "+v"(acc)
-        : "v"(c), "v"(x), "i"(L), "i"(BM));
-}
-template <int L, int BM = 15>
-__device__ __forceinline__ void fmac_row(float &acc, float c, float x)
-{
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:%4"
-        : "+v"(acc)
-        : "v"(c), "v"(x), "i"(L), "i"(BM));
-}
-// acc += (coefficient double K of this lane's cell) * x. H = 1: one cell per row, K held by lane
-// K % 16 of the row in register K / 16. H = 2: one cell per half row (lanes 0-7, 8-15), K held by
-// lane 8 h + K % 8 of half h in register K / 8; each half takes its own broadcast (two masked
-// instructions).
-template <int H, int K, class R, int NQ>
-__device__ __forceinline__ void fmac_coef(R &acc, const R (&c)[NQ], R x)
-{
-    if constexpr (H == 1) {
-        fmac_row<K % 16>(acc, c[K / 16], x);
-    } else {
-        fmac_row<K % 8, 0x3>(acc, c[K / 8], x);
-        fmac_row<8 + K % 8, 0xc>(acc, c[K / 8], x);
-    }
-}
-template <class R>
-__device__ __forceinline__ void row_fence(R &c)
-{
-    asm volatile("s_nop 1" : "+v"(c));
-}
+// Far field: multipole-to-target evaluation (M2P). A lane holds one source cell of a group's list,
+// both of its expansions in VGPRs, and the wavefront runs over the targets of the group: every
+// product with a coefficient is a plain fused multiply-add on the lane's own registers, and no lane
+// is idle while a chunk of 64 list entries is full, whatever the number of targets (rows of 16
+// targets per cell left 35 % of the lanes on padding, the film's groups holding 4 to 27 targets, and
+// needed a DPP broadcast per product). The last, partial chunk of a list holds its entries two or
+// four times over, each copy taking its own targets.
+//
+// Evaluation of a cell (P: degree, x in cell widths from its centre), device expansions being stored
+// times (2n - 1)!!: with rho = 1 / r^2, zeta = z rho, e = -rho (x - i y),
+//   phi = (1/r) [S_0 + 2 Re sum_{m >= 1} e^m S_m],   S_m = sum_{n >= m} M_n^m Q_n^m,
+//   Q_m^m = 1, Q_{m+1}^m = zeta, Q_n^m = zeta Q_{n-1}^m - b_n^m rho Q_{n-2}^m,
+//   b_n^m = ((n - 1)^2 - m^2) / ((2n - 1)(2n - 3)):
+// the Legendre recurrences are real and shared by the two charge sets and by the real and imaginary
+// parts, and the azimuthal factors are applied once per column (Horner's rule in e). Per (target,
+// cell) 228 instructions at degrees 8 / 4 in FP32 (350 with complex recurrences); in FP64 440 in two
+// passes, one per set (447 with complex recurrences and both sets at once).
+// Bound by VALU issue (FP32: 77 % of it on the 2M-tetrahedron film), in FP64 also by the latency of
+// the expansions' loads at two wavefronts per SIMD. M2P pass, with the row layout and with this one:
+// 2M film mixed 1.90 -> 0.85 ms, 490k film FP64 0.95 -> 0.65 ms, 48k cube FP64 0.39 -> 0.09 ms,
+// 64 dots mixed 0.50 -> 0.13 ms.
 
 template <int B, int E, class F>
 __device__ __forceinline__ void static_for(F &&f)
@@ -1420,211 +1390,300 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
-// M2P of the two expansions of a row's cell at one target per lane (x in cell widths), the first
-// to degree Q, the second to degree QV <= Q: su = sum M_u,n^m conj(I_n^m(x)), sv likewise.
-// Coefficient k of a set (k = 2 fidx(n, m), + 1 for the imaginary part) sits where
-// fmac_coef<H, k> reads it. The irregular harmonics are streamed column by column (diagonal
-// I_m^m, then I_{m+1}^m and the three-term recurrence in n), the recurrence factors of each degree
-// shared by all columns; the m = 0 column is real (M_n^0 and I_n^0 are real for real charges).
-template <int Q, int QV, int H, class R, int NQ, int NQV>
-__device__ __forceinline__ void m2p_rows(const R (&cu)[NQ], const R (&cv)[NQV], R x, R y, R z, R &su, R &sv)
+// Horner's rule in e for one set: t = sum_{m = max(MA, 1)}^{MB} e^{m - max(MA, 1)} S_m and, when
+// MA = 0, s0 = S_0.
+template <class R> struct M2pAcc {
+    R tr, ti, s0;
+};
+constexpr int m2p_reals(int q) { return q < 0 ? 1 : 2 * fcount(q); }  // q = -1: no second set
+
+template <int Q, int QV, int MA, int MB, class R>
+__device__ __forceinline__ void m2p_cell(const R (&cu)[2 * fcount(Q)], const R (&cv)[m2p_reals(QV)], R x, R y, R z,
+                                         R &su, R &sv)
 {
     const R r2 = x * x + y * y + z * z;
-    const R ir2 = fast_inv(r2), zr = z * ir2, zr2 = zr + zr, ir22 = ir2 + ir2;
-    // tz[n] = (2n - 1) z / r^2 and un[n] = (n - 1)^2 / r^2; column m takes
-    // un[n] - m^2 / r^2 = (n + m - 1)(n - m - 1) / r^2
-    R tz[Q + 1], un[Q + 1];
-    tz[1] = zr;
-    un[1] = R(0);
-    {
-        R st = ir2;
-#pragma unroll
-        for (int n = 2; n <= Q; n++) {
-            tz[n] = tz[n - 1] + zr2;
-            un[n] = un[n - 1] + st;
-            st += ir22;
+    const R rho = fast_inv(r2), zeta = z * rho, zeta2 = zeta * zeta;
+    const R er = -x * rho, ei = y * rho;
+    M2pAcc<R> u{R(0), R(0), R(0)}, v{R(0), R(0), R(0)};
+    // columns from the highest down
+    static_for<0, MB - MA + 1>([&](auto ic) {
+        constexpr int m = MB - decltype(ic)::value;
+        // S_m of the two sets: real, imaginary
+        constexpr bool V = m <= QV;
+        R ur = cu[2 * fidx(m, m)], ui = m ? cu[2 * fidx(m, m) + 1] : R(0), vr = R(0), vi = R(0);
+        if constexpr (V) {
+            vr = cv[2 * fidx(m, m)];
+            if constexpr (m > 0) vi = cv[2 * fidx(m, m) + 1];
         }
-    }
-    R dre = fast_rsqrt(r2), dim = R(0);
-    R au = R(0), av = R(0);
-    fmac_coef<H, 0>(au, cu, dre);
-    fmac_coef<H, 0>(av, cv, dre);
-    if constexpr (Q >= 1) {
-        constexpr int k1 = 2 * fidx(1, 0);
-        R p2 = dre, p1 = zr * dre;
-        fmac_coef<H, k1>(au, cu, p1);
-        if constexpr (QV >= 1) fmac_coef<H, k1>(av, cv, p1);
-        static_for<2, Q + 1>([&](auto nc) {
-            constexpr int n = decltype(nc)::value, k = 2 * fidx(n, 0);
-            const R c = tz[n] * p1 - un[n] * p2;
-            fmac_coef<H, k>(au, cu, c);
-            if constexpr (n <= QV) fmac_coef<H, k>(av, cv, c);
-            p2 = p1;
-            p1 = c;
-        });
-    }
-    R hu = R(0), hv = R(0);
-    R fd = -ir2, vm = R(0), dv = ir2;  // fd = (1 - 2m) / r^2, vm = m^2 / r^2
-    static_for<1, Q + 1>([&](auto mc) {
-        constexpr int m = decltype(mc)::value, kd = 2 * fidx(m, m);
-        const R nre = fd * (x * dre - y * dim), nim = fd * (x * dim + y * dre);
-        fd -= ir22;
-        vm += dv;
-        dv += ir22;
-        dre = nre;
-        dim = nim;
-        fmac_coef<H, kd>(hu, cu, dre);
-        fmac_coef<H, kd + 1>(hu, cu, dim);
-        if constexpr (m <= QV) {
-            fmac_coef<H, kd>(hv, cv, dre);
-            fmac_coef<H, kd + 1>(hv, cv, dim);
-        }
-        if constexpr (m + 1 <= Q) {
-            constexpr int k1 = 2 * fidx(m + 1, m);
-            R p2re = dre, p2im = dim, p1re = tz[m + 1] * dre, p1im = tz[m + 1] * dim;
-            fmac_coef<H, k1>(hu, cu, p1re);
-            fmac_coef<H, k1 + 1>(hu, cu, p1im);
-            if constexpr (m + 1 <= QV) {
-                fmac_coef<H, k1>(hv, cv, p1re);
-                fmac_coef<H, k1 + 1>(hv, cv, p1im);
+        R p2 = R(1), p1 = zeta;
+        static_for<m + 1, Q + 1>([&](auto nc) {
+            constexpr int n = decltype(nc)::value, k = 2 * fidx(n, m);
+            R q;
+            constexpr R b = R(double((n - 1) * (n - 1) - m * m) / double((2 * n - 1) * (2 * n - 3)));
+            if constexpr (n == m + 1) q = zeta;
+            else if constexpr (n == m + 2) q = fma(rho, -b, zeta2);
+            else if constexpr (n == m + 3) q = zeta * fma(rho, -b, p1);  // p2 = zeta
+            else q = fma(zeta, p1, -(b * rho) * p2);
+            ur = fma(cu[k], q, ur);
+            if constexpr (m > 0) ui = fma(cu[k + 1], q, ui);
+            if constexpr (n <= QV) {
+                vr = fma(cv[k], q, vr);
+                if constexpr (m > 0) vi = fma(cv[k + 1], q, vi);
             }
-            static_for<m + 2, Q + 1>([&](auto nc) {
-                constexpr int n = decltype(nc)::value, k = 2 * fidx(n, m);
-                const R bb = un[n] - vm;
-                const R cre = tz[n] * p1re - bb * p2re, cim = tz[n] * p1im - bb * p2im;
-                fmac_coef<H, k>(hu, cu, cre);
-                fmac_coef<H, k + 1>(hu, cu, cim);
-                if constexpr (n <= QV) {
-                    fmac_coef<H, k>(hv, cv, cre);
-                    fmac_coef<H, k + 1>(hv, cv, cim);
+            p2 = p1;
+            p1 = q;
+        });
+        auto horner = [&](M2pAcc<R> &t, R re, R im) {
+            const R nr = fma(er, t.tr, fma(-ei, t.ti, re));
+            t.ti = fma(er, t.ti, fma(ei, t.tr, im));
+            t.tr = nr;
+        };
+        if constexpr (m > 0) {
+            if constexpr (m == MB) {
+                u.tr = ur;
+                u.ti = ui;
+            } else {
+                horner(u, ur, ui);
+            }
+            if constexpr (V) {
+                if constexpr (m == (QV < MB ? QV : MB)) {
+                    v.tr = vr;
+                    v.ti = vi;
+                } else {
+                    horner(v, vr, vi);
                 }
-                p2re = p1re;
-                p2im = p1im;
-                p1re = cre;
-                p1im = cim;
-            });
+            }
+        } else {
+            u.s0 = ur;
+            v.s0 = vr;
         }
     });
-    su = au + (hu + hu);
-    sv = av + (hv + hv);
+    // e^max(MA, 1)
+    R ar = er, ai = ei;
+#pragma unroll
+    for (int q = 1; q < (MA > 1 ? MA : 1); q++) {
+        const R nr = er * ar - ei * ai;
+        ai = er * ai + ei * ar;
+        ar = nr;
+    }
+    const R ir = fast_rsqrt(r2);
+    const R hu = ar * u.tr - ai * u.ti, hv = ar * v.tr - ai * v.ti;
+    su = ir * fma(R(2), hu, u.s0);
+    sv = ir * fma(R(2), hv, v.s0);
 }
 
-// The source cell of a row (H = 1) or half row (H = 2) in a step: both expansions in
-// row-broadcast layout (degree Q of order-P storage), its centre and 1/W, and whether it applies
-// to this lane's target.
-template <int P, int Q, int QV, int H, class R>
-struct M2pCell {
-    static constexpr int LPC = 16 / H, NK = 2 * fcount(Q), NQ = (NK + LPC - 1) / LPC;
-    static constexpr int NKV = 2 * fcount(QV), NQV = (NKV + LPC - 1) / LPC;
-    R raw[NQ], rawv[NQV];
-    double4 c;
-    bool on;
+// The columns that one pass over a chunk holds in registers: as many from MA on as fit M2P_REGS
+// 32-bit registers of coefficients. Where both sets do not fit together (FP64 from degree 6) each
+// set has its own pass: the recurrences run twice (440 operations a pair against 355 at degree 8),
+// but every coefficient is fetched once; two passes over halves of the columns of both sets, which
+// fetch each 64-byte piece twice, took 1.02 ms against 0.84 on the 490k film.
+constexpr int M2P_REGS = 172;
+template <int Q, int QV, class R>
+constexpr int m2p_last_col(int ma)
+{
+    int regs = 0, m = ma;
+    for (; m <= Q; m++) {
+        const int c = (m ? 2 : 1) * ((Q + 1 - m) + (QV >= m ? QV + 1 - m : 0)) * (int)(sizeof(R) / 4);
+        if (m > ma && regs + c > M2P_REGS) break;
+        regs += c;
+    }
+    return m - 1;
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// The expansions of a chunk's cells come through LDS in pieces of 64 bytes per cell: four lanes load
+// one cell's piece, so whole segments are fetched, and each lane then reads its own cell's. Unit u of
+// row r sits at 4 r + (u ^ (r / 4) % 4): sixteen lanes cover all 64 banks in the writes (four rows)
+// and in the reads (one unit of sixteen rows).
+__device__ __forceinline__ int m2p_unit(int row, int u) { return 4 * row + (u ^ ((row >> 2) & 3)); }
+struct M2pWave {
+    u32x4 stage[64 * 4];
+    double tx[16][3];  // the tile's targets and their octants
+    int32_t toct[16];
 };
 
-// List entries [b, e) of a group, evaluated to degree Q <= P (expansions stored to P): step s puts
-// entry b + s cps + slot in each cell slot (other wavefronts on the SIMD hide the loads' latency).
-// Every lane runs every step (invalid lanes evaluate at a dummy offset and add 0).
-template <int P, int Q, int QV, int H, class R>
-__device__ __forceinline__ void m2p_range(int b, int e, int cps, int slot, bool tv, int oc, double4 y,
-                                          const int32_t *__restrict__ u_cell, const uint8_t *__restrict__ u_mask,
-                                          const double4 *__restrict__ cen, const R *__restrict__ Md, double &pu,
-                                          double &pv)
+// Coefficients k of [0, NK) of one set (base: its first element of a cell's storage) that belong to
+// columns MA..MB, of this lane's cell, into c.
+template <int P, int NK, int BASE, int MA, int MB, class R>
+__device__ __forceinline__ void m2p_load(const R *__restrict__ M, const int32_t (&cells)[4], int nload, int row,
+                                         M2pWave &W, R (&c)[NK])
 {
-    using C = M2pCell<P, Q, QV, H, R>;
-    constexpr int NCo = fcount(P), LPC = C::LPC, NK = C::NK, NQ = C::NQ, NKV = C::NKV, NQV = C::NQV;
-    const int j = threadIdx.x & (LPC - 1);  // lane within the cell's lanes
-    const int nst = (e - b + cps - 1) / cps;  // uniform over the wavefront
-    auto fetch = [&](int s, C &cl) {
-        const int ei = b + s * cps + slot;
-        const bool ev = slot < cps && ei < e;
-        const int ec = ev ? ei : b;
-        const int cell = u_cell[ec];
-        cl.c = cen[cell];
-        cl.on = tv && ev && ((u_mask[ec] >> oc) & 1);
-        const R *src = Md + (size_t)cell * 4 * NCo;
+    constexpr int E = 16 / (int)sizeof(R);           // elements per 16-byte unit
+    constexpr int S0 = BASE / E * E, PE = 4 * E;  // first element of the first piece; elements of a piece
+    constexpr int NP = (BASE + NK - S0 + PE - 1) / PE;
+    const int lane = threadIdx.x & 63, sub = lane & 3;
+    constexpr int G = 8;  // pieces in flight (their registers are the coefficients' own until then)
+    static_for<0, (NP + G - 1) / G>([&](auto gc) {
+        constexpr int g0 = decltype(gc)::value * G, ng = NP - g0 < G ? NP - g0 : G;
+        u32x4 raw[ng][4];
+        // a cell's pieces one after another: the two halves of a cache line are fetched together
 #pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            // lanes past the last coefficient repeat it; no DPP read takes them
-            cl.raw[q] = src[min(LPC * q + j, NK - 1)];
+        for (int i = 0; i < 4; i++)
+            if (i < nload)
+#pragma unroll
+                for (int q = 0; q < ng; q++)
+                    raw[q][i] = *reinterpret_cast<const u32x4 *>(M + (size_t)cells[i] * 4 * fcount(P) + S0 +
+                                                                 (g0 + q) * PE + sub * E);
+        static_for<0, ng>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            __builtin_amdgcn_wave_barrier();  // the rows are this wavefront's own: LDS keeps its order
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i < nload) W.stage[m2p_unit(16 * i + (lane >> 2), sub)] = raw[q][i];
+            __builtin_amdgcn_wave_barrier();
+            static_for<0, 4>([&](auto uc) {
+                constexpr int un = decltype(uc)::value;
+                const u32x4 w = W.stage[m2p_unit(row, un)];
+                static_for<0, E>([&](auto ec) {
+                    constexpr int e = decltype(ec)::value, k = S0 + (g0 + q) * PE + un * E + e - BASE;
+                    if constexpr (k >= 0 && k < NK) {
+                        constexpr int n = XL<P>::deg(k), m = (k >> 1) - fidx(n, 0);
+                        if constexpr (m >= MA && m <= MB && !(m == 0 && (k & 1))) {
+                            if constexpr (sizeof(R) == 4) {
+                                c[k] = __uint_as_float(w[e]);
+                            } else {
+                                c[k] = __longlong_as_double(((long long)w[2 * e + 1] << 32) | w[2 * e]);
+                            }
+                        }
+                    }
+                });
+            });
+        });
+    });
+}
+
+// The targets of a task and where its sums go: part[target - tb].
+struct M2pTargets {
+    int tb, te;
+    const double4 *pos;
+    const uint8_t *oct;
+    double2 *part;
+};
+struct M2pLane {
+    double4 c;      // the lane's cell: centre and 1 / W
+    unsigned mask;  // child octants that it applies to
+    int32_t cells[4];
+    int nload, row, copy, ncopy;
+};
+
+// Sum of a tile's D over its rows (the lanes of each target): lane l holds D's rows l / 16 + 4 q of
+// column l % 16; the result, for target l % 16, in every lane.
+__device__ __forceinline__ double m2p_fold(const f64x4 &D)
+{
+    double s = (D[0] + D[1]) + (D[2] + D[3]);
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    return s;
+}
+
+// One pass of a chunk over all targets of the group: expansions of degree Q from element BASE of a
+// cell's storage (and the second set to degree QV, unless -1), columns from MA on. Targets run in
+// tiles of 16, the columns of D: each (target, lane) value enters the FP64 matrix product D += A B
+// with A the lanes' values and B selecting the target's column, so that the 64 lanes of a target are
+// summed in FP64 on the matrix cores beside the vector work (a cross-lane sum in the vector unit
+// takes 36 instructions a target). OUT: which sums it writes (1: u, 2: v, 3: both), added to the
+// pass before it where MA > 0.
+template <int P, int Q, int QV, int BASE, int MA, int OUT, class R>
+__device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, const R *__restrict__ M, M2pWave &W)
+{
+    constexpr int MB = m2p_last_col<Q, QV, R>(MA);
+    const int lane = threadIdx.x & 63;
+    const double4 c = l.c;
+    R cu[2 * fcount(Q)], cv[m2p_reals(QV)];
+    m2p_load<P, 2 * fcount(Q), BASE, MA, MB, R>(M, l.cells, l.nload, l.row, W, cu);
+    if constexpr (MA <= QV) m2p_load<P, m2p_reals(QV), 2 * fcount(P), MA, MB, R>(M, l.cells, l.nload, l.row, W, cv);
+#pragma unroll 1
+    for (int tb = T.tb; tb < T.te; tb += 16) {
+        const int nt = min(16, T.te - tb);
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 16) {
+            const int t = tb + min(lane, nt - 1);
+            const double4 y = T.pos[t];
+            W.tx[lane][0] = y.x;
+            W.tx[lane][1] = y.y;
+            W.tx[lane][2] = y.z;
+            W.toct[lane] = T.oct[t];
         }
-#pragma unroll
-        for (int q = 0; q < NQV; q++) cl.rawv[q] = src[2 * NCo + min(LPC * q + j, NKV - 1)];
-    };
-    auto eval = [&](C &cl) {
-        R cf[NQ], cfv[NQV];
-#pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            cf[q] = cl.raw[q];
-            row_fence(cf[q]);
+        __builtin_amdgcn_wave_barrier();
+        f64x4 Du = {0, 0, 0, 0}, Dv = {0, 0, 0, 0};
+#pragma unroll 1
+        for (int t0 = 0; t0 < nt; t0 += l.ncopy) {
+            const int t = t0 + l.copy, tc = min(t, nt - 1);
+            const R x = (R)((W.tx[tc][0] - c.x) * c.w), y = (R)((W.tx[tc][1] - c.y) * c.w),
+                    z = (R)((W.tx[tc][2] - c.z) * c.w);
+            const bool on = t < nt && ((l.mask >> W.toct[tc]) & 1);
+            R su, sv;
+            m2p_cell<Q, QV, MA, MB, R>(cu, cv, x, y, z, su, sv);
+            const double sel = (lane & 15) == tc ? 1.0 : 0.0;
+            Du = Mfma<double>::mma(on ? (double)su * c.w : 0.0, sel, Du);
+            if constexpr (MA <= QV) Dv = Mfma<double>::mma(on ? (double)sv * c.w : 0.0, sel, Dv);
         }
-#pragma unroll
-        for (int q = 0; q < NQV; q++) {
-            cfv[q] = cl.rawv[q];
-            row_fence(cfv[q]);
+        const double fu = m2p_fold(Du);
+        double2 *d = T.part + (tb - T.tb) + lane;
+        if constexpr (OUT == 3) {
+            const double fv = m2p_fold(Dv);
+            if (lane < nt) *d = MA ? make_double2(d->x + fu, d->y + fv) : make_double2(fu, fv);
+        } else {
+            double *o = OUT == 1 ? &d->x : &d->y;
+            if (lane < nt) *o = MA ? *o + fu : fu;
         }
-        const double4 c = cl.c;
-        const R x = cl.on ? (R)((y.x - c.x) * c.w) : R(2), yy = cl.on ? (R)((y.y - c.y) * c.w) : R(0),
-                z = cl.on ? (R)((y.z - c.z) * c.w) : R(0);
-        R su, sv;
-        m2p_rows<Q, QV, H, R, NQ, NQV>(cf, cfv, x, yy, z, su, sv);
-        pu += cl.on ? (double)su * c.w : 0.0;
-        pv += cl.on ? (double)sv * c.w : 0.0;
-    };
-    for (int s = 0; s < nst; s++) {
-        C A;
-        fetch(s, A);
-        eval(A);
+    }
+    if constexpr (MB < Q) m2p_pass<P, Q, QV, BASE, MB + 1, OUT, R>(l, T, M, W);
+}
+
+// One chunk of at most 64 list entries [b, b + n) against the task's targets, to degree Q (QV for the
+// second set).
+template <int P, int Q, int QV, class R>
+__device__ __forceinline__ void m2p_chunk(int b, int n, const M2pTargets &T, const int32_t *__restrict__ u_cell,
+                                          const uint8_t *__restrict__ u_mask, const double4 *__restrict__ cen,
+                                          const R *__restrict__ M, M2pWave &W)
+{
+    const int lane = threadIdx.x & 63;
+    // lanes per copy of the entries: 64, 32 or 16 (a target's lanes stay whole rows of 16)
+    const int sh = n > 32 ? 6 : n > 16 ? 5 : 4;
+    M2pLane l;
+    l.row = lane & ((1 << sh) - 1);
+    l.copy = lane >> sh;
+    l.ncopy = 64 >> sh;
+    l.nload = 1 << (sh - 4);
+    const bool ev = l.row < n;
+    const int e = b + (ev ? l.row : n - 1);
+#pragma unroll
+    for (int i = 0; i < 4; i++) l.cells[i] = u_cell[b + min(16 * i + (lane >> 2), n - 1)];
+    l.c = cen[u_cell[e]];
+    l.mask = ev ? u_mask[e] : 0u;
+    if constexpr (m2p_last_col<Q, QV, R>(0) == Q) {
+        m2p_pass<P, Q, QV, 0, 0, 3, R>(l, T, M, W);
+    } else {
+        m2p_pass<P, Q, -1, 0, 0, 1, R>(l, T, M, W);
+        m2p_pass<P, QV, -1, 2 * fcount(P), 0, 2, R>(l, T, M, W);
     }
 }
 
-// H = 1: groups of any size, chunks of up to 64 targets as above. H = 2: groups of at most 8
-// targets; each half row holds its own cell, lanes 8 h + i of row r evaluate cell slot 2 r + h for
-// target i, so a step covers 8 cells (each coefficient product then takes two masked broadcasts).
-// gid lists the groups of the launch.
-template <int P, int PF, int PV, int H, class R>
-__global__ __launch_bounds__(256) void k_fmm_m2p(int ng, const int32_t *__restrict__ gid,
-                                                 const int32_t *__restrict__ grp_tb,
-                                                 const int32_t *__restrict__ grp_te,
-                                                 const int32_t *__restrict__ u_ptr, const int32_t *__restrict__ u_far,
-                                                 const int32_t *__restrict__ u_cell,
-                                                 const uint8_t *__restrict__ u_mask,
-                                                 const uint8_t *__restrict__ tgt_oct, const double4 *__restrict__ tpos,
-                                                 const double4 *__restrict__ cen, const R *__restrict__ M,
-                                                 double2 *__restrict__ far)
+// A task is one chunk of a group's list, one wavefront and block each (task = group, first entry,
+// entries, offset of its sums in part); the first nnear tasks are evaluated to degree P, the others
+// (far entries) to degree PF. Each task writes one partial sum per target of its group, which
+// k_fmm_finish adds in list order. Whole lists per wavefront, four wavefronts to a block, left
+// half of the wave slots empty behind the longest lists (4.1 of 8 waves per CU on average).
+template <int P, int PF, int PV, class R>
+__global__ __launch_bounds__(64, sizeof(R) == 4 && P <= 8 ? 3 : 2) void k_fmm_m2p(
+    const int4 *__restrict__ task, const int32_t *__restrict__ grp_tb, const int32_t *__restrict__ grp_te,
+    const int32_t *__restrict__ u_far, const int32_t *__restrict__ u_cell, const uint8_t *__restrict__ u_mask,
+    const uint8_t *__restrict__ tgt_oct, const double4 *__restrict__ tpos, const double4 *__restrict__ cen,
+    const R *__restrict__ M, double2 *__restrict__ part)
 {
-    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int gi = xcd_block(blockIdx.x, gridDim.x) * 4 + wv;
-    if (gi >= ng) return;  // whole wavefront
-    const int g = gid[gi];
-    const int lane = threadIdx.x & 63, row = lane >> 4, j = lane & 15;
-    const int tb = grp_tb[g], te = grp_te[g], ub = u_ptr[g], ue = u_ptr[g + 1], uf = u_far[g];
-    for (int t0 = tb; t0 < te; t0 += 64) {
-        const int nt = min(64, te - t0);
-        // H = 1: nr target rows, cps = 4 / nr cells per step; H = 2: one target row of 8 lanes
-        // per half, 8 cells per step
-        const int nr = H == 1 ? (nt + 15) >> 4 : 1, cps = H == 1 ? 4 / nr : 8;
-        const int tri = H == 1 ? row % nr : 0, slot = H == 1 ? row / nr : 2 * row + (j >> 3);
-        const int ti = H == 1 ? 16 * tri + j : j & 7;
-        const int t = t0 + ti;
-        const bool tv = slot < cps && ti < nt;
-        const double4 y = tpos[tv ? t : t0];
-        const int oc = tv ? tgt_oct[t] : 0;
-        double pu = 0, pv = 0;
-        if constexpr (PF == P) {
-            m2p_range<P, P, PV, H, R>(ub, ue, cps, slot, tv, oc, y, u_cell, u_mask, cen, M, pu, pv);
-        } else {
-            m2p_range<P, P, PV, H, R>(ub, uf, cps, slot, tv, oc, y, u_cell, u_mask, cen, M, pu, pv);
-            m2p_range<P, PF, (PV < PF ? PV : PF), H, R>(uf, ue, cps, slot, tv, oc, y, u_cell, u_mask, cen, M, pu, pv);
-        }
-        // each target's cell slots, in slot order (all lanes take part in the shuffles)
-        double su = 0, sv = 0;
-        for (int q = 0; q < cps; q++) {
-            const int src = H == 1 ? ((q * nr + tri) << 4) + j : ((q >> 1) << 4) + ((q & 1) << 3) + (j & 7);
-            su += __shfl(pu, src, 64);
-            sv += __shfl(pv, src, 64);
-        }
-        if (slot == 0 && tv) far[t] = make_double2(su, sv);
-    }
+    __shared__ M2pWave W;
+    const int4 k = task[xcd_block(blockIdx.x, gridDim.x)];
+    M2pTargets T;
+    T.tb = grp_tb[k.x];
+    T.te = grp_te[k.x];
+    T.pos = tpos;
+    T.oct = tgt_oct;
+    T.part = part + k.w;
+    if (PF == P || k.y < u_far[k.x])
+        m2p_chunk<P, P, PV, R>(k.y, k.z, T, u_cell, u_mask, cen, M, W);
+    else
+        m2p_chunk<P, PF, (PV < PF ? PV : PF), R>(k.y, k.z, T, u_cell, u_mask, cen, M, W);
 }
 
 // Per target: the multipole part (M2P), the local expansion of the group's ancestor (scaled like
@@ -1633,15 +1692,23 @@ __global__ __launch_bounds__(256) void k_fmm_m2p(int ng, const int32_t *__restri
 template <int P, class R>
 __global__ __launch_bounds__(256) void k_fmm_finish(int T, const int32_t *__restrict__ tgt_lc,
                                                     const double4 *__restrict__ tpos, const double4 *__restrict__ cen,
-                                                    const R *__restrict__ Lx, const double2 *__restrict__ far,
+                                                    const R *__restrict__ Lx, const int4 *__restrict__ tgt_far,
+                                                    const double2 *__restrict__ far,
                                                     const double2 *__restrict__ pot, const int32_t *__restrict__ tgt_node,
                                                     NodeRec *__restrict__ nxt, double mscale)
 {
     constexpr int NCo = fcount(P), CW = 2 * NCo;
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= T) return;
-    const double2 f = far[t];
-    double su = f.x, sv = f.y;
+    // M2P's partial sums of the target: f.z of them from f.x on, f.y apart
+    const int4 f = tgt_far[t];
+    double su = 0, sv = 0;
+#pragma unroll 4
+    for (int k = 0; k < f.z; k++) {
+        const double2 p = far[f.x + (size_t)k * f.y];
+        su += p.x;
+        sv += p.y;
+    }
     const int lc = tgt_lc[t];
     if (lc >= 0) {
         const double4 c = cen[lc], y = tpos[t];
@@ -1659,22 +1726,34 @@ __global__ __launch_bounds__(256) void k_fmm_finish(int T, const int32_t *__rest
 
 void fmm_build_near(Ctx &c, FmmPlan &P);
 
-// Groups of at most this many targets are evaluated with one source cell per half row.
-constexpr int M2P_HALF_MAX = 8;
-
-// Lane slots executed by k_fmm_m2p's mapping: per 64-target chunk of a group, one wavefront per
-// step of cps cells (degree-P and far entries stepped separately).
-static int64_t m2p_lane_slots(const FmmPlan &P)
+// Tasks of k_fmm_m2p: chunks of up to 64 entries of each group's list, near and far entries apart,
+// with the offset of their partial sums; tgt_far: per target the first of its partial sums, their
+// distance (the group's targets) and their number. Also the lane slots that the tasks execute: each
+// target of the group once on 64, 32 or 16 lanes per tile of 16 targets.
+static std::vector<int4> m2p_tasks(FmmPlan &P, std::vector<int4> &tgt_far, size_t &npart)
 {
-    int64_t slots = 0;
-    for (size_t g = 0; g < P.grp_tb.size(); g++)
-        for (int t0 = P.grp_tb[g]; t0 < P.grp_te[g]; t0 += 64) {
-            const int nt = std::min(64, P.grp_te[g] - t0);
-            const int cps = P.grp_te[g] - P.grp_tb[g] <= M2P_HALF_MAX ? 8 : 4 / ((nt + 15) / 16);
-            const int near = P.u_far[g] - P.u_ptr[g], far = P.u_ptr[g + 1] - P.u_far[g];
-            slots += 64 * (int64_t)((near + cps - 1) / cps + (far + cps - 1) / cps);
-        }
-    return slots;
+    std::vector<int4> v;
+    tgt_far.assign(std::max<size_t>(1, P.tgt_node.size()), make_int4(0, 0, 0, 0));
+    npart = 0;
+    P.m2p_slots = 0;
+    for (size_t g = 0; g < P.grp_tb.size(); g++) {
+        const int tb = P.grp_tb[g], nt = P.grp_te[g] - tb;
+        const size_t first = npart;
+        int chunks = 0;
+        auto list = [&](int b, int e) {
+            for (; b < e; b += 64, chunks++, npart += nt) {
+                const int n = std::min(64, e - b), copies = n > 32 ? 1 : n > 16 ? 2 : 4;
+                v.push_back(make_int4((int)g, b, n, (int)npart));
+                for (int t = 0; t < nt; t += 16)
+                    P.m2p_slots += 64 * (int64_t)((std::min(16, nt - t) + copies - 1) / copies);
+            }
+        };
+        list(P.u_ptr[g], P.u_far[g]);
+        list(P.u_far[g], P.u_ptr[g + 1]);
+        for (int t = tb; t < tb + nt; t++) tgt_far[t] = make_int4((int)(first + t - tb), nt, chunks, 0);
+    }
+    if (npart > (size_t)INT32_MAX) throw std::string("FMM plan: the far field's partial sums exceed int32 (range)");
+    return v;
 }
 
 // The M2M (K = 0) or L2L (K = 1) operators of the 8 child octants in real form, in the fragment
@@ -1696,8 +1775,10 @@ static std::vector<double> xlate_pack(const FmmPlan &Pl, int K, bool pair)
             for (int n = 0; n <= P; n++)
                 for (int m = 0; m <= n; m++) {
                     const cplx v = K == 0 ? m2m_coef(e.data(), Rd, n, m) : l2l_coef(e.data(), Rd, P, n, m);
-                    T[(size_t)(2 * fidx(n, m)) * NR + j] = v.re;
-                    T[(size_t)(2 * fidx(n, m) + 1) * NR + j] = v.im;
+                    // multipoles are stored times fmm_stored(degree), local expansions as they are
+                    const double sc = K == 0 ? fmm_stored(n) / fmm_stored(L::deg(j)) : 1.0;
+                    T[(size_t)(2 * fidx(n, m)) * NR + j] = sc * v.re;
+                    T[(size_t)(2 * fidx(n, m) + 1) * NR + j] = sc * v.im;
                 }
         }
         for (int R = 0; R < NT; R++)
@@ -1775,8 +1856,9 @@ static std::vector<double> m2l_pack(const FmmPlan &Pl)
             for (int n = 0; n <= P; n++)
                 for (int m = 0; m <= n; m++) {
                     const cplx v = m2l_coef(e.data(), It, P, n, m);
-                    T[(size_t)(2 * fidx(n, m)) * NR + j] = v.re;
-                    T[(size_t)(2 * fidx(n, m) + 1) * NR + j] = v.im;
+                    const double sc = 1.0 / fmm_stored(L::deg(j));
+                    T[(size_t)(2 * fidx(n, m)) * NR + j] = sc * v.re;
+                    T[(size_t)(2 * fidx(n, m) + 1) * NR + j] = sc * v.im;
                 }
         }
         for (int R = 0; R < NT; R++)
@@ -1897,13 +1979,18 @@ int fmm_create(Ctx &c)
         P->d_leaf_sb = dput(P->leaf_sb);
         P->d_leaf_se = dput(P->leaf_se);
         P->d_grp_tb = dput(P->grp_tb);
-        P->m2p_gid.clear();
-        for (int pass = 0; pass < 2; pass++) {
-            for (size_t g = 0; g < P->grp_tb.size(); g++)
-                if ((P->grp_te[g] - P->grp_tb[g] <= M2P_HALF_MAX) == (pass == 1)) P->m2p_gid.push_back((int32_t)g);
-            if (pass == 0) P->m2p_n1 = (int)P->m2p_gid.size();
+        {
+            std::vector<int4> tf;
+            size_t npart = 0;
+            const std::vector<int4> tk = m2p_tasks(*P, tf, npart);
+            P->m2p_ntask = (int)tk.size();
+            P->d_m2p_task = dput(tk);
+            P->d_tgt_far = dput(tf);
+            void *d = nullptr;
+            if (hipMalloc(&d, std::max<size_t>(1, npart) * sizeof(double2)) != hipSuccess)
+                throw std::string("hipMalloc M2P partial sums");
+            P->d_far = (double2 *)d;
         }
-        P->d_m2p_gid = dput(P->m2p_gid);
         P->d_grp_te = dput(P->grp_te);
         P->d_grp_lcell = dput(P->grp_lcell);
         P->d_u_ptr = dput(P->u_ptr);
@@ -1918,7 +2005,6 @@ int fmm_create(Ctx &c)
             for (size_t g = 0; g < P->grp_tb.size(); g++)
                 for (int t = P->grp_tb[g]; t < P->grp_te[g]; t++) tlc[t] = P->grp_lcell[g];
             P->d_tgt_lc = dput(tlc);
-            P->d_far = dput(std::vector<double2>(std::max<size_t>(1, P->tgt_node.size()), make_double2(0, 0)));
         }
         P->d_leaf_cell = dput(P->leaf_cell);
         P->d_m2m_cells = dput(P->m2m_cells);
@@ -1953,7 +2039,8 @@ int fmm_create(Ctx &c)
         P->d_l2l_child = dput(P->l2l_child);
         const size_t nexp = (size_t)P->ncell() * 2 * P->nc;
         void *d = nullptr;
-        if (hipMalloc(&d, nexp * 2 * fsz) != hipSuccess) throw std::string("hipMalloc M");
+        // 64 bytes past the end: M2P loads expansions in whole 64-byte pieces
+        if (hipMalloc(&d, nexp * 2 * fsz + 64) != hipSuccess) throw std::string("hipMalloc M");
         P->d_M = d;
         if (hipMalloc(&d, nexp * 2 * fsz) != hipSuccess) throw std::string("hipMalloc L");
         P->d_L = d;
@@ -1966,7 +2053,6 @@ int fmm_create(Ctx &c)
                     P->m2p_pairs += on;
                     if (k >= P->u_far[g]) P->m2p_far_pairs += on;
                 }
-        P->m2p_slots = m2p_lane_slots(*P);
         for (int32_t ci : P->m2l_cells) P->m2l_pairs += P->il_ptr[ci + 1] - P->il_ptr[ci];
         return FG_OK;
     } catch (const std::string &e) {
@@ -2128,7 +2214,7 @@ void fmm_destroy(Ctx &c)
 {
     FmmPlan *P = c.fmm;
     if (!P) return;
-    void *ptrs[] = {P->d_cen, P->d_m2p_gid, P->d_leaf_sb, P->d_leaf_se, P->d_grp_tb, P->d_grp_te, P->d_grp_lcell, P->d_u_ptr,
+    void *ptrs[] = {P->d_cen, P->d_m2p_task, P->d_tgt_far, P->d_leaf_sb, P->d_leaf_se, P->d_grp_tb, P->d_grp_te, P->d_grp_lcell, P->d_u_ptr,
                     P->d_u_far, P->d_u_cell, P->d_u_mask, P->d_tgt_oct, P->d_tgt_node, P->d_tgt_pos, P->d_tgt_lc, P->d_far,
                     P->d_Tm2m, P->d_Tm2m_pair, P->d_Tl2l, P->d_Tm2l, P->d_m2l_part, P->d_m2l_tile_cell, P->d_m2l_tile_chunk,
                     P->d_m2l_chunk_code, P->d_m2l_chunk_src, P->d_m2m_child, P->d_l2l_par, P->d_l2l_child, P->d_M, P->d_L, P->d_leaf_cell, P->d_m2m_cells,
@@ -2237,28 +2323,18 @@ static void run_fmm(Ctx &c)
     if (fork && hipEventRecord(c.ev_join, c.aux) != hipSuccess) throw std::string("hipEventRecord (join)");
     {
         Prof pr(c, "fmm_m2p");
-        const int ng = (int)P.grp_tb.size();
-        if (ng > 0) {
-            // groups of more than M2P_HALF_MAX targets with one cell per row, then the others with
-            // one cell per half row
-            auto go = [&](auto k1, auto k2) {
-                const int n1 = P.m2p_n1, n2 = ng - P.m2p_n1;
-                if (n1 > 0)
-                    k1<<<(n1 + 3) / 4, 256, 0, c.stream>>>(n1, P.d_m2p_gid, P.d_grp_tb, P.d_grp_te, P.d_u_ptr,
-                                                          P.d_u_far, P.d_u_cell, P.d_u_mask, P.d_tgt_oct, P.d_tgt_pos,
-                                                          P.d_cen, M, P.d_far);
-                if (n2 > 0)
-                    k2<<<(n2 + 3) / 4, 256, 0, c.stream>>>(n2, P.d_m2p_gid + n1, P.d_grp_tb, P.d_grp_te, P.d_u_ptr,
-                                                          P.d_u_far, P.d_u_cell, P.d_u_mask, P.d_tgt_oct, P.d_tgt_pos,
-                                                          P.d_cen, M, P.d_far);
+        if (P.m2p_ntask > 0) {
+            auto go = [&](auto k) {
+                k<<<P.m2p_ntask, 64, 0, c.stream>>>(P.d_m2p_task, P.d_grp_tb, P.d_grp_te, P.d_u_far, P.d_u_cell,
+                                                    P.d_u_mask, P.d_tgt_oct, P.d_tgt_pos, P.d_cen, M, P.d_far);
             };
             constexpr int PL = fmm_far_degree(PP);
             // the second expansion (charges of v) to degree fmm_v_degree in the FP32 mode
             constexpr int PV = std::is_same<F, float>::value ? fmm_v_degree(PP) : PP;
             if (P.pf != PP)
-                go(k_fmm_m2p<PP, PL, PV, 1, F>, k_fmm_m2p<PP, PL, PV, 2, F>);
+                go(k_fmm_m2p<PP, PL, PV, F>);
             else
-                go(k_fmm_m2p<PP, PP, PV, 1, F>, k_fmm_m2p<PP, PP, PV, 2, F>);
+                go(k_fmm_m2p<PP, PP, PV, F>);
         }
     }
     // join: the near field, M2L and L2L are in
@@ -2268,7 +2344,7 @@ static void run_fmm(Ctx &c)
         Prof pr(c, "fmm_finish");
         const int T = (int)P.tgt_node.size();
         if (T > 0)
-            k_fmm_finish<PP, F><<<(T + 255) / 256, 256, 0, c.stream>>>(T, P.d_tgt_lc, P.d_tgt_pos, P.d_cen, Lx, P.d_far,
+            k_fmm_finish<PP, F><<<(T + 255) / 256, 256, 0, c.stream>>>(T, P.d_tgt_lc, P.d_tgt_pos, P.d_cen, Lx, P.d_tgt_far, P.d_far,
                                                                         P.d_pot, P.d_tgt_node, c.rec[1 - c.cur],
                                                                         P.mscale);
     }

@@ -340,6 +340,15 @@ __host__ __device__ constexpr double p2m_scale(int n, int m)
     return 1.0 / f;
 }
 
+// The device keeps multipole coefficients of degree n times (2n - 1)!!, which makes the Legendre
+// recurrence of their evaluation monic (k_fmm_m2p); P2M and the M2M and M2L operators carry it.
+__host__ __device__ constexpr double fmm_stored(int n)
+{
+    double f = 1.0;
+    for (int k = 2; k <= n; k++) f *= 2 * k - 1;
+    return f;
+}
+
 // L2P: sum_{n,m} L_n^m R_n^m(x), x in cell widths.
 __host__ __device__ inline double l2p_eval(const double2 *L, int p, double x, double y, double z)
 {
