@@ -567,63 +567,95 @@ __global__ __launch_bounds__(GB) void k_guess_backward(int N, const float *__res
 }
 
 // Partial weight gradients over a chunk of nodes: G[r][c] = sum_n A[n][r] B[n][c] with an implicit
-// last column B[n][rb] = 1 (the bias gradient). B is an activation array, or the GELU of a
-// pre-activation array when act is set. One partial of ra*(rb+1) values per block.
-constexpr int WG_CHUNK = 2048, WG_TILE = 32;
-__global__ __launch_bounds__(256) void k_guess_wgrad(int N, const float *__restrict__ A, int ra,
-                                                     const float *__restrict__ B, int rb, int act,
-                                                     float *__restrict__ part)
+// last column B[n][rb] = 1 (the bias gradient), on the FP32 matrix cores with the nodes as the inner
+// dimension. B is an activation array, or the GELU of a pre-activation array when act is set. Block
+// (b, l) takes chunk b of layer l; 64 nodes at a time go through LDS and each wavefront keeps up to
+// five 16 x 16 tiles of G. One partial in parameter layout per chunk, about WG_BLOCKS of them: with
+// chunks of 2,048 nodes and a thread per element of G a mesh of 20 k nodes kept 11 blocks busy
+// (3.4 ms for the three layers; 0.02 ms now).
+constexpr int WG_TILE = 64, WG_BLOCKS = 512, WG_PAD = 80;  // rows of 80: four rows meet 64 banks once
+__host__ inline int wg_chunk(int N) { return WG_TILE * ((N + WG_TILE * WG_BLOCKS - 1) / (WG_TILE * WG_BLOCKS)); }
+struct WgLayer {
+    const float *A;
+    int ra;
+    const float *B;
+    int rb, act, wofs, bofs;
+};
+struct WgLayers {
+    WgLayer l[3];
+};
+__global__ __launch_bounds__(256) void k_guess_wgrad(int N, int chunk, WgLayers Ls, float *__restrict__ part)
 {
-    __shared__ float sA[WG_TILE][NH];
-    __shared__ float sB[WG_TILE][NH + 1];
-    const int n0 = blockIdx.x * WG_CHUNK, n1 = min(N, n0 + WG_CHUNK);
-    const int ne = ra * (rb + 1);
-    float acc[17];
-    for (int q = 0; q < 17; q++) acc[q] = 0.f;
+    __shared__ float sA[WG_TILE][WG_PAD], sB[WG_TILE][WG_PAD];
+    const WgLayer L = Ls.l[blockIdx.y];
+    const int ra = L.ra, rb = L.rb, nct = rb / 16 + 1, ntile = (ra + 15) / 16 * nct;
+    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, col = l & 15, kq = l >> 4;
+    const int n0 = blockIdx.x * chunk, n1 = min(N, n0 + chunk);
+    constexpr int MT = 5;  // tiles per wavefront: 64 x 65 has 20
+    f32x4 acc[MT];
+#pragma unroll
+    for (int q = 0; q < MT; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int t0 = n0; t0 < n1; t0 += WG_TILE) {
         const int nt = min(WG_TILE, n1 - t0);
-        for (int k = threadIdx.x; k < WG_TILE * NH; k += blockDim.x) {
-            const int r = k / NH, c = k % NH;
+        for (int k = tid; k < WG_TILE * WG_PAD; k += 256) {
+            const int r = k / WG_PAD, c = k - r * WG_PAD;
             float a = 0.f, bv = 0.f;
-            if (r < nt && c < ra) a = A[(size_t)(t0 + r) * ra + c];
-            if (r < nt && c < rb) {
-                bv = B[(size_t)(t0 + r) * rb + c];
-                if (act) bv = gelu(bv);
+            if (r < nt) {
+                if (c < ra) a = L.A[(size_t)(t0 + r) * ra + c];
+                if (c < rb) {
+                    bv = L.B[(size_t)(t0 + r) * rb + c];
+                    if (L.act) bv = gelu(bv);
+                } else if (c == rb) {
+                    bv = 1.f;
+                }
             }
             sA[r][c] = a;
             sB[r][c] = bv;
         }
         __syncthreads();
-        for (int q = 0; q < 17; q++) {
-            const int e = threadIdx.x + q * 256;
-            if (e >= ne) break;
-            const int r = e / (rb + 1), c = e % (rb + 1);
-            float s = 0.f;
-            if (c < rb)
-                for (int n = 0; n < nt; n++) s += sA[n][r] * sB[n][c];
-            else
-                for (int n = 0; n < nt; n++) s += sA[n][r];
-            acc[q] += s;
+#pragma unroll
+        for (int q = 0; q < MT; q++) {
+            const int t = w + 4 * q;
+            if (t >= ntile) break;  // uniform over the wavefront
+            const int r0 = 16 * (t / nct), c0 = 16 * (t % nct);
+#pragma unroll
+            for (int ks = 0; ks < WG_TILE / 4; ks++)
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(sA[4 * ks + kq][r0 + col], sB[4 * ks + kq][c0 + col],
+                                                              acc[q], 0, 0, 0);
         }
         __syncthreads();
     }
-    for (int q = 0; q < 17; q++) {
-        const int e = threadIdx.x + q * 256;
-        if (e < ne) part[(size_t)blockIdx.x * ne + e] = acc[q];
+    float *d = part + (size_t)blockIdx.x * NTRAIN;
+#pragma unroll
+    for (int q = 0; q < MT; q++) {
+        const int t = w + 4 * q;
+        if (t >= ntile) break;
+        const int c = 16 * (t % nct) + col;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int r = 16 * (t / nct) + 4 * kq + j;
+            if (r >= ra || c > rb) continue;
+            d[c < rb ? L.wofs + r * rb + c : L.bofs + r] = acc[q][j];
+        }
     }
 }
 
-// grad[dst(e)] = sum over blocks of part[blk][e], scattered into the parameter layout:
-// weights at wofs + r * rb + c, bias at bofs + r
-__global__ void k_guess_reduce(int nblk, int ra, int rb, const float *__restrict__ part, int wofs, int bofs,
-                               float *__restrict__ grad)
+// grad[e] = sum over the chunks of part[chunk][e]: 32 parameters per block, eight threads each, in
+// FP64 and a fixed order
+__global__ __launch_bounds__(256) void k_guess_reduce(int nblk, const float *__restrict__ part,
+                                                      float *__restrict__ grad)
 {
-    const int ne = ra * (rb + 1);
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
-        double s = 0;
-        for (int b = 0; b < nblk; b++) s += part[(size_t)b * ne + e];
-        const int r = e / (rb + 1), c = e % (rb + 1);
-        grad[c < rb ? wofs + r * rb + c : bofs + r] = (float)s;
+    __shared__ double sh[8][32];
+    const int l = threadIdx.x & 31, g = threadIdx.x >> 5, e = blockIdx.x * 32 + l;
+    double s = 0;
+    if (e < NTRAIN)
+#pragma unroll 4
+        for (int b = g; b < nblk; b += 8) s += part[(size_t)b * NTRAIN + e];
+    sh[g][l] = s;
+    __syncthreads();
+    if (g == 0 && e < NTRAIN) {
+        for (int k = 1; k < 8; k++) s += sh[k][l];
+        grad[e] = (float)s;
     }
 }
 
@@ -708,7 +740,7 @@ void guess_init(Ctx &c, uint64_t seed)
         c.guess = g;
         g->N = c.N;
         for (int32_t m : c.h_mag) g->nmag += m != 0;
-        g->nblk = (c.N + WG_CHUNK - 1) / WG_CHUNK;
+        g->nblk = (c.N + wg_chunk(c.N) - 1) / wg_chunk(c.N);
         galloc(&g->params, NPARAM);
         galloc(&g->wbf, NTRAIN);
         galloc(&g->adam_m, NTRAIN);
@@ -812,7 +844,7 @@ static void ensure_training_buffers(GuessNet *g)
     galloc(&g->dz1, (size_t)g->N * NH);
     galloc(&g->dz2, (size_t)g->N * NH);
     galloc(&g->dout, (size_t)g->N * NO);
-    galloc(&g->gpart, (size_t)g->nblk * NH * (NH + 1));
+    galloc(&g->gpart, (size_t)g->nblk * NTRAIN);
 }
 
 static void compute_scales(Ctx &c)
@@ -861,18 +893,11 @@ static void loss_and_gradient(Ctx &c, double *loss, double *loss_ref)
                                                  g->xin, g->z1, g->z2, g->dout, g->lpart);
     k_guess_backward<<<nbf, GB, 0, c.stream>>>(c.N, g->params, g->wbf, g->z1, g->z2, g->dout, g->dz1, g->dz2);
     // weight gradients: (dout, h2) -> W3, b3; (dz2, h1) -> W2, b2; (dz1, x) -> W1, b1
-    struct L {
-        const float *A;
-        int ra;
-        const float *B;
-        int rb, act, wofs, bofs;
-    } layers[3] = {{g->dout, NO, g->z2, NH, 1, OFF_W3, OFF_B3},
-                   {g->dz2, NH, g->z1, NH, 1, OFF_W2, OFF_B2},
-                   {g->dz1, NH, g->xin, NX, 0, OFF_W1, OFF_B1}};
-    for (auto &l : layers) {
-        k_guess_wgrad<<<g->nblk, 256, 0, c.stream>>>(c.N, l.A, l.ra, l.B, l.rb, l.act, g->gpart);
-        k_guess_reduce<<<32, 256, 0, c.stream>>>(g->nblk, l.ra, l.rb, g->gpart, l.wofs, l.bofs, g->grad);
-    }
+    const WgLayers Ls{{{g->dout, NO, g->z2, NH, 1, OFF_W3, OFF_B3},
+                       {g->dz2, NH, g->z1, NH, 1, OFF_W2, OFF_B2},
+                       {g->dz1, NH, g->xin, NX, 0, OFF_W1, OFF_B1}}};
+    k_guess_wgrad<<<dim3(g->nblk, 3), 256, 0, c.stream>>>(c.N, wg_chunk(c.N), Ls, g->gpart);
+    k_guess_reduce<<<(NTRAIN + 31) / 32, 256, 0, c.stream>>>(g->nblk, g->gpart, g->grad);
     if (hipMemcpyAsync(g->h_l, g->lpart, 2 * nbf * sizeof(double), hipMemcpyDeviceToHost, c.stream) != hipSuccess)
         throw std::string("hipMemcpy (guess loss)");
     sync_or_throw(c, "guess training");
