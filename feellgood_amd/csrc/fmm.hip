@@ -1308,6 +1308,10 @@ __global__ __launch_bounds__(256) void k_nf_build(int T, const int32_t *__restri
 // one column list (the runs of the adjacent leaves); each element value is gathered once and
 // applied to up to four targets' coefficient rows at a time. Coefficients are FP64, or FP32 in the
 // mixed-precision mode (products and sums stay FP64).
+// Bound by memory latency, then bandwidth: a wavefront's list is some 400 columns, so its loads have to
+// be in flight together. Four chunks of 64 columns at a time, and the coefficients' loads depend on the
+// position alone, not on the column just read, so that columns and coefficients travel together and
+// only the gather of the element values waits.
 template <class TC>
 __global__ __launch_bounds__(256) void k_nf_apply(int ntl, const int32_t *__restrict__ tl_tb,
                                                   const int32_t *__restrict__ tl_te, const int64_t *__restrict__ lc_ptr,
@@ -1328,22 +1332,30 @@ __global__ __launch_bounds__(256) void k_nf_apply(int ntl, const int32_t *__rest
 #pragma unroll
         for (int i = 0; i < 4; i++) vb[i] = nf_ptr[t0 + min(i, nt - 1)];
         double au[4] = {0, 0, 0, 0}, av[4] = {0, 0, 0, 0};
-        constexpr int U = 2;  // column chunks per iteration: both chunks' gathers are issued first
+        constexpr int U = 4;
         for (int j0 = lane; j0 < nc; j0 += 64 * U) {
             int col[U];
+            TC val[4][U];
 #pragma unroll
-            for (int u = 0; u < U; u++) col[u] = j0 + 64 * u < nc ? lc_col[cb + j0 + 64 * u] : -1;
+            for (int u = 0; u < U; u++) col[u] = lc_col[cb + min(j0 + 64 * u, nc - 1)];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i < nt)
+#pragma unroll
+                    for (int u = 0; u < U; u++) val[i][u] = nf_val[vb[i] + min(j0 + 64 * u, nc - 1)];
             double2 q[U];
 #pragma unroll
-            for (int u = 0; u < U; u++) q[u] = col[u] >= 0 ? qe[col[u]] : make_double2(0.0, 0.0);
+            for (int u = 0; u < U; u++) {
+                q[u] = qe[col[u]];
+                if (j0 + 64 * u >= nc) q[u] = make_double2(0.0, 0.0);
+            }
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 if (i < nt) {
 #pragma unroll
                     for (int u = 0; u < U; u++) {
-                        const double v = col[u] >= 0 ? (double)nf_val[vb[i] + j0 + 64 * u] : 0.0;
-                        au[i] += v * q[u].x;
-                        av[i] += v * q[u].y;
+                        au[i] += (double)val[i][u] * q[u].x;
+                        av[i] += (double)val[i][u] * q[u].y;
                     }
                 }
         }
