@@ -22,8 +22,9 @@ struct KernelStat {
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
-    // a second stream (default priority) on which the FMM's near field, M2L and L2L run beside M2P:
-    // ev_mid (multipoles complete) forks it, ev_join joins it before the final per-target sum
+    // a second stream (default priority) on which the FMM's coarse M2M, M2L and L2L run beside the
+    // near field and M2P: ev_mid (multipoles of M2P's levels complete) forks it, ev_join joins it
+    // before the final per-target sum
     hipStream_t aux = nullptr;
     hipEvent_t ev_mid = nullptr, ev_join = nullptr;
     fg_options opt{};

@@ -97,6 +97,7 @@ struct FmmPlan {
     double mscale = 1.0;         // expansions times mscale (a power of two) in the FP32 mode
     int64_t m2p_pairs = 0, m2l_pairs = 0, lc_cols = 0;
     int64_t m2p_slots = 0, m2p_far_pairs = 0;  // lane slots the M2P launch mapping executes (useful pairs / slots = SIMD efficiency)
+    int m2p_lmin = 0;   // coarsest level of a source cell that M2P evaluates
     int m2p_ntask = 0;  // M2P tasks (m2p_tasks) and the partial sums of every target
     int4 *d_m2p_task = nullptr, *d_tgt_far = nullptr;
     int64_t nf_nnz = 0;
@@ -1996,6 +1997,8 @@ int fmm_create(Ctx &c)
             size_t npart = 0;
             const std::vector<int4> tk = m2p_tasks(*P, tf, npart);
             P->m2p_ntask = (int)tk.size();
+            P->m2p_lmin = P->Lmax;
+            for (int32_t ci : P->u_cell) P->m2p_lmin = std::min(P->m2p_lmin, (int)P->cen[ci].w);
             P->d_m2p_task = dput(tk);
             P->d_tgt_far = dput(tf);
             void *d = nullptr;
@@ -2247,13 +2250,33 @@ static void run_fmm(Ctx &c)
     FmmPlan &P = *c.fmm;
     const int NL = (int)P.leaf_cell.size();
     F *M = (F *)P.d_M, *Lx = (F *)P.d_L;
-    // The near field reads the element values and corrections and writes potentials that only the
-    // final sum reads, and M2L and L2L need the multipoles only: once M2M is done all three run on
-    // the second stream beside M2P (memory latency and matrix-core work against VALU issue). Beside
-    // P2M and M2M the near field slowed them more than it gained. Profiled runs keep one stream, so
-    // each kernel's time is its own.
+    // M2P needs the multipoles of the two finest levels of each tree only, and nothing of the coarser
+    // M2M levels, M2L and L2L before the final sum: once M2M has reached those levels the coarse
+    // M2M, M2L and L2L (a chain of small launches) run on the second stream beside the near field
+    // and M2P. The near field itself goes first on the main stream: beside M2P, whose wavefronts
+    // take all registers of a SIMD, it finished after it (1.3 ms against 0.31 alone on the 2M film),
+    // and beside P2M and the fine M2M it slowed them more than it gained. Profiled runs keep one
+    // stream, so each kernel's time is its own.
     const bool fork = !c.opt.profile && c.aux;
     hipStream_t ns = fork ? c.aux : c.stream;
+    // M2M onto the parents of levels hi down to lo
+    auto m2m = [&](int hi, int lo, hipStream_t st) {
+        Prof pr(c, "fmm_m2m");
+        for (int l = hi; l >= lo; l--) {
+            const int n = P.m2m_lev_off[l + 1] - P.m2m_lev_off[l];
+            if (n == 0) continue;
+            // a block per row tile where parents are few (a level then takes as long as one
+            // block), all row tiles in one block where they are many
+            if (n >= M2M_ALL_MIN)
+                k_fmm_m2m_all<PP, F><<<(n + 15) / 16 * 2, 256, 0, st>>>(
+                    n, P.d_m2m_cells + P.m2m_lev_off[l], P.d_m2m_child + (size_t)8 * P.m2m_lev_off[l],
+                    (const F *)(std::is_same<F, float>::value ? P.d_Tm2m_pair : P.d_Tm2m), M);
+            else
+                k_fmm_xlate<PP, 0, F><<<(n + 15) / 16 * 2 * XL<PP>::NT, 256, 0, st>>>(
+                    n, P.d_m2m_cells + P.m2m_lev_off[l], P.d_m2m_child + (size_t)8 * P.m2m_lev_off[l],
+                    (const F *)P.d_Tm2m, M);
+        }
+    };
     {
         Prof pr(c, "fmm_p2m");
         constexpr int G = 8;  // lanes per leaf (4 measured slower: longer per-lane source loops)
@@ -2276,37 +2299,19 @@ static void run_fmm(Ctx &c)
             }
         }
     }
-    {
-        Prof pr(c, "fmm_m2m");
-        for (int l = P.Lmax - 1; l >= 2; l--) {
-            const int n = P.m2m_lev_off[l + 1] - P.m2m_lev_off[l];
-            if (n == 0) continue;
-            // a block per row tile where parents are few (a level then takes as long as one
-            // block), all row tiles in one block where they are many
-            if (n >= M2M_ALL_MIN)
-                k_fmm_m2m_all<PP, F><<<(n + 15) / 16 * 2, 256, 0, c.stream>>>(
-                    n, P.d_m2m_cells + P.m2m_lev_off[l], P.d_m2m_child + (size_t)8 * P.m2m_lev_off[l],
-                    (const F *)(std::is_same<F, float>::value ? P.d_Tm2m_pair : P.d_Tm2m), M);
-            else
-                k_fmm_xlate<PP, 0, F><<<(n + 15) / 16 * 2 * XL<PP>::NT, 256, 0, c.stream>>>(
-                    n, P.d_m2m_cells + P.m2m_lev_off[l], P.d_m2m_child + (size_t)8 * P.m2m_lev_off[l],
-                    (const F *)P.d_Tm2m, M);
-        }
-    }
-    // the near field and the downward pass (M2L, L2L) on the second stream once the multipoles are
-    // complete, beside M2P
-    if (fork) {
-        if (hipEventRecord(c.ev_mid, c.stream) != hipSuccess || hipStreamWaitEvent(c.aux, c.ev_mid, 0) != hipSuccess)
-            throw std::string("hipEventRecord / hipStreamWaitEvent (downward-pass fork)");
-    }
+    const int fine = std::max(2, P.m2p_lmin);
+    m2m(P.Lmax - 1, fine, c.stream);
+    if (fork && (hipEventRecord(c.ev_mid, c.stream) != hipSuccess || hipStreamWaitEvent(ns, c.ev_mid, 0) != hipSuccess))
+        throw std::string("hipEventRecord / hipStreamWaitEvent (fork beside M2P)");
+    m2m(fine - 1, 2, ns);
     {
         Prof pr(c, "fmm_near");
         const unsigned nb = (unsigned)(((int64_t)P.ntl * 64 + 255) / 256);
         if (P.ntl > 0 && P.d_nf_valf)
-            k_nf_apply<float><<<nb, 256, 0, ns>>>(P.ntl, P.d_tl_tb, P.d_tl_te, P.d_lc_ptr, P.d_lc_col, P.d_nf_ptr,
+            k_nf_apply<float><<<nb, 256, 0, c.stream>>>(P.ntl, P.d_tl_tb, P.d_tl_te, P.d_lc_ptr, P.d_lc_col, P.d_nf_ptr,
                                                   P.d_nf_valf, c.qe, P.d_tgt_node, c.corr, P.d_pot);
         else if (P.ntl > 0)
-            k_nf_apply<double><<<nb, 256, 0, ns>>>(P.ntl, P.d_tl_tb, P.d_tl_te, P.d_lc_ptr, P.d_lc_col, P.d_nf_ptr,
+            k_nf_apply<double><<<nb, 256, 0, c.stream>>>(P.ntl, P.d_tl_tb, P.d_tl_te, P.d_lc_ptr, P.d_lc_col, P.d_nf_ptr,
                                                    P.d_nf_val, c.qe, P.d_tgt_node, c.corr, P.d_pot);
     }
 
@@ -2349,7 +2354,7 @@ static void run_fmm(Ctx &c)
                 go(k_fmm_m2p<PP, PP, PV, F>);
         }
     }
-    // join: the near field, M2L and L2L are in
+    // join: M2L and L2L are in
     if (fork && hipStreamWaitEvent(c.stream, c.ev_join, 0) != hipSuccess)
         throw std::string("hipStreamWaitEvent (join)");
     {
