@@ -20,14 +20,45 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace fg {
 
 // ------------------------------------------------------------------ reductions
+// Value of another lane of the row of 16 through a data-parallel-primitive move (no LDS round trip):
+// CTRL 0xB1 swaps within pairs, 0x4E pairs within quads, 0x141 mirrors half rows, 0x140 rows.
+template <int CTRL>
+__device__ inline double dpp_mov(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// the moves within quads, either precision (the lanes of a row of the stencil)
+template <int CTRL>
+__device__ inline double quad_mov(double v) { return dpp_mov<CTRL>(v); }
+template <int CTRL>
+__device__ inline float quad_mov(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ inline double read_lane(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Sum over the wavefront, in every lane (all 64 active): rows of 16 by DPP moves, then the four rows.
+// The six dependent LDS shuffles of a butterfly were about 0.4 us of every reduction.
 __device__ inline double wave_sum(double v)
 {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    v += dpp_mov<0xB1>(v);
+    v += dpp_mov<0x4E>(v);
+    v += dpp_mov<0x141>(v);
+    v += dpp_mov<0x140>(v);
+    return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 __device__ inline double wave_max(double v)
 {
@@ -62,9 +93,6 @@ __device__ inline double lane_fold(const double *__restrict__ p, int nb, double 
 }
 struct AddOp {
     __device__ double operator()(double a, double b) const { return a + b; }
-};
-struct MaxOp {
-    __device__ double operator()(double a, double b) const { return fmax(a, b); }
 };
 struct MinOp {
     __device__ double operator()(double a, double b) const { return fmin(a, b); }
@@ -296,8 +324,9 @@ __global__ __launch_bounds__(BLOCK) void k_node_assemble(
     const double4 *__restrict__ eout, const double *__restrict__ mass,
     const double *__restrict__ sdiag, double4 *__restrict__ ep4, double4 *__restrict__ eq4,
     double4 *__restrict__ Dg, double2 *__restrict__ dprec, double2 *__restrict__ b,
-    double2 *__restrict__ x, double4 *__restrict__ w, double *__restrict__ part)
+    double2 *__restrict__ x, double4 *__restrict__ w, double *__restrict__ part, KrylovCtl *ctl)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->vmax2 = 0.0;  // k_update takes maxima into it
     double bb = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
         const NodeRec n = cur[i];
@@ -346,28 +375,107 @@ __global__ __launch_bounds__(BLOCK) void k_node_assemble(
 }
 
 // ------------------------------------------------------------------ stencil SpMV
+// Form (FORM) of the solver's kernels, by the mesh's size (krylov_shape):
+//   4: four lanes per row, and BLOCK / 4 rows per block in the vector phases, where a lane per row
+//      would leave most CUs idle and each row one serial chain of gathers;
+//   1: a lane per row, four stencil entries in flight, while the rows fit one pass of the grid: bound
+//      by the latency of the gathers;
+//   0: a lane per row, one entry after another: with many wavefronts per SIMD to hide the latency the
+//      fewer registers and instructions win.
+// Per product, the old form (0) and the new one: 8.7 -> 5.3 us on 9,261 nodes (4), 16.1 -> 14.0 us on
+// 98,784 (1); 39.2 (0) against 41.5 (1) us on 392,784.
+__device__ constexpr int form_lanes(int form) { return form == 4 ? 4 : 1; }
+// The first row of this thread and the rows between its passes: stencil kernels (lane sub of the
+// row's lanes) and vector kernels (one lane per row; lanes past the block's rows have none).
+template <int FORM>
+__device__ inline int row_first(int blk) { return blk * (BLOCK / form_lanes(FORM)) + (int)threadIdx.x / form_lanes(FORM); }
+template <int FORM>
+__device__ inline int vec_first(int blk, int N)
+{
+    constexpr int RB = BLOCK / form_lanes(FORM);
+    return (int)threadIdx.x < RB ? blk * RB + (int)threadIdx.x : N;
+}
+template <int FORM>
+__device__ inline int row_step() { return (int)gridDim.x * (BLOCK / form_lanes(FORM)); }
+template <int FORM>
+__device__ inline int row_sub() { return (int)threadIdx.x & (form_lanes(FORM) - 1); }
+
+// z_i = sum_j S'_ij w_j, in every lane of the row (lane sub of LPR takes entries sub, sub + LPR, ...);
+// but in form 0 four entries' columns and values are loaded together, then their w.
+template <int FORM, class T, class T4>
+__device__ inline void stencil_sum(int i, int sub, const int64_t *__restrict__ sptr, const int32_t *__restrict__ swid,
+                                   const int32_t *__restrict__ scol, const T *__restrict__ sval,
+                                   const T4 *__restrict__ w, T &zx, T &zy, T &zz)
+{
+    const int sl = i >> 6, lane = i & 63;
+    const int width = swid[sl];
+    const int64_t off = sptr[sl] + lane;
+    constexpr int U = 4, LPR = form_lanes(FORM);
+    zx = zy = zz = 0;
+    if constexpr (FORM == 0) {
+        for (int k = 0; k < width; k++) {
+            const int64_t e = off + (int64_t)k * SELL_C;
+            const int j = scol[e];
+            const T v = sval[e];
+            const T4 x = w[j];
+            zx += v * x.x;
+            zy += v * x.y;
+            zz += v * x.z;
+        }
+        return;
+    }
+    for (int k0 = sub; k0 < width; k0 += LPR * U) {
+        int j[U];
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = k0 + LPR * u;
+            const int64_t e = off + (int64_t)min(k, width - 1) * SELL_C;
+            j[u] = scol[e];
+            v[u] = sval[e];
+            if (k >= width) v[u] = 0;
+        }
+        T4 x[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) x[u] = w[j[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            zx += v[u] * x[u].x;
+            zy += v[u] * x[u].y;
+            zz += v[u] * x[u].z;
+        }
+    }
+    if constexpr (LPR == 4) {
+        zx += quad_mov<0xB1>(zx);
+        zy += quad_mov<0xB1>(zy);
+        zz += quad_mov<0xB1>(zz);
+        zx += quad_mov<0x4E>(zx);
+        zy += quad_mov<0x4E>(zy);
+        zz += quad_mov<0x4E>(zz);
+    }
+}
+
 // y_i = c [eq_i . z_i, ep_i . z_i] + Dg_i x_i with z_i = sum_j S'_ij w_j, zero for
 // non-magnetic rows (applyMask after mult, src/algebra/bicg.h:201,216).
+template <int FORM = 0>
 __device__ inline double2 stencil_row(int i, double cst, const int64_t *__restrict__ sptr,
                                       const int32_t *__restrict__ swid, const int32_t *__restrict__ scol,
                                       const double *__restrict__ sval, const double4 *__restrict__ w,
                                       const double4 *__restrict__ ep4, const double4 *__restrict__ eq4,
-                                      const double4 *__restrict__ Dg, double2 xi)
+                                      const double4 *__restrict__ Dg, double2 xi, int sub = 0)
 {
-    const int sl = i >> 6, lane = i & 63;
-    const int64_t off = sptr[sl];
-    const int width = swid[sl];
-    double zx = 0, zy = 0, zz = 0;
-    for (int k = 0; k < width; k++) {
-        const int64_t e = off + (int64_t)k * SELL_C + lane;
-        const int j = scol[e];
-        const double sv = sval[e];
-        const double4 wj = w[j];
-        zx += sv * wj.x;
-        zy += sv * wj.y;
-        zz += sv * wj.z;
-    }
-    const double4 p = ep4[i], q = eq4[i], g = Dg[i];
+    // on small meshes the row's own data is read under the gathers, on large ones after them (more
+    // wavefronts in flight)
+    double4 p, q, g;
+    auto own = [&]() {
+        p = ep4[i];
+        q = eq4[i];
+        g = Dg[i];
+    };
+    if constexpr (FORM == 4) own();
+    double zx, zy, zz;
+    stencil_sum<FORM>(i, sub, sptr, swid, scol, sval, w, zx, zy, zz);
+    if constexpr (FORM != 4) own();
     double2 y;
     y.x = cst * (q.x * zx + q.y * zy + q.z * zz) + (g.x * xi.x + g.y * xi.y);
     y.y = cst * (p.x * zx + p.y * zy + p.z * zz) + (g.z * xi.x + g.w * xi.y);
@@ -381,44 +489,50 @@ __device__ inline double2 stencil_row(int i, double cst, const int64_t *__restri
         const double4 *__restrict__ Dg, const int32_t *__restrict__ mag
 #define STENCIL_PASS c.slice_ptr, c.slice_w, c.scol, c.sval, c.ep4, c.eq4, c.Dg, c.mag
 
-// r = b - A x (masked); rt = r; p = r; partials ||r||^2, rt.r  (src/algebra/bicg.h:172-184)
-__global__ __launch_bounds__(BLOCK) void k_r0(int N, double cst, STENCIL_ARGS, const double4 *__restrict__ w,
+// ||b|| from the assembly's partials (one wavefront)
+__device__ inline double rhs_norm(const double *__restrict__ part, int nb)
+{
+    return sqrt(fabs(wave_sum(lane_fold(part, nb, 0.0, AddOp()))));
+}
+
+// r = b - A x (masked); rt = r; p = r; partials ||r||^2, rt.r  (src/algebra/bicg.h:172-184); block 0
+// sets ||b|| (nba: the assembly's blocks) and the loop's scalars
+template <int FORM>
+__global__ __launch_bounds__(BLOCK) void k_r0(int N, int nba, double cst, STENCIL_ARGS, const double4 *__restrict__ w,
                                               const double2 *__restrict__ x, const double2 *__restrict__ b,
                                               double2 *__restrict__ r, double2 *__restrict__ rt,
                                               double2 *__restrict__ p, KrylovCtl *ctl, double *__restrict__ part)
 {
     double rr = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+    const int sub = row_sub<FORM>();
+    for (int i = row_first<FORM>(blockIdx.x); i < N; i += row_step<FORM>()) {
         double2 ri = make_double2(0, 0);
         if (mag[i]) {
-            const double2 y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, x[i]);
             const double2 bi = b[i];
+            const double2 y = stencil_row<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, x[i], sub);
             ri = make_double2(bi.x - y.x, bi.y - y.y);
         }
-        r[i] = ri;
-        rt[i] = ri;
-        p[i] = ri;
-        rr += ri.x * ri.x + ri.y * ri.y;
+        if (sub == 0) {
+            r[i] = ri;
+            rt[i] = ri;
+            p[i] = ri;
+            rr += ri.x * ri.x + ri.y * ri.y;
+        }
     }
     // rt = r, so rt . r = ||r||^2 for the first iteration
     const double vals[2] = {rr, rr};
     const int slots[2] = {1, 2};
     block_store<2>(vals, slots, part, blockIdx.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctl->nit = 0;
-        ctl->status = -1;
-        ctl->done = ctl->stop = 0;
-        ctl->rho1 = ctl->rho2 = ctl->alpha = ctl->omega = ctl->beta = 0.0;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        const double bn = rhs_norm(part, nba);
+        if (threadIdx.x == 0) {
+            ctl->rhsn = bn;
+            ctl->nit = 0;
+            ctl->status = -1;
+            ctl->done = ctl->stop = 0;
+            ctl->rho1 = ctl->rho2 = ctl->alpha = ctl->omega = ctl->beta = 0.0;
+        }
     }
-}
-
-// ||b|| into the control block (one block)
-__global__ void k_set_rhsn(int nb, KrylovCtl *ctl, const double *__restrict__ part)
-{
-    const int slots[1] = {0};
-    double v[1];
-    block_load<1>(part, slots, nb, v);
-    if (threadIdx.x == 0) ctl->rhsn = sqrt(fabs(v[0]));
 }
 
 // Batched instances: ||b_k||^2 of each instance (one block per instance), then the stopping scale
@@ -451,8 +565,14 @@ __global__ void k_inst_rhsn(int K, const double *__restrict__ n2, KrylovCtl *ctl
     if (mn > 0) ctl->rhsn = sqrt(mn);
 }
 
+// The five phases of an iteration. On small meshes each is a chain of dependent memory reads (the
+// control block, the last phase's partials, the rows) of about a microsecond each, so a phase issues
+// all three together and decides afterwards; a row read by a phase that then has nothing to do is
+// read in vain.
+
 // (C) loop head: convergence on ||r||, rho_1 = rt.r, beta, p = r + beta (p - omega v),
 // p^ = D p, w = lift(p^)  (src/algebra/bicg.h:180-199)
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void k_iter_p(int N, int nb, KrylovCtl *ctl, const double4 *__restrict__ ep4,
                                                   const double4 *__restrict__ eq4,
                                                   const double2 *__restrict__ dprec,
@@ -460,29 +580,42 @@ __global__ __launch_bounds__(BLOCK) void k_iter_p(int N, int nb, KrylovCtl *ctl,
                                                   double2 *__restrict__ p, double2 *__restrict__ ph,
                                                   double4 *__restrict__ w, const double *__restrict__ part)
 {
-    if (ctl->done) return;
+    int i = vec_first<FORM>(blockIdx.x, N);
+    double2 ri, vi, pi, d;
+    double4 e, q;
+    auto load = [&]() {
+        ri = r[i];
+        vi = v[i];
+        pi = p[i];
+        d = dprec[i];
+        e = ep4[i];
+        q = eq4[i];
+    };
+    if (i < N) load();
+    const KrylovCtl k = *ctl;
     const int slots[2] = {1, 2};
     double red[2];
     block_load<2>(part, slots, nb, red);
+    if (k.done) return;
     const double res = sqrt(fabs(red[0]));
     const double rho1 = red[1];
-    const int nit = ctl->nit;
-    int status = ctl->status, done = 0;
+    const int nit = k.nit;
+    int status = k.status, done = 0;
     if (isnan(res)) {
         status = 2;
         done = 1;
-    } else if (res <= ctl->rhsn * ctl->tol) {
+    } else if (res <= k.rhsn * k.tol) {
         status = 0;
         done = 1;
     }
     double beta = 0;
-    const double omega = ctl->omega;
+    const double omega = k.omega;
     if (!done && nit > 0) {
-        if (ctl->rho2 == 0 || omega == 0) {
+        if (k.rho2 == 0 || omega == 0) {
             status = 2;
             done = 1;
         } else {
-            beta = (rho1 / ctl->rho2) * (ctl->alpha / omega);
+            beta = (rho1 / k.rho2) * (k.alpha / omega);
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -493,47 +626,51 @@ __global__ __launch_bounds__(BLOCK) void k_iter_p(int N, int nb, KrylovCtl *ctl,
         if (done) ctl->done = 1;
     }
     if (done) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        double2 pi;
-        const double2 ri = r[i];
+    while (i < N) {
         if (nit > 0) {
-            const double2 vi = v[i];
-            pi = p[i];
             pi.x = (pi.x - omega * vi.x) * beta + ri.x;
             pi.y = (pi.y - omega * vi.y) * beta + ri.y;
         } else {
             pi = ri;
         }
         p[i] = pi;
-        const double2 d = dprec[i];
         const double2 h = make_double2(d.x * pi.x, d.y * pi.y);
         ph[i] = h;
-        const double4 e = ep4[i], q = eq4[i];
         w[i] = make_double4(h.x * e.x + h.y * q.x, h.x * e.y + h.y * q.y, h.x * e.z + h.y * q.z, 0.0);
+        i += row_step<FORM>();
+        if (i < N) load();
     }
 }
 
 // (D) v = A p^ (masked); partial v . rt
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void k_spmv_v(int N, double cst, STENCIL_ARGS, const KrylovCtl *ctl,
                                                   const double4 *__restrict__ w, const double2 *__restrict__ ph,
                                                   const double2 *__restrict__ rt, double2 *__restrict__ v,
                                                   double *__restrict__ part)
 {
-    if (ctl->done) return;
+    const int sub = row_sub<FORM>();
+    const int done = ctl->done;
     double vr = 0;
-    for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+    for (int i = row_first<FORM>(lblock()); i < N; i += row_step<FORM>()) {
+        if (FORM == 0 && done) return;
         double2 y = make_double2(0, 0);
-        if (mag[i]) y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i]);
-        v[i] = y;
-        const double2 q = rt[i];
-        vr += y.x * q.x + y.y * q.y;
+        if (mag[i]) y = stencil_row<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i], sub);
+        if (done) return;
+        if (sub == 0) {
+            v[i] = y;
+            const double2 q = rt[i];
+            vr += y.x * q.x + y.y * q.y;
+        }
     }
+    if (done) return;
     const double vals[1] = {vr};
     const int slots[1] = {3};
     block_store<1>(vals, slots, part, lblock());
 }
 
 // (E) alpha = rho_1 / (v . rt); s = r - alpha v; s^ = D s; w = lift(s^); partial ||s||^2
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void k_iter_s(int N, int nb, KrylovCtl *ctl, const double4 *__restrict__ ep4,
                                                   const double4 *__restrict__ eq4,
                                                   const double2 *__restrict__ dprec,
@@ -541,23 +678,35 @@ __global__ __launch_bounds__(BLOCK) void k_iter_s(int N, int nb, KrylovCtl *ctl,
                                                   double2 *__restrict__ s, double2 *__restrict__ sh,
                                                   double4 *__restrict__ w, double *__restrict__ part)
 {
-    if (ctl->done) return;
+    int i = vec_first<FORM>(blockIdx.x, N);
+    double2 ri, vi, d;
+    double4 e, q;
+    auto load = [&]() {
+        ri = r[i];
+        vi = v[i];
+        d = dprec[i];
+        e = ep4[i];
+        q = eq4[i];
+    };
+    if (i < N) load();
+    const int done = ctl->done;
+    const double rho1 = ctl->rho1;
     const int slots[1] = {3};
     double red[1];
     block_load<1>(part, slots, nb, red);
-    const double alpha = ctl->rho1 / red[0];
+    if (done) return;
+    const double alpha = rho1 / red[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl->alpha = alpha;
     double ss = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        const double2 ri = r[i], vi = v[i];
+    while (i < N) {
         const double2 si = make_double2(ri.x + (-alpha) * vi.x, ri.y + (-alpha) * vi.y);
         s[i] = si;
         ss += si.x * si.x + si.y * si.y;
-        const double2 d = dprec[i];
         const double2 h = make_double2(d.x * si.x, d.y * si.y);
         sh[i] = h;
-        const double4 e = ep4[i], q = eq4[i];
         w[i] = make_double4(h.x * e.x + h.y * q.x, h.x * e.y + h.y * q.y, h.x * e.z + h.y * q.z, 0.0);
+        i += row_step<FORM>();
+        if (i < N) load();
     }
     const double vals[1] = {ss};
     const int slots2[1] = {4};
@@ -566,23 +715,35 @@ __global__ __launch_bounds__(BLOCK) void k_iter_s(int N, int nb, KrylovCtl *ctl,
 
 // (F) convergence on ||s|| (x += alpha p^ when converged), else t = A s^ (masked);
 // partials t.s, t.t  (src/algebra/bicg.h:206-217)
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STENCIL_ARGS, KrylovCtl *ctl,
                                                   const double4 *__restrict__ w, const double2 *__restrict__ sh,
                                                   const double2 *__restrict__ s, const double2 *__restrict__ ph,
                                                   double2 *__restrict__ x, double2 *__restrict__ t,
                                                   double *__restrict__ part)
 {
-    if (ctl->done) return;
+    const int sub = row_sub<FORM>();
+    int i = row_first<FORM>(lblock());
+    // the first row's product goes under the reads of the control block and the partials (but form 0)
+    double2 y = make_double2(0, 0), si = make_double2(0, 0);
+    auto row = [&]() {
+        y = make_double2(0, 0);
+        if (mag[i]) y = stencil_row<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, sh[i], sub);
+        si = s[i];
+    };
+    const KrylovCtl k = *ctl;
+    if (FORM != 0 && i < N) row();
     const int slots[1] = {4};
     double red[1];
     block_load<1>(part, slots, nb, red);
+    if (k.done) return;
     const double res = sqrt(fabs(red[0]));
-    int status = ctl->status, done = 0;
+    int status = k.status, done = 0;
     bool conv = false;
     if (isnan(res)) {
         status = 2;
         done = 1;
-    } else if (res <= ctl->rhsn * ctl->tol) {
+    } else if (res <= k.rhsn * k.tol) {
         status = 0;
         done = 1;
         conv = true;
@@ -595,9 +756,9 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STE
         ctl->stop = 1;
     }
     if (done) {
-        if (conv) {
-            const double alpha = ctl->alpha;
-            for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+        if (conv && sub == 0) {
+            const double alpha = k.alpha;
+            for (; i < N; i += row_step<FORM>()) {
                 double2 xi = x[i];
                 const double2 h = ph[i];
                 xi.x += alpha * h.x;
@@ -608,13 +769,15 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STE
         return;
     }
     double ts = 0, tt = 0;
-    for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        double2 y = make_double2(0, 0);
-        if (mag[i]) y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, sh[i]);
-        t[i] = y;
-        const double2 si = s[i];
-        ts += y.x * si.x + y.y * si.y;
-        tt += y.x * y.x + y.y * y.y;
+    if (FORM == 0 && i < N) row();
+    while (i < N) {
+        if (sub == 0) {
+            t[i] = y;
+            ts += y.x * si.x + y.y * si.y;
+            tt += y.x * y.x + y.y * y.y;
+        }
+        i += row_step<FORM>();
+        if (i < N) row();
     }
     const double vals[2] = {ts, tt};
     const int slots2[2] = {5, 6};
@@ -622,26 +785,37 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STE
 }
 
 // (G) omega = (t.s)/(t.t); x += alpha p^ + omega s^; r = s - omega t; partials ||r||^2, rt.r
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void k_iter_x(int N, int nb, KrylovCtl *ctl, const double2 *__restrict__ ph,
                                                   const double2 *__restrict__ sh, const double2 *__restrict__ s,
                                                   const double2 *__restrict__ t, const double2 *__restrict__ rt,
                                                   double2 *__restrict__ x, double2 *__restrict__ r,
                                                   double *__restrict__ part)
 {
-    if (ctl->done) return;
-    if (ctl->stop) {  // stopped on ||s|| by the previous phase
-        if (blockIdx.x == 0 && threadIdx.x == 0) ctl->done = 1;
-        return;
-    }
+    int i = vec_first<FORM>(blockIdx.x, N);
+    double2 xi, h, hs, si, ti, q;
+    auto load = [&]() {
+        xi = x[i];
+        h = ph[i];
+        hs = sh[i];
+        si = s[i];
+        ti = t[i];
+        q = rt[i];
+    };
+    if (i < N) load();
+    const KrylovCtl k = *ctl;
     const int slots[2] = {5, 6};
     double red[2];
     block_load<2>(part, slots, nb, red);
+    if (k.done) return;
+    if (k.stop) {  // stopped on ||s|| by the previous phase
+        if (blockIdx.x == 0 && threadIdx.x == 0) ctl->done = 1;
+        return;
+    }
     const double omega = red[0] / red[1];
-    const double alpha = ctl->alpha;
+    const double alpha = k.alpha;
     double rr = 0, rtr = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        double2 xi = x[i];
-        const double2 h = ph[i], hs = sh[i], si = s[i], ti = t[i], q = rt[i];
+    while (i < N) {
         xi.x += alpha * h.x;
         xi.y += alpha * h.y;
         xi.x += omega * hs.x;
@@ -651,16 +825,18 @@ __global__ __launch_bounds__(BLOCK) void k_iter_x(int N, int nb, KrylovCtl *ctl,
         r[i] = ri;
         rr += ri.x * ri.x + ri.y * ri.y;
         rtr += q.x * ri.x + q.y * ri.y;
+        i += row_step<FORM>();
+        if (i < N) load();
     }
     const double vals[2] = {rr, rtr};
     const int slots2[2] = {1, 2};
     block_store<2>(vals, slots2, part, blockIdx.x);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl->omega = omega;
-        ctl->rho2 = ctl->rho1;
-        const int nit = ctl->nit + 1;
+        ctl->rho2 = k.rho1;
+        const int nit = k.nit + 1;
         ctl->nit = nit;
-        if (nit >= ctl->max_iter) ctl->status = 1;
+        if (nit >= k.max_iter) ctl->status = 1;
     }
 }
 
@@ -853,26 +1029,16 @@ __global__ __launch_bounds__(BS) void k_bicg_batch(const int32_t *__restrict__ o
 // loop's scalars and stopping rules (src/algebra/bicg.h:162-234); the outer block (ctl) keeps
 // ||b||, the tolerance, the status and the counts.
 
+template <int FORM>
 __device__ inline float2 stencil_row_f(int i, float cst, const int64_t *__restrict__ sptr,
                                        const int32_t *__restrict__ swid, const int32_t *__restrict__ scol,
                                        const float *__restrict__ sval, const float4 *__restrict__ w,
                                        const float4 *__restrict__ ep4, const float4 *__restrict__ eq4,
-                                       const float4 *__restrict__ Dg, float2 xi)
+                                       const float4 *__restrict__ Dg, float2 xi, int sub)
 {
-    const int sl = i >> 6, lane = i & 63;
-    const int64_t off = sptr[sl];
-    const int width = swid[sl];
-    float zx = 0, zy = 0, zz = 0;
-    for (int k = 0; k < width; k++) {
-        const int64_t e = off + (int64_t)k * SELL_C + lane;
-        const int j = scol[e];
-        const float sv = sval[e];
-        const float4 wj = w[j];
-        zx += sv * wj.x;
-        zy += sv * wj.y;
-        zz += sv * wj.z;
-    }
     const float4 p = ep4[i], q = eq4[i], g = Dg[i];
+    float zx, zy, zz;
+    stencil_sum<FORM>(i, sub, sptr, swid, scol, sval, w, zx, zy, zz);
     float2 y;
     y.x = cst * (q.x * zx + q.y * zy + q.z * zz) + (g.x * xi.x + g.y * xi.y);
     y.y = cst * (p.x * zx + p.y * zy + p.z * zz) + (g.z * xi.x + g.w * xi.y);
@@ -908,11 +1074,12 @@ __global__ __launch_bounds__(BLOCK) void k_to_f32(int N, const double4 *__restri
     }
 }
 
-// the outer loop's start (||b||, or the batch's criterion, is set by the assembly): counts and
-// status reset
-__global__ void k_mixed_init(KrylovCtl *ctl)
+// the outer loop's start: ||b|| from the assembly's partials, counts and status reset
+__global__ void k_mixed_init(int nba, KrylovCtl *ctl, const double *__restrict__ part)
 {
+    const double bn = rhs_norm(part, nba);
     if (threadIdx.x == 0) {
+        ctl->rhsn = bn;
         ctl->nit = 0;
         ctl->status = -1;
         ctl->done = ctl->stop = 0;
@@ -924,6 +1091,7 @@ __global__ void k_mixed_init(KrylovCtl *ctl)
 // FP64 residual r = b - A x (masked, with w = lift(x)); r in FP32 as the inner right-hand side,
 // rt = p = r, d = 0; partials: slot 0 the FP64 ||r||^2, slots 1 and 2 the FP32 vector's (the inner
 // loop's first ||r|| and rt . r)
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void k_resid(int N, double cst, STENCIL_ARGS, const KrylovCtl *ctl,
                                                  const double4 *__restrict__ w, const double2 *__restrict__ x,
                                                  const double2 *__restrict__ b, float2 *__restrict__ rf,
@@ -931,14 +1099,16 @@ __global__ __launch_bounds__(BLOCK) void k_resid(int N, double cst, STENCIL_ARGS
                                                  float2 *__restrict__ df, double *__restrict__ part)
 {
     if (ctl->done) return;
+    const int sub = row_sub<FORM>();
     double rr = 0, ff = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+    for (int i = row_first<FORM>(blockIdx.x); i < N; i += row_step<FORM>()) {
         double2 ri = make_double2(0, 0);
         if (mag[i]) {
-            const double2 y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, x[i]);
             const double2 bi = b[i];
+            const double2 y = stencil_row<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, x[i], sub);
             ri = make_double2(bi.x - y.x, bi.y - y.y);
         }
+        if (sub) continue;
         rr += ri.x * ri.x + ri.y * ri.y;
         const float2 f = make_float2((float)ri.x, (float)ri.y);
         rf[i] = f;
@@ -1005,35 +1175,49 @@ __global__ __launch_bounds__(BLOCK) void k_refine(int N, KrylovCtl *ctl, const K
 }
 
 // The FP32 loop: the same five phases as the FP64 one, on ic
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void kf_iter_p(int N, int nb, KrylovCtl *ic, const float4 *__restrict__ ep4,
                                                    const float4 *__restrict__ eq4, const float2 *__restrict__ dprec,
                                                    const float2 *__restrict__ r, const float2 *__restrict__ v,
                                                    float2 *__restrict__ p, float2 *__restrict__ ph,
                                                    float4 *__restrict__ w, const double *__restrict__ part)
 {
-    if (ic->done) return;
+    int i = vec_first<FORM>(blockIdx.x, N);
+    float2 ri, vi, pi, d;
+    float4 e, q;
+    auto load = [&]() {
+        ri = r[i];
+        vi = v[i];
+        pi = p[i];
+        d = dprec[i];
+        e = ep4[i];
+        q = eq4[i];
+    };
+    if (i < N) load();
+    const KrylovCtl k = *ic;
     const int slots[2] = {1, 2};
     double red[2];
     block_load<2>(part, slots, nb, red);
+    if (k.done) return;
     const double res = sqrt(fabs(red[0]));
     const double rho1 = red[1];
-    const int nit = ic->nit;
-    int status = ic->status, done = 0;
+    const int nit = k.nit;
+    int status = k.status, done = 0;
     if (isnan(res)) {
         status = 2;
         done = 1;
-    } else if (res <= ic->rhsn * ic->tol) {
+    } else if (res <= k.rhsn * k.tol) {
         status = 0;
         done = 1;
     }
     double beta = 0;
-    const double omega = ic->omega;
+    const double omega = k.omega;
     if (!done && nit > 0) {
-        if (ic->rho2 == 0 || omega == 0) {
+        if (k.rho2 == 0 || omega == 0) {
             status = 2;
             done = 1;
         } else {
-            beta = (rho1 / ic->rho2) * (ic->alpha / omega);
+            beta = (rho1 / k.rho2) * (k.alpha / omega);
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -1045,90 +1229,119 @@ __global__ __launch_bounds__(BLOCK) void kf_iter_p(int N, int nb, KrylovCtl *ic,
     }
     if (done) return;
     const float om = (float)omega, be = (float)beta;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        float2 pi;
-        const float2 ri = r[i];
+    while (i < N) {
         if (nit > 0) {
-            const float2 vi = v[i];
-            pi = p[i];
             pi.x = (pi.x - om * vi.x) * be + ri.x;
             pi.y = (pi.y - om * vi.y) * be + ri.y;
         } else {
             pi = ri;
         }
         p[i] = pi;
-        const float2 d = dprec[i];
         const float2 h = make_float2(d.x * pi.x, d.y * pi.y);
         ph[i] = h;
-        w[i] = lift_f(h, ep4[i], eq4[i]);
+        w[i] = lift_f(h, e, q);
+        i += row_step<FORM>();
+        if (i < N) load();
     }
 }
 
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void kf_spmv_v(int N, float cst, STENCIL_ARGS_F, const KrylovCtl *ic,
                                                    const float4 *__restrict__ w, const float2 *__restrict__ ph,
                                                    const float2 *__restrict__ rt, float2 *__restrict__ v,
                                                    double *__restrict__ part)
 {
-    if (ic->done) return;
+    const int sub = row_sub<FORM>();
+    const int done = ic->done;
     double vr = 0;
-    for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+    for (int i = row_first<FORM>(lblock()); i < N; i += row_step<FORM>()) {
+        if (FORM == 0 && done) return;
         float2 y = make_float2(0, 0);
-        if (mag[i]) y = stencil_row_f(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i]);
-        v[i] = y;
-        const float2 q = rt[i];
-        vr += (double)y.x * q.x + (double)y.y * q.y;
+        if (mag[i]) y = stencil_row_f<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i], sub);
+        if (done) return;
+        if (sub == 0) {
+            v[i] = y;
+            const float2 q = rt[i];
+            vr += (double)y.x * q.x + (double)y.y * q.y;
+        }
     }
+    if (done) return;
     const double vals[1] = {vr};
     const int slots[1] = {3};
     block_store<1>(vals, slots, part, lblock());
 }
 
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void kf_iter_s(int N, int nb, KrylovCtl *ic, const float4 *__restrict__ ep4,
                                                    const float4 *__restrict__ eq4, const float2 *__restrict__ dprec,
                                                    const float2 *__restrict__ r, const float2 *__restrict__ v,
                                                    float2 *__restrict__ s, float2 *__restrict__ sh,
                                                    float4 *__restrict__ w, double *__restrict__ part)
 {
-    if (ic->done) return;
+    int i = vec_first<FORM>(blockIdx.x, N);
+    float2 ri, vi, d;
+    float4 e, q;
+    auto load = [&]() {
+        ri = r[i];
+        vi = v[i];
+        d = dprec[i];
+        e = ep4[i];
+        q = eq4[i];
+    };
+    if (i < N) load();
+    const int done = ic->done;
+    const double rho1 = ic->rho1;
     const int slots[1] = {3};
     double red[1];
     block_load<1>(part, slots, nb, red);
-    const double alpha = ic->rho1 / red[0];
+    if (done) return;
+    const double alpha = rho1 / red[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) ic->alpha = alpha;
     const float al = (float)alpha;
     double ss = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        const float2 ri = r[i], vi = v[i];
+    while (i < N) {
         const float2 si = make_float2(ri.x + (-al) * vi.x, ri.y + (-al) * vi.y);
         s[i] = si;
         ss += (double)si.x * si.x + (double)si.y * si.y;
-        const float2 d = dprec[i];
         const float2 h = make_float2(d.x * si.x, d.y * si.y);
         sh[i] = h;
-        w[i] = lift_f(h, ep4[i], eq4[i]);
+        w[i] = lift_f(h, e, q);
+        i += row_step<FORM>();
+        if (i < N) load();
     }
     const double vals[1] = {ss};
     const int slots2[1] = {4};
     block_store<1>(vals, slots2, part, blockIdx.x);
 }
 
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void kf_spmv_t(int N, int nb, float cst, STENCIL_ARGS_F, KrylovCtl *ic,
                                                    const float4 *__restrict__ w, const float2 *__restrict__ sh,
                                                    const float2 *__restrict__ s, const float2 *__restrict__ ph,
                                                    float2 *__restrict__ x, float2 *__restrict__ t,
                                                    double *__restrict__ part)
 {
-    if (ic->done) return;
+    const int sub = row_sub<FORM>();
+    int i = row_first<FORM>(lblock());
+    float2 y = make_float2(0, 0), si = make_float2(0, 0);
+    auto row = [&]() {
+        y = make_float2(0, 0);
+        if (mag[i]) y = stencil_row_f<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, sh[i], sub);
+        si = s[i];
+    };
+    const KrylovCtl k = *ic;
+    if (FORM != 0 && i < N) row();
     const int slots[1] = {4};
     double red[1];
     block_load<1>(part, slots, nb, red);
+    if (k.done) return;
     const double res = sqrt(fabs(red[0]));
-    int status = ic->status, done = 0;
+    int status = k.status, done = 0;
     bool conv = false;
     if (isnan(res)) {
         status = 2;
         done = 1;
-    } else if (res <= ic->rhsn * ic->tol) {
+    } else if (res <= k.rhsn * k.tol) {
         status = 0;
         done = 1;
         conv = true;
@@ -1141,9 +1354,9 @@ __global__ __launch_bounds__(BLOCK) void kf_spmv_t(int N, int nb, float cst, STE
         ic->stop = 1;
     }
     if (done) {
-        if (conv) {
-            const float al = (float)ic->alpha;
-            for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+        if (conv && sub == 0) {
+            const float al = (float)k.alpha;
+            for (; i < N; i += row_step<FORM>()) {
                 float2 xi = x[i];
                 const float2 h = ph[i];
                 xi.x += al * h.x;
@@ -1154,39 +1367,52 @@ __global__ __launch_bounds__(BLOCK) void kf_spmv_t(int N, int nb, float cst, STE
         return;
     }
     double ts = 0, tt = 0;
-    for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        float2 y = make_float2(0, 0);
-        if (mag[i]) y = stencil_row_f(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, sh[i]);
-        t[i] = y;
-        const float2 si = s[i];
-        ts += (double)y.x * si.x + (double)y.y * si.y;
-        tt += (double)y.x * y.x + (double)y.y * y.y;
+    if (FORM == 0 && i < N) row();
+    while (i < N) {
+        if (sub == 0) {
+            t[i] = y;
+            ts += (double)y.x * si.x + (double)y.y * si.y;
+            tt += (double)y.x * y.x + (double)y.y * y.y;
+        }
+        i += row_step<FORM>();
+        if (i < N) row();
     }
     const double vals[2] = {ts, tt};
     const int slots2[2] = {5, 6};
     block_store<2>(vals, slots2, part, lblock());
 }
 
+template <int FORM>
 __global__ __launch_bounds__(BLOCK) void kf_iter_x(int N, int nb, KrylovCtl *ic, const float2 *__restrict__ ph,
                                                    const float2 *__restrict__ sh, const float2 *__restrict__ s,
                                                    const float2 *__restrict__ t, const float2 *__restrict__ rt,
                                                    float2 *__restrict__ x, float2 *__restrict__ r,
                                                    double *__restrict__ part)
 {
-    if (ic->done) return;
-    if (ic->stop) {  // stopped on ||s|| by the previous phase
-        if (blockIdx.x == 0 && threadIdx.x == 0) ic->done = 1;
-        return;
-    }
+    int i = vec_first<FORM>(blockIdx.x, N);
+    float2 xi, h, hs, si, ti, q;
+    auto load = [&]() {
+        xi = x[i];
+        h = ph[i];
+        hs = sh[i];
+        si = s[i];
+        ti = t[i];
+        q = rt[i];
+    };
+    if (i < N) load();
+    const KrylovCtl k = *ic;
     const int slots[2] = {5, 6};
     double red[2];
     block_load<2>(part, slots, nb, red);
+    if (k.done) return;
+    if (k.stop) {  // stopped on ||s|| by the previous phase
+        if (blockIdx.x == 0 && threadIdx.x == 0) ic->done = 1;
+        return;
+    }
     const double omega = red[0] / red[1];
-    const float al = (float)ic->alpha, om = (float)omega;
+    const float al = (float)k.alpha, om = (float)omega;
     double rr = 0, rtr = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        float2 xi = x[i];
-        const float2 h = ph[i], hs = sh[i], si = s[i], ti = t[i], q = rt[i];
+    while (i < N) {
         xi.x += al * h.x;
         xi.y += al * h.y;
         xi.x += om * hs.x;
@@ -1196,16 +1422,18 @@ __global__ __launch_bounds__(BLOCK) void kf_iter_x(int N, int nb, KrylovCtl *ic,
         r[i] = ri;
         rr += (double)ri.x * ri.x + (double)ri.y * ri.y;
         rtr += (double)q.x * ri.x + (double)q.y * ri.y;
+        i += row_step<FORM>();
+        if (i < N) load();
     }
     const double vals[2] = {rr, rtr};
     const int slots2[2] = {1, 2};
     block_store<2>(vals, slots2, part, blockIdx.x);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ic->omega = omega;
-        ic->rho2 = ic->rho1;
-        const int nit = ic->nit + 1;
+        ic->rho2 = k.rho1;
+        const int nit = k.nit + 1;
         ic->nit = nit;
-        if (nit >= ic->max_iter) ic->status = 1;
+        if (nit >= k.max_iter) ic->status = 1;
     }
 }
 
@@ -1232,7 +1460,7 @@ __global__ __launch_bounds__(BLOCK) void k_lift(int N, const double4 *__restrict
 }
 
 // ------------------------------------------------------------------ update
-// v = gamma0 (x_p ep + x_q eq); u_next = normalize(u + dt v); partial max |x_i|^2
+// v = gamma0 (x_p ep + x_q eq); u_next = normalize(u + dt v); max |x_i|^2 into ctl->vmax2
 // (src/solver.cpp:74-88, src/node.h:116-122)
 // The solve ended and is accepted: converged, no overflow or breakdown, final residual within tol
 // (the host's test of the same control block)
@@ -1245,9 +1473,9 @@ __global__ __launch_bounds__(BLOCK) void k_update(int N, double dt, const int32_
                                                   const double2 *__restrict__ x, const double4 *__restrict__ ep4,
                                                   const double4 *__restrict__ eq4,
                                                   const NodeRec *__restrict__ cur, NodeRec *__restrict__ next,
-                                                  double *__restrict__ part, const KrylovCtl *gate)
+                                                  KrylovCtl *ctl, bool gated)
 {
-    if (gate && !solved(gate)) return;
+    if (gated && !solved(ctl)) return;
     double m2 = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
         if (!mag[i]) continue;
@@ -1279,16 +1507,11 @@ __global__ __launch_bounds__(BLOCK) void k_update(int N, double dt, const int32_
     if (threadIdx.x == 0) {
         double s = sh[0];
         for (int q = 1; q < BLOCK / 64; q++) s = fmax(s, sh[q]);
-        part[7 * MAX_PART + blockIdx.x] = s;
-    }
-}
-
-__global__ void k_finish_update(int nb, KrylovCtl *ctl, const double *__restrict__ part, bool gated)
-{
-    if (gated && !solved(ctl)) return;
-    if (threadIdx.x < 64) {
-        const double m = wave_max(lane_fold(part + 7 * MAX_PART, nb, 0.0, MaxOp()));
-        if (threadIdx.x == 0) ctl->vmax2 = m;
+        // the order of nonnegative doubles is that of their bits, and a maximum does not depend on
+        // the order of the blocks
+        unsigned long long *m = reinterpret_cast<unsigned long long *>(&ctl->vmax2);
+        const unsigned long long b = (unsigned long long)__double_as_longlong(s);
+        if (b > __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(m, b);
     }
 }
 
@@ -1800,9 +2023,13 @@ void launch_node_assemble(Ctx &c, double r, double cst, double /*dt*/)
         Prof pr(c, "node_assemble");
         k_node_assemble<<<nb, BLOCK, 0, c.stream>>>(c.N, cos(r), sin(r), cst, c.rec[c.cur], vsrc, c.mag, c.inc_ptr,
                                                     c.elem_out, c.mass, c.sdiag, c.ep4, c.eq4, c.Dg,
-                                                    c.dprec, c.b, c.x, c.w, c.part);
+                                                    c.dprec, c.b, c.x, c.w, c.part, c.ctl);
     }
-    k_set_rhsn<<<1, 64, 0, c.stream>>>(nb, c.ctl, c.part);
+}
+
+// A batch's stopping scale in place of ||b|| of the union
+static void launch_batch_scale(Ctx &c)
+{
     const int K = (int)c.inst_node_off.size() - 1;
     if (K > 1) {
         k_inst_norm2<<<K, BLOCK, 0, c.stream>>>(c.d_inst_node_off, c.b, c.inst_bn2);
@@ -1815,37 +2042,61 @@ void launch_basis(Ctx &c, double r)
     k_basis<<<c.blocks_for(c.N), BLOCK, 0, c.stream>>>(c.N, cos(r), sin(r), c.rec[c.cur], c.ep4, c.eq4);
 }
 
+// Form of the solver's kernels and their blocks: four lanes per row while a row's lanes all have a
+// thread, a lane per row in one pass up to the grid's size, then passes over the rows.
+template <class F>
+static void krylov_shape(const Ctx &c, F &&go)
+{
+    if (c.N <= MAX_PART * BLOCK / 4)
+        go(std::integral_constant<int, 4>(), (c.N + BLOCK / 4 - 1) / (BLOCK / 4));
+    else if (c.N <= MAX_PART * BLOCK)
+        go(std::integral_constant<int, 1>(), c.blocks_for(c.N));
+    else
+        go(std::integral_constant<int, 0>(), c.blocks_for(c.N));
+}
+
 void launch_r0(Ctx &c, double cst)
 {
-    const int nb = c.blocks_for(c.N);
-    Prof pr(c, "spmv_r0");
-    k_r0<<<nb, BLOCK, 0, c.stream>>>(c.N, cst, STENCIL_PASS, c.w, c.x, c.b, c.r, c.rt, c.p, c.ctl, c.part);
+    {
+        Prof pr(c, "spmv_r0");
+        krylov_shape(c, [&](auto l, int nb) {
+            constexpr int L = decltype(l)::value;
+            k_r0<L><<<nb, BLOCK, 0, c.stream>>>(c.N, c.blocks_for(c.N), cst, STENCIL_PASS, c.w, c.x, c.b, c.r, c.rt, c.p,
+                                                c.ctl, c.part);
+        });
+    }
+    launch_batch_scale(c);
 }
 
 void launch_iteration(Ctx &c, double cst, int part)
 {
-    const int nb = c.blocks_for(c.N);
-    if (part != 2) {
-        Prof pr(c, "iter_p");
-        k_iter_p<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ctl, c.ep4, c.eq4, c.dprec, c.r, c.v, c.p, c.ph, c.w, c.part);
-    }
-    if (part == 1) return;
-    {
-        Prof pr(c, "spmv");
-        k_spmv_v<<<nb, BLOCK, 0, c.stream>>>(c.N, cst, STENCIL_PASS, c.ctl, c.w, c.ph, c.rt, c.v, c.part);
-    }
-    {
-        Prof pr(c, "iter_s");
-        k_iter_s<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ctl, c.ep4, c.eq4, c.dprec, c.r, c.v, c.s, c.sh, c.w, c.part);
-    }
-    {
-        Prof pr(c, "spmv");
-        k_spmv_t<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, cst, STENCIL_PASS, c.ctl, c.w, c.sh, c.s, c.ph, c.x, c.t, c.part);
-    }
-    {
-        Prof pr(c, "iter_x");
-        k_iter_x<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ctl, c.ph, c.sh, c.s, c.t, c.rt, c.x, c.r, c.part);
-    }
+    krylov_shape(c, [&](auto l, int nb) {
+        constexpr int L = decltype(l)::value;
+        if (part != 2) {
+            Prof pr(c, "iter_p");
+            k_iter_p<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ctl, c.ep4, c.eq4, c.dprec, c.r, c.v, c.p, c.ph, c.w,
+                                                    c.part);
+        }
+        if (part == 1) return;
+        {
+            Prof pr(c, "spmv");
+            k_spmv_v<L><<<nb, BLOCK, 0, c.stream>>>(c.N, cst, STENCIL_PASS, c.ctl, c.w, c.ph, c.rt, c.v, c.part);
+        }
+        {
+            Prof pr(c, "iter_s");
+            k_iter_s<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ctl, c.ep4, c.eq4, c.dprec, c.r, c.v, c.s, c.sh, c.w,
+                                                    c.part);
+        }
+        {
+            Prof pr(c, "spmv");
+            k_spmv_t<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, cst, STENCIL_PASS, c.ctl, c.w, c.sh, c.s, c.ph, c.x, c.t,
+                                                    c.part);
+        }
+        {
+            Prof pr(c, "iter_x");
+            k_iter_x<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ctl, c.ph, c.sh, c.s, c.t, c.rt, c.x, c.r, c.part);
+        }
+    });
 }
 
 void launch_mixed_start(Ctx &c)
@@ -1855,47 +2106,52 @@ void launch_mixed_start(Ctx &c)
         Prof pr(c, "to_f32");
         k_to_f32<<<nb, BLOCK, 0, c.stream>>>(c.N, c.ep4, c.eq4, c.Dg, c.dprec, c.ep4f, c.eq4f, c.Dgf, c.dprecf);
     }
-    k_mixed_init<<<1, 64, 0, c.stream>>>(c.ctl);
+    k_mixed_init<<<1, 64, 0, c.stream>>>(nb, c.ctl, c.part);
+    launch_batch_scale(c);
 }
 
 void launch_mixed_residual(Ctx &c, double cst, double tol_in, int max_inner)
 {
-    const int nb = c.blocks_for(c.N);
-    {
-        Prof pr(c, "spmv_r0");
-        k_resid<<<nb, BLOCK, 0, c.stream>>>(c.N, cst, STENCIL_PASS, c.ctl, c.w, c.x, c.b, c.rf, c.rtf, c.pf, c.df,
-                                            c.part);
-    }
-    k_outer<<<1, 64, 0, c.stream>>>(nb, c.ctl, c.ic, tol_in, max_inner, c.part);
+    krylov_shape(c, [&](auto l, int nb) {
+        constexpr int L = decltype(l)::value;
+        {
+            Prof pr(c, "spmv_r0");
+            k_resid<L><<<nb, BLOCK, 0, c.stream>>>(c.N, cst, STENCIL_PASS, c.ctl, c.w, c.x, c.b, c.rf, c.rtf, c.pf, c.df,
+                                                   c.part);
+        }
+        k_outer<<<1, 64, 0, c.stream>>>(nb, c.ctl, c.ic, tol_in, max_inner, c.part);
+    });
 }
 
 void launch_inner_iteration(Ctx &c, double cst)
 {
-    const int nb = c.blocks_for(c.N);
     const float cf = (float)cst;
-    {
-        Prof pr(c, "iter_p");
-        kf_iter_p<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ic, c.ep4f, c.eq4f, c.dprecf, c.rf, c.vf, c.pf, c.phf, c.wf,
-                                              c.part);
-    }
-    {
-        Prof pr(c, "spmv");
-        kf_spmv_v<<<nb, BLOCK, 0, c.stream>>>(c.N, cf, STENCIL_PASS_F, c.ic, c.wf, c.phf, c.rtf, c.vf, c.part);
-    }
-    {
-        Prof pr(c, "iter_s");
-        kf_iter_s<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ic, c.ep4f, c.eq4f, c.dprecf, c.rf, c.vf, c.sf, c.shf, c.wf,
-                                              c.part);
-    }
-    {
-        Prof pr(c, "spmv");
-        kf_spmv_t<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, cf, STENCIL_PASS_F, c.ic, c.wf, c.shf, c.sf, c.phf, c.df, c.tf,
-                                              c.part);
-    }
-    {
-        Prof pr(c, "iter_x");
-        kf_iter_x<<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ic, c.phf, c.shf, c.sf, c.tf, c.rtf, c.df, c.rf, c.part);
-    }
+    krylov_shape(c, [&](auto l, int nb) {
+        constexpr int L = decltype(l)::value;
+        {
+            Prof pr(c, "iter_p");
+            kf_iter_p<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ic, c.ep4f, c.eq4f, c.dprecf, c.rf, c.vf, c.pf, c.phf,
+                                                     c.wf, c.part);
+        }
+        {
+            Prof pr(c, "spmv");
+            kf_spmv_v<L><<<nb, BLOCK, 0, c.stream>>>(c.N, cf, STENCIL_PASS_F, c.ic, c.wf, c.phf, c.rtf, c.vf, c.part);
+        }
+        {
+            Prof pr(c, "iter_s");
+            kf_iter_s<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ic, c.ep4f, c.eq4f, c.dprecf, c.rf, c.vf, c.sf, c.shf,
+                                                     c.wf, c.part);
+        }
+        {
+            Prof pr(c, "spmv");
+            kf_spmv_t<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, cf, STENCIL_PASS_F, c.ic, c.wf, c.shf, c.sf, c.phf, c.df,
+                                                     c.tf, c.part);
+        }
+        {
+            Prof pr(c, "iter_x");
+            kf_iter_x<L><<<nb, BLOCK, 0, c.stream>>>(c.N, nb, c.ic, c.phf, c.shf, c.sf, c.tf, c.rtf, c.df, c.rf, c.part);
+        }
+    });
 }
 
 void launch_batch_solve(Ctx &c, double cst, int block)
@@ -1919,13 +2175,9 @@ void launch_refine(Ctx &c)
 
 void launch_update(Ctx &c, double dt, bool gated)
 {
-    const int nb = c.blocks_for(c.N);
-    {
-        Prof pr(c, "update");
-        k_update<<<nb, BLOCK, 0, c.stream>>>(c.N, dt, c.mag, c.x, c.ep4, c.eq4, c.rec[c.cur], c.rec[1 - c.cur], c.part,
-                                             gated ? c.ctl : nullptr);
-    }
-    k_finish_update<<<1, 64, 0, c.stream>>>(nb, c.ctl, c.part, gated);
+    Prof pr(c, "update");
+    k_update<<<std::min(c.blocks_for(c.N), 256), BLOCK, 0, c.stream>>>(c.N, dt, c.mag, c.x, c.ep4, c.eq4, c.rec[c.cur],
+                                                        c.rec[1 - c.cur], c.ctl, gated);
 }
 
 void launch_spmv_debug(Ctx &c, double cst, const double2 *xin, double2 *yout)

@@ -1,0 +1,40 @@
+"""The solver's kernels in each of their forms (four lanes per row, a lane per row in one pass of the
+grid, a lane per row in several passes) at the edges between them: 65,536 nodes and the next mesh,
+262,144 and the next, and meshes of less than a block. The accepted solution's residual is recomputed in
+numpy from the assembled system; BiCGSTAB tests its recursive residual, which drifts from the true
+one by rounding only, so it is held to twice the tolerance. In FP32 iterations the accepted residual is
+the true one."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from feellgood_amd import native as nv
+from feellgood_amd.engine import Engine
+from feellgood_amd.mesh import HostMesh
+
+TOL = 1e-9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("krylov", ["fp64", "mixed"])
+@pytest.mark.parametrize("cells", [(1, 1, 1), (2, 2, 6), (4, 4, 4), (31, 31, 63), (32, 31, 63), (63, 63, 63), (64, 63, 63)])
+def test_solution_at_form_edges(cells, krylov):
+    m = HostMesh.cuboid(tuple(3.0 * c for c in cells), cells, jitter=0.1, seed=5)
+    m.prepare({"volume": dict(Ms=8e5, Ae=1.3e-11, alpha=0.1)})
+    rng = np.random.default_rng(1)
+    u = np.array([1.0, 0.4, 0.0]) + rng.uniform(-0.2, 0.2, size=(m.n_nodes, 3))
+    u /= np.linalg.norm(u, axis=1, keepdims=True)
+    g = Engine(m.mesh, tol=TOL, max_iter=1000, krylov=krylov)
+    g.set_state(nv.FG_BOTH, u=u)
+    dt = 2e-14
+    g.base_projection(0.3)
+    g.prepare_elements(np.array([1e4, 2e4, -3e3]), dt, 1.05)
+    failed, info = g.solve(dt)
+    assert not failed and info.iterations > 0
+    rp, col, val, rhs = g.system()
+    A = sp.csr_matrix((val, col, rp), shape=(len(rhs), len(rhs)))
+    x = g.solution()
+    assert np.linalg.norm(rhs - A @ x) <= 2 * TOL * np.linalg.norm(rhs)
+    assert info.rhs_norm == pytest.approx(np.linalg.norm(rhs), rel=1e-12)
+    v = np.sqrt((x.reshape(-1, 2) ** 2).sum(1).max())
+    assert info.v_max == pytest.approx(1.76085962784e11 * nv.MU0 * v, rel=1e-12)
