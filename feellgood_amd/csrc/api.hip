@@ -1070,7 +1070,10 @@ int fg_solve(fg_ctx *x, double dt, fg_solve_info *info)
         if (c.opt.krylov == FG_KRYLOV_MIXED) return solve_mixed(x, dt, cst, info);
         if (c.opt.batch_solver == FG_BATCH_PERSISTENT && c.inst_node_off.size() > 2)
             return solve_batch(x, dt, cst, info);
-        launch_r0(c, cst);
+        // a small mesh: the whole loop in one launch
+        const bool one = c.inst_node_off.size() == 2 && block_solve_fits(c);
+        if (one) launch_block_solve(c, cst);
+        else launch_r0(c, cst);
         // BiCGSTAB: batches of iterations, the device control block says when to stop. Iteration
         // n's convergence is tested at the start of iteration n + 1, so the first batch is the
         // previous solve's count plus that test: a solve that converges like the last one needs a
@@ -1085,6 +1088,7 @@ int fg_solve(fg_ctx *x, double dt, fg_solve_info *info)
         bool open = false;  // the last batch ended with the first phase of iteration launched + 1
         int batch = std::max(2, std::min(x->last_nit + 1, c.opt.max_iter));
         while (true) {
+            if (one) launched = c.opt.max_iter + 1;
             if (open) {
                 launch_iteration(c, cst, 2);
                 launched++;

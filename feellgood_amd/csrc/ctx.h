@@ -189,6 +189,9 @@ void launch_inner_iteration(Ctx &c, double c_stencil);
 void launch_refine(Ctx &c);
 // FG_BATCH_PERSISTENT: every instance's bicg_dir in one launch (one block per instance)
 void launch_batch_solve(Ctx &c, double c_stencil, int block);
+// the same for a context of one small mesh: its whole bicg_dir in one block, the result in c.ctl
+bool block_solve_fits(const Ctx &c);
+void launch_block_solve(Ctx &c, double c_stencil);
 // gated: only if the control block says the solve was accepted (launched with the last
 // iterations, before the host has read it)
 void launch_update(Ctx &c, double dt, bool gated = false);

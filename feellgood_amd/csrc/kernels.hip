@@ -840,65 +840,153 @@ __global__ __launch_bounds__(BLOCK) void k_iter_x(int N, int nb, KrylovCtl *ctl,
     }
 }
 
-// ------------------------------------------------------------------ batched instances, one launch
-// FG_BATCH_PERSISTENT: one block per instance runs that instance's whole bicg_dir
-// (src/algebra/bicg.h:162-234) in a single launch for the batch, with block-level reductions (a
-// fixed tree), its own criterion ||r_k|| <= tol ||b_k|| and no host read or grid-wide step between
-// iterations: the stencil never crosses instances, so a block needs only its own rows and their
-// lifted vectors. The phases and scalars are those of the grid kernels above. Blocks take the
-// instances largest first (order[]), so the long solves start early.
+// ------------------------------------------------------------------ a solve in one launch
+// One block per instance runs that instance's whole bicg_dir (src/algebra/bicg.h:162-234) in a single
+// launch, with block-level reductions (a fixed tree), its own criterion ||r_k|| <= tol ||b_k|| and no
+// host read or grid-wide step between iterations: the stencil never crosses instances, so a block
+// needs only its own rows and their lifted vectors. The phases and scalars are those of the grid
+// kernels above. FG_BATCH_PERSISTENT runs every instance of a batch this way, largest first
+// (order[]), so the long solves start early; a context of one small mesh its only one (ctl set: the
+// control block of the grid kernels gets the result).
+// Bound by the latency of one CU's reads: the lifted vector is kept in LDS (LW) where the largest
+// instance's fits, and four entries of a row are in flight (64 dots of 1,160 nodes on average: 0.47 ms
+// a solve with the vector in memory and one entry at a time, 0.24 ms now). Four lanes per row were
+// slower at every size (five iterations on 189 nodes 71 against 59 us).
 
-// sums of NV values over the block (fixed tree), the same in every thread
+// sums of NV values over the block (fixed tree), the same in every thread; sh alternates between two
+// buffers from call to call, so that one barrier per sum is enough
 template <int NV, int BS>
-__device__ inline void bsum(double (&v)[NV], double (*sh)[BS / 64])
+__device__ inline void bsum(double (&v)[NV], double (*sh)[2][BS / 64], int &turn)
 {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double (*m)[BS / 64] = sh[turn];
+    turn ^= 1;
 #pragma unroll
     for (int k = 0; k < NV; k++) {
         const double r = wave_sum(v[k]);
-        if (lane == 0) sh[k][wid] = r;
+        if (lane == 0) m[k][wid] = r;
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        double s = sh[k][0];
-        for (int q = 1; q < BS / 64; q++) s += sh[k][q];
+        double s = m[k][0];
+#pragma unroll
+        for (int q = 1; q < BS / 64; q++) s += m[k][q];
         v[k] = s;
     }
-    __syncthreads();  // sh is free again
 }
 
-template <int BS>
-__global__ __launch_bounds__(BS) void k_bicg_batch(const int32_t *__restrict__ order,
-                                                   const int64_t *__restrict__ off, double cst, double tol,
+// the lifted vector of an instance's rows [n0, ..): in LDS, three doubles a row, or in memory
+template <bool LW>
+struct LiftVec {
+    double *l;
+    double4 *g;
+    int n0;
+    __device__ void put(int i, double2 h, const double4 &e, const double4 &q) const
+    {
+        const double x = h.x * e.x + h.y * q.x, y = h.x * e.y + h.y * q.y, z = h.x * e.z + h.y * q.z;
+        if constexpr (LW) {
+            double *d = l + 3 * (i - n0);
+            d[0] = x;
+            d[1] = y;
+            d[2] = z;
+        } else {
+            g[i] = make_double4(x, y, z, 0.0);
+        }
+    }
+    __device__ double4 operator[](int j) const
+    {
+        if constexpr (LW) {
+            const double *d = l + 3 * (j - n0);
+            return make_double4(d[0], d[1], d[2], 0.0);
+        } else {
+            return g[j];
+        }
+    }
+};
+
+// y = A x over the block's rows, one lane per row, four of its entries in flight: row(i, y)
+template <int BS, bool LW, class F>
+__device__ inline void block_spmv(int n0, int n1, double cst, STENCIL_ARGS, const LiftVec<LW> &w, const double2 *x,
+                                  F &&row)
+{
+    for (int i = n0 + (int)threadIdx.x; i < n1; i += BS) {
+        double2 y = make_double2(0, 0);
+        const double4 p = ep4[i], q = eq4[i], g = Dg[i];
+        const double2 xi = x[i];
+        if (mag[i]) {
+            const int sl = i >> 6, width = swid[sl];
+            const int64_t off = sptr[sl] + (i & 63);
+            constexpr int U = 4;
+            double zx = 0, zy = 0, zz = 0;
+            for (int k0 = 0; k0 < width; k0 += U) {
+                int j[U];
+                double v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int64_t e = off + (int64_t)min(k0 + u, width - 1) * SELL_C;
+                    j[u] = scol[e];
+                    v[u] = sval[e];
+                    if (k0 + u >= width) v[u] = 0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const double4 a = w[j[u]];
+                    zx += v[u] * a.x;
+                    zy += v[u] * a.y;
+                    zz += v[u] * a.z;
+                }
+            }
+            y.x = cst * (q.x * zx + q.y * zy + q.z * zz) + (g.x * xi.x + g.y * xi.y);
+            y.y = cst * (p.x * zx + p.y * zy + p.z * zz) + (g.z * xi.x + g.w * xi.y);
+        }
+        row(i, y);
+    }
+}
+
+template <int BS, bool LW>
+__global__ __launch_bounds__(BS) void k_bicg_block(const int32_t *__restrict__ order,
+                                                   const int64_t *__restrict__ off, int N, double cst, double tol,
                                                    int max_iter, STENCIL_ARGS, const double2 *__restrict__ dprec,
                                                    const double2 *__restrict__ b, double2 *__restrict__ x,
                                                    double2 *__restrict__ r, double2 *__restrict__ rt,
                                                    double2 *__restrict__ p, double2 *__restrict__ ph,
                                                    double2 *__restrict__ v, double2 *__restrict__ s,
                                                    double2 *__restrict__ sh, double2 *__restrict__ t,
-                                                   double4 *__restrict__ w, int2 *__restrict__ stat,
-                                                   double2 *__restrict__ resn)
+                                                   double4 *__restrict__ wg, int2 *__restrict__ stat,
+                                                   double2 *__restrict__ resn, KrylovCtl *ctl)
 {
-    __shared__ double red[2][BS / 64];
-    const int k = order[blockIdx.x];
-    const int n0 = (int)off[k], n1 = (int)off[k + 1];
-    // r = b - A x0 (w = lift(x0) from the assembly or the guess), rt = p = r
-    double a2[2] = {0, 0};
-    for (int i = n0 + threadIdx.x; i < n1; i += BS) {
-        double2 ri = make_double2(0, 0);
-        const double2 bi = b[i];
-        if (mag[i]) {
-            const double2 y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, x[i]);
-            ri = make_double2(bi.x - y.x, bi.y - y.y);
+    extern __shared__ double lds[];
+    __shared__ double red[2][2][BS / 64];
+    const int k = order ? order[blockIdx.x] : 0;
+    const int n0 = order ? (int)off[k] : 0, n1 = order ? (int)off[k + 1] : N;
+    const LiftVec<LW> w{lds, wg, n0};
+    int turn = 0;
+    auto spmv = [&](const double2 *xv, auto &&row) {
+        block_spmv<BS, LW>(n0, n1, cst, sptr, swid, scol, sval, ep4, eq4, Dg, mag, w, xv, row);
+    };
+    // r = b - A x0, rt = p = r (the lifted x0 is in wg: the assembly's or the guess's)
+    if constexpr (LW) {
+        for (int i = n0 + threadIdx.x; i < n1; i += BS) {
+            const double4 a = wg[i];
+            double *d = lds + 3 * (i - n0);
+            d[0] = a.x;
+            d[1] = a.y;
+            d[2] = a.z;
         }
+        __syncthreads();
+    }
+    double a2[2] = {0, 0};
+    spmv(x, [&](int i, double2 y) {
+        const double2 bi = b[i];
+        const double2 ri = mag[i] ? make_double2(bi.x - y.x, bi.y - y.y) : make_double2(0, 0);
         r[i] = ri;
         rt[i] = ri;
         p[i] = ri;
         a2[0] += ri.x * ri.x + ri.y * ri.y;
         a2[1] += bi.x * bi.x + bi.y * bi.y;
-    }
-    bsum<2, BS>(a2, red);
+    });
+    bsum<2, BS>(a2, red, turn);
     const double rhsn = sqrt(fabs(a2[1]));
     double res = sqrt(fabs(a2[0])), rho1 = a2[0], rho2 = 0, alpha = 0, omega = 0, beta = 0;
     int nit = 0, status = -1;
@@ -934,19 +1022,16 @@ __global__ __launch_bounds__(BS) void k_bicg_batch(const int32_t *__restrict__ o
             const double2 d = dprec[i];
             const double2 h = make_double2(d.x * pi.x, d.y * pi.y);
             ph[i] = h;
-            const double4 e = ep4[i], q = eq4[i];
-            w[i] = make_double4(h.x * e.x + h.y * q.x, h.x * e.y + h.y * q.y, h.x * e.z + h.y * q.z, 0.0);
+            w.put(i, h, ep4[i], eq4[i]);
         }
         __syncthreads();  // the instance's w
         double a1[1] = {0};
-        for (int i = n0 + threadIdx.x; i < n1; i += BS) {
-            double2 y = make_double2(0, 0);
-            if (mag[i]) y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i]);
+        spmv(ph, [&](int i, double2 y) {
             v[i] = y;
             const double2 q = rt[i];
             a1[0] += y.x * q.x + y.y * q.y;
-        }
-        bsum<1, BS>(a1, red);  // every thread has read w before it is rewritten below
+        });
+        bsum<1, BS>(a1, red, turn);  // every thread has read w before it is rewritten below
         alpha = rho1 / a1[0];
         double a3[1] = {0};
         for (int i = n0 + threadIdx.x; i < n1; i += BS) {
@@ -957,10 +1042,9 @@ __global__ __launch_bounds__(BS) void k_bicg_batch(const int32_t *__restrict__ o
             const double2 d = dprec[i];
             const double2 h = make_double2(d.x * si.x, d.y * si.y);
             sh[i] = h;
-            const double4 e = ep4[i], q = eq4[i];
-            w[i] = make_double4(h.x * e.x + h.y * q.x, h.x * e.y + h.y * q.y, h.x * e.z + h.y * q.z, 0.0);
+            w.put(i, h, ep4[i], eq4[i]);
         }
-        bsum<1, BS>(a3, red);  // also publishes the instance's w
+        bsum<1, BS>(a3, red, turn);  // also publishes the instance's w
         // the test on ||s|| (src/algebra/bicg.h:206-212)
         const double rs = sqrt(fabs(a3[0]));
         if (isnan(rs)) {
@@ -985,15 +1069,13 @@ __global__ __launch_bounds__(BS) void k_bicg_batch(const int32_t *__restrict__ o
             break;
         }
         double a4[2] = {0, 0};
-        for (int i = n0 + threadIdx.x; i < n1; i += BS) {
-            double2 y = make_double2(0, 0);
-            if (mag[i]) y = stencil_row(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, sh[i]);
+        spmv(sh, [&](int i, double2 y) {
             t[i] = y;
             const double2 si = s[i];
             a4[0] += y.x * si.x + y.y * si.y;
             a4[1] += y.x * y.x + y.y * y.y;
-        }
-        bsum<2, BS>(a4, red);
+        });
+        bsum<2, BS>(a4, red, turn);
         omega = a4[0] / a4[1];
         double a5[2] = {0, 0};
         for (int i = n0 + threadIdx.x; i < n1; i += BS) {
@@ -1009,15 +1091,25 @@ __global__ __launch_bounds__(BS) void k_bicg_batch(const int32_t *__restrict__ o
             a5[0] += ri.x * ri.x + ri.y * ri.y;
             a5[1] += q.x * ri.x + q.y * ri.y;
         }
-        bsum<2, BS>(a5, red);
+        bsum<2, BS>(a5, red, turn);
         res = sqrt(fabs(a5[0]));
         rho2 = rho1;
         rho1 = a5[1];
         if (++nit >= max_iter) status = FG_ITER_OVERFLOW;
     }
     if (threadIdx.x == 0) {
-        stat[k] = make_int2(status, nit);
-        resn[k] = make_double2(res, rhsn);
+        if (stat) {
+            stat[k] = make_int2(status, nit);
+            resn[k] = make_double2(res, rhsn);
+        }
+        if (ctl) {
+            ctl->rhsn = rhsn;
+            ctl->res = res;
+            ctl->nit = nit;
+            ctl->status = status;
+            ctl->stop = 0;
+            ctl->done = 1;
+        }
     }
 }
 
@@ -2154,17 +2246,51 @@ void launch_inner_iteration(Ctx &c, double cst)
     });
 }
 
+// Nodes up to which one block's solve is faster than the grid kernels' five launches an iteration:
+// five iterations take 59, 100 and 128 us in one block on 189, 935 and 1,365 nodes, 120 in the grid
+// kernels whatever the size.
+constexpr int BLOCK_SOLVE_MAX = 1024;
+// Rows whose lifted vector the LDS of one block holds (24 bytes each of 152 KiB)
+constexpr int BLOCK_LDS_ROWS = 6400;
+template <int BS>
+static void launch_bicg_block(Ctx &c, double cst, int nblocks, int nmax, bool batch)
+{
+    const bool lw = nmax <= BLOCK_LDS_ROWS;
+    const size_t bytes = lw ? (size_t)24 * nmax : 0;
+#define FG_BLOCK_ARGS                                                                                              \
+    batch ? c.d_inst_order : nullptr, c.d_inst_node_off, c.N, cst, c.opt.tol, c.opt.max_iter, STENCIL_PASS, c.dprec, \
+        c.b, c.x, c.r, c.rt, c.p, c.ph, c.v, c.s, c.sh, c.t, c.w, batch ? c.d_inst_stat : nullptr, c.d_inst_resn,    \
+        batch ? nullptr : c.ctl
+    if (lw) {
+        if (bytes > 48 * 1024 &&
+            hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bicg_block<BS, true>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 24 * BLOCK_LDS_ROWS) != hipSuccess)
+            throw std::string("hipFuncSetAttribute (one-launch solve)");
+        k_bicg_block<BS, true><<<nblocks, BS, bytes, c.stream>>>(FG_BLOCK_ARGS);
+    } else {
+        k_bicg_block<BS, false><<<nblocks, BS, 0, c.stream>>>(FG_BLOCK_ARGS);
+    }
+#undef FG_BLOCK_ARGS
+}
+
 void launch_batch_solve(Ctx &c, double cst, int block)
 {
     const int K = (int)c.inst_node_off.size() - 1;
+    int nmax = 0;
+    for (int k = 0; k < K; k++) nmax = std::max(nmax, (int)(c.inst_node_off[k + 1] - c.inst_node_off[k]));
     Prof pr(c, "bicg_batch");
-#define FG_BATCH_ARGS                                                                                         \
-    c.d_inst_order, c.d_inst_node_off, cst, c.opt.tol, c.opt.max_iter, STENCIL_PASS, c.dprec, c.b, c.x, c.r, c.rt, \
-        c.p, c.ph, c.v, c.s, c.sh, c.t, c.w, c.d_inst_stat, c.d_inst_resn
-    if (block == 1024) k_bicg_batch<1024><<<K, 1024, 0, c.stream>>>(FG_BATCH_ARGS);
-    else if (block == 512) k_bicg_batch<512><<<K, 512, 0, c.stream>>>(FG_BATCH_ARGS);
-    else k_bicg_batch<256><<<K, 256, 0, c.stream>>>(FG_BATCH_ARGS);
-#undef FG_BATCH_ARGS
+    if (block == 1024) launch_bicg_block<1024>(c, cst, K, nmax, true);
+    else if (block == 512) launch_bicg_block<512>(c, cst, K, nmax, true);
+    else launch_bicg_block<256>(c, cst, K, nmax, true);
+}
+
+bool block_solve_fits(const Ctx &c) { return c.N <= BLOCK_SOLVE_MAX; }
+void launch_block_solve(Ctx &c, double cst)
+{
+    Prof pr(c, "bicg_block");
+    if (c.N <= 256) launch_bicg_block<256>(c, cst, 1, c.N, false);
+    else if (c.N <= 512) launch_bicg_block<512>(c, cst, 1, c.N, false);
+    else launch_bicg_block<1024>(c, cst, 1, c.N, false);
 }
 
 void launch_refine(Ctx &c)
