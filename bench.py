@@ -205,12 +205,9 @@ def kernel_model(name, n):
         "node_assemble": ("hbm", 332 * N + 144 * T),
         "element": ("hbm", 284 * T + 64 * N),
         "update": ("hbm", 164 * N),
-        "evolution": ("hbm", 128 * N),
-        "charges_tet": ("hbm", 16 * T + 96 * T + 4 * T + 80 * T + 64 * N),
-        "charges_tri": ("hbm", 16 * F + 128 * F + 64 * F + 48 * F + 96 * N),
-        "corr_gather": ("hbm", 8 * N + 4 * 3 * F + 16 * 3 * F + 16 * N),
-        "energy": ("hbm", 16 * T + 136 * T + 4 * T + 64 * N),
-        "max_angle": ("hbm", 4 * nnz + 64 * N),
+        "charges": ("hbm", 16 * T + 96 * T + 4 * T + 80 * T + 64 * N + 16 * F + 128 * F + 64 * F + 48 * F + 96 * N),
+        # the tetrahedra's energies, the triangles', and the nodes' largest angle with the evolution
+        "energy_angle_evolution": ("hbm", 16 * T + 136 * T + 4 * T + 64 * N + 136 * F + 4 * nnz + 128 * N),
         "p2p_direct": ("valu64", 2 * 10.0 * N * S),
     }
     f = n.get("fmm")

@@ -473,7 +473,6 @@ void build_plan(Ctx &c, const fg_mesh *m)
     upload(c.cinc_ptr, cincp, st);
     c.cinc_idx = dalloc<int32_t>(cinci.size());
     upload(c.cinc_idx, cinci, st);
-    c.corr = dalloc<double2>(N);
     c.src_pos = dalloc<double4>(c.S);
     upload(c.src_pos, spos, st);
     // the direct sum's partial potentials follow the charges in one allocation
@@ -522,7 +521,7 @@ void free_all(Ctx &c)
     void *ptrs[] = {c.rec[0], c.rec[1], c.pos4, c.ep4, c.eq4, c.mag, c.mass, c.sdiag, c.Dg, c.dprec, c.b, c.x, c.r,
                     c.rt, c.p, c.ph, c.v, c.s, c.sh, c.t, c.w, c.ctl, c.part, c.epart, c.res, c.slice_ptr, c.slice_w,
                     c.scol, c.sval, c.tet_nodes, c.geo, c.tet_reg, c.regions, c.elem_out, c.inc_ptr, c.epos,
-                    c.trik_nodes, c.trik_geo, c.tri_nodes, c.tri_geo, c.tri_corr, c.cinc_ptr, c.cinc_idx, c.corr,
+                    c.trik_nodes, c.trik_geo, c.tri_nodes, c.tri_geo, c.tri_corr, c.cinc_ptr, c.cinc_idx,
                     c.src_pos, c.src_q, c.src_pos_f, c.src_rank, c.d_inst_node_off, c.inst_bn2, c.d_node_inst, c.d_inst_src,
                     c.hsp, c.hst, c.spin_s, c.spin_pref, c.svalf, c.ep4f, c.eq4f, c.Dgf, c.wf, c.dprecf, c.rf,
                     c.rtf, c.pf, c.phf, c.vf, c.sf, c.shf, c.tf, c.df, c.ic, c.d_inst_order, c.d_inst_stat,
@@ -1215,10 +1214,8 @@ int fg_step(fg_ctx *x, const double Hext[3], double dt, double prefactor, double
         launch_charges(c);
         if (c.opt.demag_method == FG_DEMAG_FMM) launch_fmm(c);
         else launch_direct_p2p(c);
-        launch_energy(c, Hext);
-        launch_evolution(c);
+        launch_after(c, Hext);
         x->basis_valid = false;
-        launch_max_angle(c);
         HIPCHK(hipMemcpyAsync(c.h_part, c.res, 9 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
         HIPCHK(hipStreamSynchronize(c.stream));
         E[FG_E_EXCHANGE] = c.h_part[0];

@@ -80,6 +80,19 @@ struct KrylovCtl {
     int stop;
 };
 
+// Sum of a node's triangle-vertex corrections (u, v): entries cptr[i] .. cptr[i + 1] of cidx
+__device__ inline double2 vertex_corr(int i, const int32_t *__restrict__ cptr, const int32_t *__restrict__ cidx,
+                                      const double2 *__restrict__ corr3)
+{
+    double2 c = make_double2(0, 0);
+    for (int k = cptr[i]; k < cptr[i + 1]; k++) {
+        const double2 e = corr3[cidx[k]];
+        c.x += e.x;
+        c.y += e.y;
+    }
+    return c;
+}
+
 // small vector helpers
 struct d3 {
     double x, y, z;

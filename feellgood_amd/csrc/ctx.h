@@ -119,7 +119,6 @@ struct Ctx {
     double *tri_geo = nullptr;   // SoA [16][Fm]: n xyz, w0..3, dMs, surf, pad x3, Ks, uk xyz
     double2 *tri_corr = nullptr; // [3][Fm] vertex corrections (u, v)
     int32_t *cinc_ptr = nullptr, *cinc_idx = nullptr;  // node -> tri_corr entries
-    double2 *corr = nullptr;     // [N]
 
     // demag sources
     double4 *src_pos = nullptr;  // [S] in tree order when the FMM is used
@@ -203,6 +202,8 @@ void launch_energy(Ctx &c, const double Hext[3], const double *hsp = nullptr, do
 // c.hst from the node spin accumulation c.spin_s and the per-region prefactors c.spin_pref
 void launch_spin_field(Ctx &c);
 void launch_max_angle(Ctx &c);
+// energies, max_angle and evolution of a step in one launch
+void launch_after(Ctx &c, const double Hext[3]);
 void launch_average(Ctx &c, int which);
 void launch_evolution(Ctx &c);
 

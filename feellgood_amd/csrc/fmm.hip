@@ -89,7 +89,7 @@ struct FmmPlan {
     int32_t *d_tl_tb = nullptr, *d_tl_te = nullptr;  // their target ranges
     int64_t *d_lc_ptr = nullptr;  // [ntl+1] shared column list of each such leaf
     int32_t *d_lc_col = nullptr;
-    double2 *d_pot = nullptr;  // [T] near-field + correction potential
+    double2 *d_pot = nullptr;  // [T] near-field potential
     double2 *d_far = nullptr;  // M2P's partial sums of the multipole (far) part of the potentials
     int32_t *d_tgt_lc = nullptr;  // [T] local-expansion cell of each target's group (-1: none)
     float *d_nf_valf = nullptr;  // FP32 coefficients (mixed precision; d_nf_val is then released)
@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(256) void k_nf_build(int T, const int32_t *__restri
     }
 }
 
-// Near field + vertex corrections: one wavefront per leaf with targets. The leaf's targets share
+// Near field: one wavefront per leaf with targets. The leaf's targets share
 // one column list (the runs of the adjacent leaves); each element value is gathered once and
 // applied to up to four targets' coefficient rows at a time. Coefficients are FP64, or FP32 in the
 // mixed-precision mode (products and sums stay FP64).
@@ -1318,7 +1318,6 @@ __global__ __launch_bounds__(256) void k_nf_apply(int ntl, const int32_t *__rest
                                                   const int32_t *__restrict__ tl_te, const int64_t *__restrict__ lc_ptr,
                                                   const int32_t *__restrict__ lc_col, const int64_t *__restrict__ nf_ptr,
                                                   const TC *__restrict__ nf_val, const double2 *__restrict__ qe,
-                                                  const int32_t *__restrict__ tgt_node, const double2 *__restrict__ corr,
                                                   double2 *__restrict__ pot)
 {
     const int w = ((int)xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + (int)threadIdx.x) >> 6;
@@ -1364,10 +1363,7 @@ __global__ __launch_bounds__(256) void k_nf_apply(int ntl, const int32_t *__rest
         for (int i = 0; i < 4; i++) {
             if (i >= nt) break;
             const double su = wsum64(au[i]), sv = wsum64(av[i]);
-            if (lane == 0) {
-                const double2 c = corr[tgt_node[t0 + i]];
-                pot[t0 + i] = make_double2(su + c.x, sv + c.y);
-            }
+            if (lane == 0) pot[t0 + i] = make_double2(su, sv);
         }
     }
 }
@@ -1708,7 +1704,9 @@ __global__ __launch_bounds__(256) void k_fmm_finish(int T, const int32_t *__rest
                                                     const R *__restrict__ Lx, const int4 *__restrict__ tgt_far,
                                                     const double2 *__restrict__ far,
                                                     const double2 *__restrict__ pot, const int32_t *__restrict__ tgt_node,
-                                                    NodeRec *__restrict__ nxt, double mscale)
+                                                    const int32_t *__restrict__ cptr, const int32_t *__restrict__ cidx,
+                                                    const double2 *__restrict__ corr3, NodeRec *__restrict__ nxt,
+                                                    double mscale)
 {
     constexpr int NCo = fcount(P), CW = 2 * NCo;
     const int t = blockIdx.x * 256 + threadIdx.x;
@@ -1732,9 +1730,11 @@ __global__ __launch_bounds__(256) void k_fmm_finish(int T, const int32_t *__rest
     su /= mscale;
     sv /= mscale;
     const double2 pn = pot[t];
-    NodeRec *r = nxt + tgt_node[t];
-    r->phi = (pn.x + su) / (4 * M_PI);
-    r->phiv = (pn.y + sv) / (4 * M_PI);
+    const int i = tgt_node[t];
+    const double2 vc = vertex_corr(i, cptr, cidx, corr3);
+    NodeRec *r = nxt + i;
+    r->phi = ((pn.x + vc.x) + su) / (4 * M_PI);
+    r->phiv = ((pn.y + vc.y) + sv) / (4 * M_PI);
 }
 
 void fmm_build_near(Ctx &c, FmmPlan &P);
@@ -2309,10 +2309,10 @@ static void run_fmm(Ctx &c)
         const unsigned nb = (unsigned)(((int64_t)P.ntl * 64 + 255) / 256);
         if (P.ntl > 0 && P.d_nf_valf)
             k_nf_apply<float><<<nb, 256, 0, c.stream>>>(P.ntl, P.d_tl_tb, P.d_tl_te, P.d_lc_ptr, P.d_lc_col, P.d_nf_ptr,
-                                                  P.d_nf_valf, c.qe, P.d_tgt_node, c.corr, P.d_pot);
+                                                  P.d_nf_valf, c.qe, P.d_pot);
         else if (P.ntl > 0)
             k_nf_apply<double><<<nb, 256, 0, c.stream>>>(P.ntl, P.d_tl_tb, P.d_tl_te, P.d_lc_ptr, P.d_lc_col, P.d_nf_ptr,
-                                                   P.d_nf_val, c.qe, P.d_tgt_node, c.corr, P.d_pot);
+                                                   P.d_nf_val, c.qe, P.d_pot);
     }
 
     {
@@ -2362,8 +2362,8 @@ static void run_fmm(Ctx &c)
         const int T = (int)P.tgt_node.size();
         if (T > 0)
             k_fmm_finish<PP, F><<<(T + 255) / 256, 256, 0, c.stream>>>(T, P.d_tgt_lc, P.d_tgt_pos, P.d_cen, Lx, P.d_tgt_far, P.d_far,
-                                                                        P.d_pot, P.d_tgt_node, c.rec[1 - c.cur],
-                                                                        P.mscale);
+                                                                        P.d_pot, P.d_tgt_node, c.cinc_ptr, c.cinc_idx,
+                                                                        c.tri_corr, c.rec[1 - c.cur], P.mscale);
     }
 }
 

@@ -1609,15 +1609,11 @@ __global__ __launch_bounds__(BLOCK) void k_update(int N, double dt, const int32_
 
 // ------------------------------------------------------------------ demag sources
 // Tet::charges (src/tetra.cpp:347-359): q_g = -Ms w_g div(u), for u and v NEXT at once.
-__global__ __launch_bounds__(BLOCK) void k_charges_tet(int Tm, const int4 *__restrict__ tn,
-                                                       const double *__restrict__ geo,
-                                                       const int32_t *__restrict__ treg,
-                                                       const DevRegion *__restrict__ regs,
-                                                       const NodeRec *__restrict__ nxt,
-                                                       const int64_t *__restrict__ rank,
-                                                       double2 *__restrict__ q, double2 *__restrict__ qe)
+__device__ inline void charges_tet(int t, int Tm, const int4 *__restrict__ tn, const double *__restrict__ geo,
+                                   const int32_t *__restrict__ treg, const DevRegion *__restrict__ regs,
+                                   const NodeRec *__restrict__ nxt, const int64_t *__restrict__ rank,
+                                   double2 *__restrict__ q, double2 *__restrict__ qe)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= Tm) return;
     const int4 qn = tn[t];
     const int nd[4] = {qn.x, qn.y, qn.z, qn.w};
@@ -1667,15 +1663,11 @@ __device__ inline double tri_potential(const d3 P[3], const double s[3], double 
 }
 
 // Tri::charges + Tri::correctionCharges (src/triangle.cpp:45-78) for u and v NEXT at once.
-__global__ __launch_bounds__(BLOCK) void k_charges_tri(int Fm, int64_t src_off, const int4 *__restrict__ tn,
-                                                       const double *__restrict__ tg,
-                                                       const double4 *__restrict__ pos4,
-                                                       const NodeRec *__restrict__ nxt,
-                                                       const int64_t *__restrict__ rank,
-                                                       double2 *__restrict__ q, double2 *__restrict__ corr3,
-                                                       double2 *__restrict__ qe, int Tm)
+__device__ inline void charges_tri(int f, int Fm, int64_t src_off, const int4 *__restrict__ tn,
+                                   const double *__restrict__ tg, const double4 *__restrict__ pos4,
+                                   const NodeRec *__restrict__ nxt, const int64_t *__restrict__ rank,
+                                   double2 *__restrict__ q, double2 *__restrict__ corr3, double2 *__restrict__ qe, int Tm)
 {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= Fm) return;
     const int4 qn = tn[f];
     const int nd[3] = {qn.x, qn.y, qn.z};
@@ -1718,19 +1710,21 @@ __global__ __launch_bounds__(BLOCK) void k_charges_tri(int Fm, int64_t src_off, 
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_corr_gather(int N, const int32_t *__restrict__ cptr,
-                                                       const int32_t *__restrict__ cidx,
-                                                       const double2 *__restrict__ corr3, double2 *__restrict__ corr)
+// Both kinds of charges in one launch: blocks below nbf take triangles (few, and the longer work per
+// thread), the others tetrahedra.
+__global__ __launch_bounds__(BLOCK) void k_charges(int nbf, int Tm, const int4 *__restrict__ tn,
+                                                   const double *__restrict__ geo, const int32_t *__restrict__ treg,
+                                                   const DevRegion *__restrict__ regs, int Fm,
+                                                   const int4 *__restrict__ fn, const double *__restrict__ tg,
+                                                   const double4 *__restrict__ pos4, const NodeRec *__restrict__ nxt,
+                                                   const int64_t *__restrict__ rank, double2 *__restrict__ q,
+                                                   double2 *__restrict__ corr3, double2 *__restrict__ qe)
 {
-    for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-        double cu = 0, cv = 0;
-        for (int k = cptr[i]; k < cptr[i + 1]; k++) {
-            const double2 e = corr3[cidx[k]];
-            cu += e.x;
-            cv += e.y;
-        }
-        corr[i] = make_double2(cu, cv);
-    }
+    const int b = blockIdx.x;
+    if (b < nbf)
+        charges_tri(b * BLOCK + threadIdx.x, Fm, (int64_t)5 * Tm, fn, tg, pos4, nxt, rank, q, corr3, qe, Tm);
+    else
+        charges_tet((b - nbf) * BLOCK + threadIdx.x, Tm, tn, geo, treg, regs, nxt, rank, q, qe);
 }
 
 // 1/sqrt(x) in FP64: the hardware approximation (about 24 correct bits) and one third-order step
@@ -1846,7 +1840,9 @@ __global__ __launch_bounds__(BLOCK) void k_p2p_direct(int N, int64_t S, int nspl
 constexpr int P2P_FIN = 32;
 __global__ __launch_bounds__(BLOCK) void k_p2p_finish(int N, int nsplit, const int32_t *__restrict__ mag,
                                                       const double2 *__restrict__ part,
-                                                      const double2 *__restrict__ corr, NodeRec *__restrict__ nxt)
+                                                      const int32_t *__restrict__ cptr,
+                                                      const int32_t *__restrict__ cidx,
+                                                      const double2 *__restrict__ corr3, NodeRec *__restrict__ nxt)
 {
     __shared__ double2 sh[BLOCK / P2P_FIN][P2P_FIN];
     const int l = threadIdx.x % P2P_FIN, g = threadIdx.x / P2P_FIN;
@@ -1866,7 +1862,7 @@ __global__ __launch_bounds__(BLOCK) void k_p2p_finish(int N, int nsplit, const i
             pu += sh[k][l].x;
             pv += sh[k][l].y;
         }
-        const double2 c = corr[i];
+        const double2 c = vertex_corr(i, cptr, cidx, corr3);
         nxt[i].phi = (pu + c.x) / (4 * M_PI);
         nxt[i].phiv = (pv + c.y) / (4 * M_PI);
     }
@@ -1875,16 +1871,14 @@ __global__ __launch_bounds__(BLOCK) void k_p2p_finish(int N, int nsplit, const i
 // ------------------------------------------------------------------ energies
 // Fem::energy (src/energy.cpp:5-68), element energies src/tetra.cpp:309-391 and
 // src/triangle.cpp:38-43,80-85, on the NEXT state; partials per block, slots 0..3 = E[4].
-__global__ __launch_bounds__(BLOCK) void k_energy_tet(int Tm, const int4 *__restrict__ tn,
-                                                      const double *__restrict__ geo,
-                                                      const int32_t *__restrict__ treg,
-                                                      const DevRegion *__restrict__ regs,
-                                                      const NodeRec *__restrict__ nxt, double Hx, double Hy,
-                                                      double Hz, const double *__restrict__ hsp, double amp,
-                                                      double *__restrict__ part)
+__device__ inline void energy_tet(int blk, int nb, int Tm, const int4 *__restrict__ tn,
+                                  const double *__restrict__ geo, const int32_t *__restrict__ treg,
+                                  const DevRegion *__restrict__ regs, const NodeRec *__restrict__ nxt, double Hx,
+                                  double Hy, double Hz, const double *__restrict__ hsp, double amp,
+                                  double *__restrict__ part)
 {
     double e[4] = {0, 0, 0, 0};
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < Tm; t += gridDim.x * blockDim.x) {
+    for (int t = blk * BLOCK + threadIdx.x; t < Tm; t += nb * BLOCK) {
         const int4 q = tn[t];
         const int nd[4] = {q.x, q.y, q.z, q.w};
         const DevRegion R = regs[treg[t]];
@@ -1933,16 +1927,15 @@ __global__ __launch_bounds__(BLOCK) void k_energy_tet(int Tm, const int4 *__rest
         e[3] += -MU0 * R.Ms * ze;
     }
     const int slots[4] = {0, 1, 2, 3};
-    block_store<4>(e, slots, part, blockIdx.x);
+    block_store<4>(e, slots, part, blk);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_energy_tri(int Fm, const int4 *__restrict__ tn,
-                                                      const double *__restrict__ tg,
-                                                      const double *__restrict__ tks, // Ks, uk per tri (4 SoA)
-                                                      const NodeRec *__restrict__ nxt, double *__restrict__ part)
+__device__ inline void energy_tri(int blk, int nb, int Fm, const int4 *__restrict__ tn, const double *__restrict__ tg,
+                                  const double *__restrict__ tks, // Ks, uk per tri (4 SoA)
+                                  const NodeRec *__restrict__ nxt, double *__restrict__ part)
 {
     double e[2] = {0, 0};
-    for (int f = lblock() * blockDim.x + threadIdx.x; f < Fm; f += gridDim.x * blockDim.x) {
+    for (int f = blk * BLOCK + threadIdx.x; f < Fm; f += nb * BLOCK) {
         const int4 q = tn[f];
         const int nd[3] = {q.x, q.y, q.z};
         const d3 n = mk(tg[f], tg[(size_t)Fm + f], tg[(size_t)2 * Fm + f]);
@@ -1971,7 +1964,7 @@ __global__ __launch_bounds__(BLOCK) void k_energy_tri(int Fm, const int4 *__rest
         e[1] += 0.5 * MU0 * dMs * d;
     }
     const int slots[2] = {4, 5};
-    block_store<2>(e, slots, part, lblock());
+    block_store<2>(e, slots, part, blk);
 }
 
 // final sums of the partials: out[k] = sum of slot k, k < nslots; slots >= nfirst use nb_b blocks
@@ -1987,22 +1980,33 @@ __global__ void k_sum_finish(int nslots, int nfirst, int nb_a, int nb_b, const d
     }
 }
 
-// mesh::max_angle (src/mesh.h:295-306) over the magnetic edges of the stencil pattern
-__global__ __launch_bounds__(BLOCK) void k_max_angle(int N, const int64_t *__restrict__ sptr,
-                                                     const int32_t *__restrict__ swid,
-                                                     const int32_t *__restrict__ scol,
-                                                     const NodeRec *__restrict__ nxt, double *__restrict__ part)
+// mesh::max_angle (src/mesh.h:295-306) over the magnetic edges of the stencil pattern, block blk of
+// nb; and, when cur is given, Node::evolution (src/node.h:107): CURRENT = NEXT
+__device__ inline void node_angle(int blk, int nb, int N, const int64_t *__restrict__ sptr,
+                                  const int32_t *__restrict__ swid, const int32_t *__restrict__ scol,
+                                  const NodeRec *__restrict__ nxt, NodeRec *__restrict__ cur, double *__restrict__ part)
 {
     double mn = 1.0;
-    for (int i = lblock() * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+    for (int i = blk * BLOCK + threadIdx.x; i < N; i += nb * BLOCK) {
         const int sl = i >> 6, lane = i & 63;
         const int64_t off = sptr[sl];
+        const int width = swid[sl];
         const NodeRec a = nxt[i];
-        for (int k = 0; k < swid[sl]; k++) {
-            const int j = scol[off + (int64_t)k * SELL_C + lane];
-            if (j <= i) continue;
-            const NodeRec bq = nxt[j];
-            mn = fmin(mn, a.ux * bq.ux + a.uy * bq.uy + a.uz * bq.uz);
+        if (cur) cur[i] = a;
+        constexpr int U = 4;  // neighbours in flight
+        for (int k0 = 0; k0 < width; k0 += U) {
+            int j[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) j[u] = scol[off + (int64_t)min(k0 + u, width - 1) * SELL_C + lane];
+            double d[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const NodeRec *q = nxt + (j[u] > i ? j[u] : i);
+                d[u] = a.ux * q->ux + a.uy * q->uy + a.uz * q->uz;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (j[u] > i) mn = fmin(mn, d[u]);
         }
     }
     __shared__ double sh[BLOCK / 64];
@@ -2012,15 +2016,47 @@ __global__ __launch_bounds__(BLOCK) void k_max_angle(int N, const int64_t *__res
     if (threadIdx.x == 0) {
         double s = sh[0];
         for (int q = 1; q < BLOCK / 64; q++) s = fmin(s, sh[q]);
-        part[lblock()] = s;
+        part[6 * MAX_PART + blk] = s;
     }
 }
 
-__global__ void k_min_finish(int nb, const double *__restrict__ part, double *__restrict__ out)
+// What follows the potentials of a step, in one launch: the energies of the tetrahedra (the first nbt
+// blocks) and of the triangles (the next nbf), and over the nodes (nbn) the largest angle and the
+// evolution; any of the three may be left out. All read the NEXT state only, so they share the chip
+// instead of following one another.
+__global__ __launch_bounds__(BLOCK) void k_after(int nbt, int nbf, int nbn, int Tm, const int4 *__restrict__ tn,
+                                                 const double *__restrict__ geo, const int32_t *__restrict__ treg,
+                                                 const DevRegion *__restrict__ regs, double Hx, double Hy, double Hz,
+                                                 const double *__restrict__ hsp, double amp, int Fm,
+                                                 const int4 *__restrict__ fn, const double *__restrict__ tg, int N,
+                                                 const int64_t *__restrict__ sptr, const int32_t *__restrict__ swid,
+                                                 const int32_t *__restrict__ scol, const NodeRec *__restrict__ nxt,
+                                                 NodeRec *__restrict__ cur, double *__restrict__ part)
 {
-    if (threadIdx.x < 64) {
-        const double m = wave_min(lane_fold(part, nb, 1.0, MinOp()));
-        if (threadIdx.x == 0) out[0] = m;
+    const int b = blockIdx.x;
+    if (b < nbt)
+        energy_tet(b, nbt, Tm, tn, geo, treg, regs, nxt, Hx, Hy, Hz, hsp, amp, part);
+    else if (b < nbt + nbf)
+        energy_tri(xcd_block(b - nbt, nbf), nbf, Fm, fn, tg, tg + (size_t)12 * Fm, nxt, part);
+    else
+        node_angle(xcd_block(b - nbt - nbf, nbn), nbn, N, sptr, swid, scol, nxt, cur, part);
+}
+
+// its partials: wavefront k sums slot k of the energies, wavefront 6 takes the minimum of the angles'
+// dot products; out[0..5] and out[8] as the entry points read them
+__global__ __launch_bounds__(448) void k_after_finish(int nbt, int nbf, int nbn, const double *__restrict__ part,
+                                                      double *__restrict__ out)
+{
+    const int k = threadIdx.x >> 6;
+    const double *p = part + k * MAX_PART;
+    if (k == 6) {
+        if (nbn == 0) return;
+        const double m = wave_min(lane_fold(p, nbn, 1.0, MinOp()));
+        if ((threadIdx.x & 63) == 0) out[8] = m;
+    } else {
+        if (nbt == 0) return;
+        const double s = wave_sum(lane_fold(p, k < 4 ? nbt : nbf, 0.0, AddOp()));
+        if ((threadIdx.x & 63) == 0) out[k] = s;
     }
 }
 
@@ -2315,20 +2351,12 @@ void launch_spmv_debug(Ctx &c, double cst, const double2 *xin, double2 *yout)
 
 void launch_charges(Ctx &c)
 {
-    const NodeRec *nxt = c.rec[1 - c.cur];
     double2 *q = c.fmm ? nullptr : c.src_q;  // the FMM's P2M and near field take the element values
-    if (c.Tm > 0) {
-        Prof pr(c, "charges_tet");
-        k_charges_tet<<<grid1(c.Tm), BLOCK, 0, c.stream>>>(c.Tm, c.tet_nodes, c.geo, c.tet_reg, c.regions, nxt,
-                                                           c.src_rank, q, c.qe);
-    }
-    if (c.Fm > 0) {
-        Prof pr(c, "charges_tri");
-        k_charges_tri<<<grid1(c.Fm), BLOCK, 0, c.stream>>>(c.Fm, (int64_t)5 * c.Tm, c.tri_nodes, c.tri_geo, c.pos4,
-                                                           nxt, c.src_rank, q, c.tri_corr, c.qe, c.Tm);
-    }
-    Prof pr(c, "corr_gather");
-    k_corr_gather<<<c.blocks_for(c.N), BLOCK, 0, c.stream>>>(c.N, c.cinc_ptr, c.cinc_idx, c.tri_corr, c.corr);
+    const int nbf = grid1(c.Fm), nbt = grid1(c.Tm);
+    if (nbf + nbt == 0) return;
+    Prof pr(c, "charges");
+    k_charges<<<nbf + nbt, BLOCK, 0, c.stream>>>(nbf, c.Tm, c.tet_nodes, c.geo, c.tet_reg, c.regions, c.Fm, c.tri_nodes,
+                                                 c.tri_geo, c.pos4, c.rec[1 - c.cur], c.src_rank, q, c.tri_corr, c.qe);
 }
 
 // Targets per thread and shares of the sources of the direct sum: about 2,048 blocks (eight per CU)
@@ -2350,31 +2378,38 @@ void launch_direct_p2p(Ctx &c)
     else
         k_p2p_direct<1><<<nb, BLOCK, 0, c.stream>>>(c.N, c.S, ns, c.pos4, c.src_pos, c.src_q, c.p2p_part, c.d_node_inst,
                                                     c.d_inst_src);
-    k_p2p_finish<<<(c.N + P2P_FIN - 1) / P2P_FIN, BLOCK, 0, c.stream>>>(c.N, ns, c.mag, c.p2p_part, c.corr,
-                                                                        c.rec[1 - c.cur]);
+    k_p2p_finish<<<(c.N + P2P_FIN - 1) / P2P_FIN, BLOCK, 0, c.stream>>>(c.N, ns, c.mag, c.p2p_part, c.cinc_ptr,
+                                                                        c.cinc_idx, c.tri_corr, c.rec[1 - c.cur]);
+}
+
+// nbt, nbf, nbn: blocks of the parts wanted (0: left out)
+static void launch_parts(Ctx &c, const double Hext[3], const double *hsp, double amp, int nbt, int nbf, int nbn,
+                         NodeRec *cur)
+{
+    k_after<<<nbt + nbf + nbn, BLOCK, 0, c.stream>>>(nbt, nbf, nbn, c.Tm, c.tet_nodes, c.geo, c.tet_reg, c.regions,
+                                                     Hext[0], Hext[1], Hext[2], hsp, amp, c.Fm, c.tri_nodes, c.tri_geo,
+                                                     c.N, c.slice_ptr, c.slice_w, c.scol, c.rec[1 - c.cur], cur, c.epart);
+    k_after_finish<<<1, 448, 0, c.stream>>>(nbt, nbf, nbn, c.epart, c.res);
 }
 
 void launch_energy(Ctx &c, const double Hext[3], const double *hsp, double amp)
 {
-    const NodeRec *nxt = c.rec[1 - c.cur];
-    const int nbt = c.blocks_for(c.Tm), nbf = c.blocks_for(c.Fm);
-    {
-        Prof pr(c, "energy");
-        k_energy_tet<<<nbt, BLOCK, 0, c.stream>>>(c.Tm, c.tet_nodes, c.geo, c.tet_reg, c.regions, nxt, Hext[0], Hext[1],
-                                                  Hext[2], hsp, amp, c.epart);
-        if (c.Fm > 0)
-            k_energy_tri<<<nbf, BLOCK, 0, c.stream>>>(c.Fm, c.tri_nodes, c.tri_geo, c.tri_geo + (size_t)12 * c.Fm, nxt,
-                                                      c.epart);
-    }
-    k_sum_finish<<<1, 64, 0, c.stream>>>(6, 4, nbt, c.Fm > 0 ? nbf : 0, c.epart, c.res);
+    Prof pr(c, "energy");
+    launch_parts(c, Hext, hsp, amp, c.blocks_for(c.Tm), c.Fm > 0 ? c.blocks_for(c.Fm) : 0, 0, nullptr);
 }
 
 void launch_max_angle(Ctx &c)
 {
-    const int nb = c.blocks_for(c.N);
     Prof pr(c, "max_angle");
-    k_max_angle<<<nb, BLOCK, 0, c.stream>>>(c.N, c.slice_ptr, c.slice_w, c.scol, c.rec[1 - c.cur], c.epart);
-    k_min_finish<<<1, 64, 0, c.stream>>>(nb, c.epart, c.res + 8);
+    const double none[3] = {0, 0, 0};
+    launch_parts(c, none, nullptr, 0.0, 0, 0, c.blocks_for(c.N), nullptr);
+}
+
+void launch_after(Ctx &c, const double Hext[3])
+{
+    Prof pr(c, "energy_angle_evolution");
+    launch_parts(c, Hext, nullptr, 0.0, c.blocks_for(c.Tm), c.Fm > 0 ? c.blocks_for(c.Fm) : 0, c.blocks_for(c.N),
+                 c.rec[c.cur]);
 }
 
 void launch_evolution(Ctx &c)
