@@ -431,13 +431,58 @@ __global__ __launch_bounds__(ESB) void k_sp_rec_u(int N, const NodeRec *__restri
 }
 
 // Scalars of algebra::bicg_dir and algebra::iteration (src/algebra/bicg.h:82-158,
-// src/algebra/iter.h:119-178) in device memory, updated by one-block kernels between the vector
-// phases so that chunks of iterations run with no host read. stop: the loop has ended; fin = 1:
-// its last half step (x += alpha phat) is due, 2: taken.
+// src/algebra/iter.h:119-178) in device memory, so that chunks of iterations run with no host read.
+// Each phase of an iteration sums the last one's partials in every block and block 0 writes the
+// scalars that later phases need; no phase reads a scalar that its own launch writes, but for the ends
+// of the loop: half is set by the t = A shat phase (which then takes the last half step x += alpha
+// phat, or ends on an overflow) and turned into stop by the next one, because a block of the launch
+// that sets it may start after block 0 has written.
 struct SpinCtl {
-    double rho1, rho2, alpha, omega, beta, rhsn, res, tol;
-    int nit, max_iter, status, stop, fin, pad[3];
+    double rho1, rho2, alpha, omega, rhsn, res, tol;
+    int nit, max_iter, status, stop, half, pad[3];
 };
+constexpr int SP_PB = 1024;  // blocks (and partials) of a phase: beyond, the phases loop over their rows
+
+// Sum of nb partials in a fixed order, in every lane of every wavefront
+__device__ inline double part_sum(const double *__restrict__ p, int nb)
+{
+    double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
+    int i = threadIdx.x & 63;
+    for (; i + 192 < nb; i += 256) {
+        a0 += p[i];
+        a1 += p[i + 64];
+        a2 += p[i + 128];
+        a3 += p[i + 192];
+    }
+    for (; i < nb; i += 64) a0 += p[i];
+    double s = (a0 + a1) + (a2 + a3);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
+// The block's sum of v into *out: wavefronts by shuffles, then in wavefront order
+__device__ inline void part_put(double v, double *sh, double *out)
+{
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = sh[0];
+        for (int q = 1; q < ESB / 64; q++) s += sh[q];
+        *out = s;
+    }
+}
+// iteration::converged (src/algebra/iter.h:145-166): NaN sets CANNOT_CONVERGE without ending the loop,
+// as in the reference
+__device__ inline bool sp_converged(double res, const SpinCtl &k, int &status)
+{
+    if (isnan(res)) {
+        status = FG_ITER_CANNOT_CONVERGE;
+        return false;
+    }
+    const bool cv = res <= k.rhsn * k.tol;
+    if (cv) status = FG_ITER_CONVERGED;
+    return cv;
+}
 
 __global__ void k_sp_reset(SpinCtl *c, double tol, int max_iter)
 {
@@ -448,50 +493,122 @@ __global__ void k_sp_reset(SpinCtl *c, double tol, int max_iter)
     c->status = FG_ITER_UNDEFINED;
 }
 
-enum SpinPhase { SP_INIT, SP_ALPHA, SP_S, SP_OMEGA, SP_LOOP };
-
-// entry (d, e) of node i's own 3x3 block: the diffusion diagonal, and the antisymmetric s-d
-// exchange (rows y, z of X; x, z of Y; x, y of Z, with the signs of spinAcc::integrales)
-__device__ inline double self_block(int d, int e, double a, const double *S)
+// y = K x at node i (three rows): the node-pair scalars times I3, and the node's own antisymmetric s-d
+// exchange block (rows y, z of X; x, z of Y; x, y of Z, with the signs of spinAcc::integrales). The
+// node's four lanes take entries sub, sub + 4, ..., four of them in flight, and each gets the sums.
+// Bound by the latency of the gathers: with a thread per row and an entry at a time a product took
+// 13.9 us on 4,059 nodes.
+__device__ inline double3 sp_row(int i, int sub, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                 const double *__restrict__ a, const double *__restrict__ S, const double *x)
 {
-    if (d == e) return a;
-    if (d == 0) return e == 1 ? S[2] : -S[1];
-    if (d == 1) return e == 0 ? -S[2] : S[0];
-    return e == 0 ? S[1] : -S[0];
+    const int64_t b = rp[i], e = rp[i + 1];
+    const double s0 = S[3 * (size_t)i], s1 = S[3 * (size_t)i + 1], s2 = S[3 * (size_t)i + 2];
+    const double x0 = x[3 * (size_t)i], x1 = x[3 * (size_t)i + 1], x2 = x[3 * (size_t)i + 2];
+    double3 y = make_double3(0, 0, 0);
+    constexpr int U = 4;
+    for (int64_t k0 = b + sub; k0 < e; k0 += 4 * U) {
+        int j[U];
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t k = k0 + 4 * u < e ? k0 + 4 * u : k0;
+            j[u] = col[k];
+            v[u] = k0 + 4 * u < e ? a[k] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const double *q = x + 3 * (size_t)j[u];
+            y.x += v[u] * q[0];
+            y.y += v[u] * q[1];
+            y.z += v[u] * q[2];
+        }
+    }
+    for (int o = 1; o < 4; o <<= 1) {
+        y.x += __shfl_xor(y.x, o, 64);
+        y.y += __shfl_xor(y.y, o, 64);
+        y.z += __shfl_xor(y.z, o, 64);
+    }
+    y.x += s2 * x1 - s1 * x2;
+    y.y += s0 * x2 - s2 * x0;
+    y.z += s1 * x0 - s0 * x1;
+    return y;
 }
 
-// y = K x over the 3 N rows (row 3 i + d), zero on the Dirichlet rows when mask is set; partials of
-// y . w (w may be null) and, when pyy is set, of y . y. Nothing once the solver has stopped.
-__global__ __launch_bounds__(ESB) void k_sa_spmv(int n3, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+// y = K x (unmasked), before the loop
+__global__ __launch_bounds__(ESB) void k_sa_spmv(int N, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
                                                  const double *__restrict__ a, const double *__restrict__ S,
-                                                 const double *__restrict__ x, const uint8_t *__restrict__ dir, int mask,
-                                                 double *__restrict__ y, const double *__restrict__ w,
-                                                 double *__restrict__ pyw, double *__restrict__ pyy,
-                                                 const SpinCtl *__restrict__ ctl)
+                                                 const double *__restrict__ x, double *__restrict__ y)
 {
-    __shared__ double sh[ESB];
-    if (ctl && ctl->stop) return;
-    const int r = blockIdx.x * ESB + threadIdx.x;
-    double yw = 0.0, yy = 0.0;
-    if (r < n3) {
-        const int i = r / 3, d = r - 3 * i;
-        double s = 0.0;
-        for (int64_t k = rp[i]; k < rp[i + 1]; k++) {
-            const int j = col[k];
-            if (j != i) {
-                s += a[k] * x[3 * (size_t)j + d];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 3; e++) s += self_block(d, e, a[k], S + 3 * (size_t)i) * x[3 * (size_t)i + e];
-            }
-        }
-        if (mask && dir[i]) s = 0.0;
-        y[r] = s;
-        if (w) yw = s * w[r];
-        yy = s * s;
+    const int sub = threadIdx.x & 3;
+    for (int i = (blockIdx.x * ESB + threadIdx.x) >> 2; i < N; i += (gridDim.x * ESB) >> 2) {
+        const double3 z = sp_row(i, sub, rp, col, a, S, x);
+        if (sub < 3) y[3 * (size_t)i + sub] = sub == 0 ? z.x : sub == 1 ? z.y : z.z;
     }
-    if (pyw) block_sum(yw, sh, pyw + blockIdx.x);
-    if (pyy) block_sum(yy, sh, pyy + blockIdx.x);
+}
+
+// v = K phat, zero on the Dirichlet rows; partials of v . rt
+__global__ __launch_bounds__(ESB) void k_sp_v(int N, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                              const double *__restrict__ a, const double *__restrict__ S,
+                                              const uint8_t *__restrict__ dir, const SpinCtl *__restrict__ c,
+                                              const double *__restrict__ phat, const double *__restrict__ rt,
+                                              double *__restrict__ v, double *__restrict__ part)
+{
+    __shared__ double sh[ESB / 64];
+    if (c->stop) return;
+    const int sub = threadIdx.x & 3;
+    double vr = 0.0;
+    for (int i = (blockIdx.x * ESB + threadIdx.x) >> 2; i < N; i += (gridDim.x * ESB) >> 2) {
+        const double3 z = sp_row(i, sub, rp, col, a, S, phat);
+        if (sub < 3) {
+            const size_t k = 3 * (size_t)i + sub;
+            const double y = dir[i] ? 0.0 : sub == 0 ? z.x : sub == 1 ? z.y : z.z;
+            v[k] = y;
+            vr += y * rt[k];
+        }
+    }
+    part_put(vr, sh, part + 2 * SP_PB + blockIdx.x);
+}
+
+// the test on ||s|| (x += alpha phat when converged), else t = K shat, zero on the Dirichlet rows;
+// partials of t . s and t . t
+__global__ __launch_bounds__(ESB) void k_sp_t(int N, int nb3, const int64_t *__restrict__ rp,
+                                              const int32_t *__restrict__ col, const double *__restrict__ a,
+                                              const double *__restrict__ S, const uint8_t *__restrict__ dir, SpinCtl *c,
+                                              const double *__restrict__ shat, const double *__restrict__ sv,
+                                              const double *__restrict__ phat, double *__restrict__ x,
+                                              double *__restrict__ t, double *__restrict__ part)
+{
+    __shared__ double sh[2][ESB / 64];
+    const SpinCtl k = *c;
+    if (k.stop) return;
+    const double res = fabs(sqrt(part_sum(part + 3 * SP_PB, nb3)));
+    int status = k.status;
+    const bool conv = sp_converged(res, k, status);
+    const bool end = conv || status == FG_ITER_OVERFLOW || status == FG_ITER_CANNOT_CONVERGE;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c->res = res;
+        c->status = status;
+        if (end) c->half = 1;
+    }
+    const int sub = threadIdx.x & 3;
+    double ts = 0.0, tt = 0.0;
+    for (int i = (blockIdx.x * ESB + threadIdx.x) >> 2; i < N; i += (gridDim.x * ESB) >> 2) {
+        if (end) {
+            if (conv && sub < 3) x[3 * (size_t)i + sub] += k.alpha * phat[3 * (size_t)i + sub];
+            continue;
+        }
+        const double3 z = sp_row(i, sub, rp, col, a, S, shat);
+        if (sub < 3) {
+            const size_t q = 3 * (size_t)i + sub;
+            const double y = dir[i] ? 0.0 : sub == 0 ? z.x : sub == 1 ? z.y : z.z;
+            t[q] = y;
+            ts += y * sv[q];
+            tt += y * y;
+        }
+    }
+    if (end) return;
+    part_put(ts, sh[0], part + 4 * SP_PB + blockIdx.x);
+    part_put(tt, sh[1], part + 5 * SP_PB + blockIdx.x);
 }
 
 // D = 1 / diag(K), zero on the Dirichlet rows
@@ -514,10 +631,9 @@ __global__ __launch_bounds__(ESB) void k_sa_init(int n3, const double *__restric
                                                  double *__restrict__ rt, double *__restrict__ p, double *__restrict__ x,
                                                  double *__restrict__ pbb)
 {
-    __shared__ double sh[ESB];
-    const int k = blockIdx.x * ESB + threadIdx.x;
+    __shared__ double sh[ESB / 64];
     double bb = 0.0;
-    if (k < n3) {
+    for (int k = blockIdx.x * ESB + threadIdx.x; k < n3; k += gridDim.x * ESB) {
         double b = L[k];
         b -= kxd[k];
         if (dir[k / 3]) b = 0.0;
@@ -525,154 +641,120 @@ __global__ __launch_bounds__(ESB) void k_sa_init(int n3, const double *__restric
         rt[k] = b;
         p[k] = b;
         x[k] = 0.0;
-        bb = b * b;
+        bb += b * b;
     }
-    block_sum(bb, sh, pbb + blockIdx.x);
+    part_put(bb, sh, pbb + blockIdx.x);
 }
 
-// The scalar step that follows a reduction: the partials of one (two for SP_OMEGA and SP_LOOP)
-// dot products, nb each, summed in a fixed order per thread and a fixed tree; thread 0 then takes
-// the step of bicg_dir that needs them.
-__global__ __launch_bounds__(ESB) void k_sp_ctl(int nb, const double *__restrict__ part, SpinCtl *__restrict__ c,
-                                                int phase)
+// ||b||, the loop's first test, rho1 = rt . r with rt = r = b (one wavefront)
+__global__ void k_sp_init(int nb3, const double *__restrict__ part, SpinCtl *c)
 {
-    __shared__ double sh[2][ESB];
-    if (c->stop && !(phase == SP_LOOP && c->fin == 1)) return;
-    const int nsum = (phase == SP_OMEGA || phase == SP_LOOP) ? 2 : 1;
-    for (int q = 0; q < nsum; q++) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < nb; b += ESB) s += part[(size_t)q * nb + b];
-        sh[q][threadIdx.x] = s;
-    }
-    __syncthreads();
-    for (int w = ESB / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int q = 0; q < nsum; q++) sh[q][threadIdx.x] += sh[q][threadIdx.x + w];
-        __syncthreads();
-    }
+    const double bb = part_sum(part, nb3);
     if (threadIdx.x) return;
-    const double a0 = sh[0][0], a1 = nsum > 1 ? sh[1][0] : 0.0;
-    // iteration::converged (src/algebra/iter.h:145-166): NaN sets CANNOT_CONVERGE without ending
-    // the loop, as in the reference
-    auto converged = [c](double nr) {
-        c->res = fabs(nr);
-        if (isnan(c->res)) {
-            c->status = FG_ITER_CANNOT_CONVERGE;
-            return false;
-        }
-        const bool cv = c->res <= c->rhsn * c->tol;
-        if (cv) c->status = FG_ITER_CONVERGED;
-        return cv;
-    };
-    switch (phase) {
-    case SP_INIT:  // ||b||, the loop's first test, rho1 = rt . r with rt = r = b
-        c->rhsn = sqrt(a0);
-        if (converged(sqrt(a0))) {
-            c->stop = 1;
-            return;
-        }
-        c->rho1 = a0;
-        break;
-    case SP_ALPHA:  // alpha = rho1 / (v . rt)
-        c->alpha = c->rho1 / a0;
-        break;
-    case SP_S:  // the test on ||s||: the last half step, or a break on overflow / breakdown
-        if (converged(sqrt(a0))) {
-            c->stop = 1;
-            c->fin = 1;
-        } else if (c->status == FG_ITER_OVERFLOW || c->status == FG_ITER_CANNOT_CONVERGE) {
-            c->stop = 1;
-        }
-        break;
-    case SP_OMEGA:  // omega = (t . s) / (t . t)
-        c->omega = a0 / a1;
-        break;
-    case SP_LOOP:  // rho2 = rho1, ++iter, the loop's test on ||r||, rho1 = rt . r, beta
-        if (c->stop) {
-            c->fin = 2;
-            return;
-        }
-        c->rho2 = c->rho1;
-        if (++c->nit >= c->max_iter) c->status = FG_ITER_OVERFLOW;
-        if (converged(sqrt(a0))) {
-            c->stop = 1;
-            return;
-        }
-        c->rho1 = a1;
-        if (c->rho2 == 0 || c->omega == 0) {
-            c->status = FG_ITER_CANNOT_CONVERGE;
-            c->stop = 1;
-            return;
-        }
-        c->beta = (c->rho1 / c->rho2) * (c->alpha / c->omega);
-        break;
-    }
+    SpinCtl k = *c;
+    k.rhsn = sqrt(bb);
+    k.res = fabs(k.rhsn);
+    if (sp_converged(k.res, k, k.status)) k.stop = 1;
+    k.rho1 = bb;
+    *c = k;
 }
 
-// p = (p - omega v) beta + r after the first iteration; phat = D p
-__global__ __launch_bounds__(ESB) void k_sp_p(int n3, const SpinCtl *__restrict__ c, const double *__restrict__ v,
+// The loop's test on ||r||, rho1 = rt . r and beta after the first iteration, then p = (p - omega v)
+// beta + r; phat = D p
+__global__ __launch_bounds__(ESB) void k_sp_p(int n3, int nb3, SpinCtl *c, const double *__restrict__ v,
                                               const double *__restrict__ r, const double *__restrict__ D,
-                                              double *__restrict__ p, double *__restrict__ phat)
+                                              double *__restrict__ p, double *__restrict__ phat,
+                                              const double *__restrict__ part)
 {
-    if (c->stop) return;
-    const int k = blockIdx.x * ESB + threadIdx.x;
-    if (k >= n3) return;
-    double pv = p[k];
-    if (c->nit > 0) {
-        pv -= v[k] * c->omega;
-        pv *= c->beta;
-        pv += r[k];
-        p[k] = pv;
+    const SpinCtl k = *c;
+    if (k.stop) return;
+    double beta = 0.0;
+    if (k.nit > 0) {
+        const double res = fabs(sqrt(part_sum(part, nb3))), rho1 = part_sum(part + SP_PB, nb3);
+        int status = k.status;
+        bool end = sp_converged(res, k, status);
+        if (!end) {
+            if (k.rho2 == 0 || k.omega == 0) {
+                status = FG_ITER_CANNOT_CONVERGE;
+                end = true;
+            } else {
+                beta = (rho1 / k.rho2) * (k.alpha / k.omega);
+            }
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            c->res = res;
+            c->status = status;
+            c->rho1 = rho1;
+            if (end) c->stop = 1;
+        }
+        if (end) return;
     }
-    phat[k] = D[k] * pv;
+    for (int i = blockIdx.x * ESB + threadIdx.x; i < n3; i += gridDim.x * ESB) {
+        double pv = p[i];
+        if (k.nit > 0) {
+            pv -= v[i] * k.omega;
+            pv *= beta;
+            pv += r[i];
+            p[i] = pv;
+        }
+        phat[i] = D[i] * pv;
+    }
 }
 
-// s = r - alpha v; shat = D s; partials of s . s
-__global__ __launch_bounds__(ESB) void k_sp_s(int n3, const SpinCtl *__restrict__ c, const double *__restrict__ r,
+// alpha = rho1 / (v . rt); s = r - alpha v; shat = D s; partials of s . s
+__global__ __launch_bounds__(ESB) void k_sp_s(int n3, int nbn, SpinCtl *c, const double *__restrict__ r,
                                               const double *__restrict__ v, const double *__restrict__ D,
-                                              double *__restrict__ sv, double *__restrict__ shat, double *__restrict__ pss)
+                                              double *__restrict__ sv, double *__restrict__ shat,
+                                              double *__restrict__ part)
 {
-    __shared__ double sh[ESB];
+    __shared__ double sh[ESB / 64];
     if (c->stop) return;
-    const int k = blockIdx.x * ESB + threadIdx.x;
+    const double alpha = c->rho1 / part_sum(part + 2 * SP_PB, nbn);
+    if (blockIdx.x == 0 && threadIdx.x == 0) c->alpha = alpha;
     double ss = 0.0;
-    if (k < n3) {
-        const double s = r[k] + (-c->alpha) * v[k];
-        sv[k] = s;
-        shat[k] = D[k] * s;
-        ss = s * s;
+    for (int i = blockIdx.x * ESB + threadIdx.x; i < n3; i += gridDim.x * ESB) {
+        const double s = r[i] + (-alpha) * v[i];
+        sv[i] = s;
+        shat[i] = D[i] * s;
+        ss += s * s;
     }
-    block_sum(ss, sh, pss + blockIdx.x);
+    part_put(ss, sh, part + 3 * SP_PB + blockIdx.x);
 }
 
-// x += alpha phat; x += omega shat; r = s - omega t; partials of r . r and rt . r. Once stopped:
-// the last half step x += alpha phat if it is due.
-__global__ __launch_bounds__(ESB) void k_sp_x(int n3, const SpinCtl *__restrict__ c, const double *__restrict__ phat,
+// omega = (t . s) / (t . t); x += alpha phat; x += omega shat; r = s - omega t; partials of r . r and
+// rt . r; rho2 = rho1, ++iter
+__global__ __launch_bounds__(ESB) void k_sp_x(int n3, int nbn, SpinCtl *c, const double *__restrict__ phat,
                                               const double *__restrict__ shat, const double *__restrict__ sv,
                                               const double *__restrict__ tv, const double *__restrict__ rt,
-                                              double *__restrict__ x, double *__restrict__ r, double *__restrict__ prr,
-                                              double *__restrict__ prt)
+                                              double *__restrict__ x, double *__restrict__ r, double *__restrict__ part)
 {
-    __shared__ double sh[ESB];
-    const int k = blockIdx.x * ESB + threadIdx.x;
-    if (c->stop) {
-        if (c->fin == 1 && k < n3) x[k] += c->alpha * phat[k];
+    __shared__ double sh[2][ESB / 64];
+    const SpinCtl k = *c;
+    if (k.stop) return;
+    if (k.half) {  // ended by the phase before
+        if (blockIdx.x == 0 && threadIdx.x == 0) c->stop = 1;
         return;
     }
-    const double alpha = c->alpha, omega = c->omega;
+    const double omega = part_sum(part + 4 * SP_PB, nbn) / part_sum(part + 5 * SP_PB, nbn), alpha = k.alpha;
     double rr = 0.0, rtr = 0.0;
-    if (k < n3) {
-        double xv = x[k];
-        xv += alpha * phat[k];
-        xv += omega * shat[k];
-        x[k] = xv;
-        const double rv = sv[k] - tv[k] * omega;
-        r[k] = rv;
-        rr = rv * rv;
-        rtr = rt[k] * rv;
+    for (int i = blockIdx.x * ESB + threadIdx.x; i < n3; i += gridDim.x * ESB) {
+        double xv = x[i];
+        xv += alpha * phat[i];
+        xv += omega * shat[i];
+        x[i] = xv;
+        const double rv = sv[i] - tv[i] * omega;
+        r[i] = rv;
+        rr += rv * rv;
+        rtr += rt[i] * rv;
     }
-    block_sum(rr, sh, prr + blockIdx.x);
-    block_sum(rtr, sh, prt + blockIdx.x);
+    part_put(rr, sh[0], part + blockIdx.x);
+    part_put(rtr, sh[1], part + SP_PB + blockIdx.x);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c->omega = omega;
+        c->rho2 = k.rho1;
+        c->nit = k.nit + 1;
+        if (k.nit + 1 >= k.max_iter) c->status = FG_ITER_OVERFLOW;
+    }
 }
 
 // x += xd (the Dirichlet values); zero everywhere when zero_failed is set and the solver did not
@@ -957,6 +1039,7 @@ struct fg_spin {
     double tol = 0;
     int32_t max_iter = 0;
     int assemblies = 0;  // assemblies summed in K and L
+    int last_nit = 0;    // iterations of the last solve
     std::vector<fg_spin_volume> vol;
     hipStream_t stream = nullptr;
     DevBufs B;
@@ -1096,7 +1179,7 @@ int spin_setup(const fg_mesh *m, const fg_spin_volume *vol, const fg_spin_surfac
     sp.Ls = B.upload(Ls);
     for (double **q : {&sp.S, &sp.L, &sp.D, &sp.x, &sp.r, &sp.rt, &sp.p, &sp.ph, &sp.v, &sp.s, &sp.sh, &sp.t})
         *q = B.alloc<double>(n3);
-    sp.part = B.alloc<double>((size_t)2 * sp.nb3);
+    sp.part = B.alloc<double>((size_t)6 * SP_PB);
     sp.ctl = B.alloc<SpinCtl>(1);
     ESCHK(hipHostMalloc((void **)&sp.h_ctl, sizeof(SpinCtl), hipHostMallocDefault));
     return FG_OK;
@@ -1115,35 +1198,34 @@ void spin_run(fg_spin &sp, hipStream_t st, int acc, int zero_failed, fg_solve_in
     k_sa_node<<<sp.nb, ESB, 0, st>>>(N, T, sp.nptr, sp.nslot, sp.ke, sp.Ls, acc, sp.S, sp.L);
     sp.assemblies = acc ? sp.assemblies + 1 : 1;
     k_sa_diag<<<nb3, ESB, 0, st>>>(n3, sp.rp, sp.col, sp.a, sp.dir, sp.D);
-    k_sa_spmv<<<nb3, ESB, 0, st>>>(n3, sp.rp, sp.col, sp.a, sp.S, sp.Vd, sp.dir, 0, sp.v, nullptr, nullptr, nullptr,
-                                   nullptr);
-    k_sa_init<<<nb3, ESB, 0, st>>>(n3, sp.L, sp.v, sp.dir, sp.r, sp.rt, sp.p, sp.x, sp.part);
-    k_sp_ctl<<<1, ESB, 0, st>>>(nb3, sp.part, sp.ctl, SP_INIT);
+    const int nbv = std::min(nb3, SP_PB), nbn = std::min((4 * N + ESB - 1) / ESB, SP_PB);
+    k_sa_spmv<<<nbn, ESB, 0, st>>>(N, sp.rp, sp.col, sp.a, sp.S, sp.Vd, sp.v);
+    k_sa_init<<<nbv, ESB, 0, st>>>(n3, sp.L, sp.v, sp.dir, sp.r, sp.rt, sp.p, sp.x, sp.part);
+    k_sp_init<<<1, 64, 0, st>>>(nbv, sp.part, sp.ctl);
     ESCHK(hipGetLastError());
-    // chunks of iterations between host reads of the control block; bicg_dir ends by itself after
-    // at most max_iter + 1 iterations (the overflow status breaks the one after the max_iter-th)
+    // chunks of iterations between host reads of the control block, the first one as long as the last
+    // solve took and one more (its loop test); bicg_dir ends by itself after at most max_iter + 1
+    // iterations (the overflow status breaks the one after the max_iter-th)
     constexpr int CHUNK = 16;
-    const int max_chunks = sp.max_iter / CHUNK + 2;
-    double *pv = sp.part, *pt = sp.part + nb3;
-    for (int ch = 0;; ch++) {
+    int queued = 0, chunk = sp.last_nit > 0 ? sp.last_nit + 1 : CHUNK;
+    while (true) {
+        for (int it = 0; it < chunk; it++) {
+            k_sp_p<<<nbv, ESB, 0, st>>>(n3, nbv, sp.ctl, sp.v, sp.r, sp.D, sp.p, sp.ph, sp.part);
+            k_sp_v<<<nbn, ESB, 0, st>>>(N, sp.rp, sp.col, sp.a, sp.S, sp.dir, sp.ctl, sp.ph, sp.rt, sp.v, sp.part);
+            k_sp_s<<<nbv, ESB, 0, st>>>(n3, nbn, sp.ctl, sp.r, sp.v, sp.D, sp.s, sp.sh, sp.part);
+            k_sp_t<<<nbn, ESB, 0, st>>>(N, nbv, sp.rp, sp.col, sp.a, sp.S, sp.dir, sp.ctl, sp.sh, sp.s, sp.ph, sp.x, sp.t,
+                                        sp.part);
+            k_sp_x<<<nbv, ESB, 0, st>>>(n3, nbn, sp.ctl, sp.ph, sp.sh, sp.s, sp.t, sp.rt, sp.x, sp.r, sp.part);
+        }
+        queued += chunk;
+        ESCHK(hipGetLastError());
         ESCHK(hipMemcpyAsync(sp.h_ctl, sp.ctl, sizeof(SpinCtl), hipMemcpyDeviceToHost, st));
         ESCHK(hipStreamSynchronize(st));
         if (sp.h_ctl->stop) break;
-        if (ch >= max_chunks) throw std::string("spin solver: bicg_dir did not end");
-        for (int it = 0; it < CHUNK; it++) {
-            k_sp_p<<<nb3, ESB, 0, st>>>(n3, sp.ctl, sp.v, sp.r, sp.D, sp.p, sp.ph);
-            k_sa_spmv<<<nb3, ESB, 0, st>>>(n3, sp.rp, sp.col, sp.a, sp.S, sp.ph, sp.dir, 1, sp.v, sp.rt, pv, nullptr,
-                                           sp.ctl);
-            k_sp_ctl<<<1, ESB, 0, st>>>(nb3, sp.part, sp.ctl, SP_ALPHA);
-            k_sp_s<<<nb3, ESB, 0, st>>>(n3, sp.ctl, sp.r, sp.v, sp.D, sp.s, sp.sh, pv);
-            k_sp_ctl<<<1, ESB, 0, st>>>(nb3, sp.part, sp.ctl, SP_S);
-            k_sa_spmv<<<nb3, ESB, 0, st>>>(n3, sp.rp, sp.col, sp.a, sp.S, sp.sh, sp.dir, 1, sp.t, sp.s, pv, pt, sp.ctl);
-            k_sp_ctl<<<1, ESB, 0, st>>>(nb3, sp.part, sp.ctl, SP_OMEGA);
-            k_sp_x<<<nb3, ESB, 0, st>>>(n3, sp.ctl, sp.ph, sp.sh, sp.s, sp.t, sp.rt, sp.x, sp.r, pv, pt);
-            k_sp_ctl<<<1, ESB, 0, st>>>(nb3, sp.part, sp.ctl, SP_LOOP);
-        }
-        ESCHK(hipGetLastError());
+        if (queued > sp.max_iter + 2 * CHUNK) throw std::string("spin solver: bicg_dir did not end");
+        chunk = CHUNK;
     }
+    sp.last_nit = std::min(sp.h_ctl->nit, sp.max_iter);
     k_sp_finish<<<nb3, ESB, 0, st>>>(n3, sp.ctl, zero_failed, sp.Vd, sp.x);
     ESCHK(hipGetLastError());
     if (info) {

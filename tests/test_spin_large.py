@@ -1,0 +1,27 @@
+"""The spin solver's phases past one pass of their grids (more than 65,536 nodes, 262,144 unknowns):
+diffusion alone on a bar against the closed form of tests/test_spin_accumulation.py, whose P1 error at
+this cell size is below 1e-3; and a second solve, whose first chunk of iterations has the length of the
+first one's, gives the same field."""
+import numpy as np
+import pytest
+
+from feellgood_amd.engine import SpinSolver
+from test_electrostatic import bar
+from test_spin_accumulation import JN, MUB_E, S0, SURF, UP, vol
+
+
+@pytest.mark.gpu
+def test_diffusion_on_a_fine_bar():
+    m, own, pos = bar(0.0, cells=(60, 38, 38))
+    assert m.n_nodes > 87381
+    u = np.tile([0.0, 0.0, 1.0], (m.n_nodes, 1))
+    sp = SpinSolver(m, [vol(), vol()], SURF, np.zeros(m.n_nodes), tol=1e-10, max_iter=3000)
+    s, info = sp.solve(u, accumulate=False)
+    assert info.status == 0 and info.iterations > 16
+    x = pos[:, 0] - pos[:, 0].min()
+    L, lsf = np.ptp(pos[:, 0]), 10e-9
+    s1 = -JN * MUB_E * np.array(UP)
+    ref = (np.outer(np.sinh((L - x) / lsf), S0) + np.outer(np.sinh(x / lsf), s1)) / np.sinh(L / lsf)
+    assert np.abs(s - ref).max() <= 1e-3 * np.abs(ref).max()
+    again, info2 = sp.solve(u, accumulate=False)
+    assert info2.iterations == info.iterations and np.array_equal(again, s)
