@@ -790,17 +790,17 @@ template <> struct P2mSrc<double4> { typedef double2 W2; };
 template <> struct P2mSrc<float4> { typedef float2 W2; };
 
 template <int P, int G, unsigned MASK, class F, class S4>
-__global__ __launch_bounds__(64) void k_fmm_p2m(int nleaf, int Tm, const int32_t *__restrict__ leaf_cell,
-                                                const double4 *__restrict__ cen, const int32_t *__restrict__ sb,
-                                                const int32_t *__restrict__ se, const S4 *__restrict__ pos,
-                                                const int32_t *__restrict__ code,
-                                                const typename P2mSrc<S4>::W2 *__restrict__ tw,
-                                                const double2 *__restrict__ qe, F *__restrict__ M)
+__device__ __forceinline__ void p2m_leaf(int grp, int nleaf, int Tm, const int32_t *__restrict__ leaf_cell,
+                                         const double4 *__restrict__ cen, const int32_t *__restrict__ sb,
+                                         const int32_t *__restrict__ se, const S4 *__restrict__ pos,
+                                         const int32_t *__restrict__ code,
+                                         const typename P2mSrc<S4>::W2 *__restrict__ tw,
+                                         const double2 *__restrict__ qe, F *__restrict__ M)
 {
     constexpr int NCo = fcount(P), NH = p2m_half_count<P>(MASK);
     constexpr bool REL = std::is_same<S4, float4>::value;  // positions already relative, in cell widths
     const int lane = threadIdx.x & (G - 1);
-    const int li = (blockIdx.x * 64 + threadIdx.x) / G;
+    const int li = (grp * 64 + threadIdx.x) / G;
     const bool act = li < nleaf;
     const int cell = act ? leaf_cell[li] : 0;
     F au[2 * NH], av[2 * NH];
@@ -809,27 +809,41 @@ __global__ __launch_bounds__(64) void k_fmm_p2m(int nleaf, int Tm, const int32_t
     const double4 c = cen[cell];
     const double iw = c.w;
     const int kb = act ? sb[li] + lane : 0, ke = act ? se[li] : 0;
-    S4 x = kb < ke ? pos[kb] : S4{0, 0, 0, 0};
-    int cd = kb < ke ? code[kb] : 0;
+    // the values of the next source and the code of the one after it travel under this one's work
+    struct Val {
+        double2 a, b, d;
+        typename P2mSrc<S4>::W2 w;
+    };
+    auto load = [&](int cc) {
+        Val v{{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+        const int gk = ~cc, e0 = cc >= 0 ? cc : Tm + 3 * (gk >> 2);
+        v.a = qe[e0];
+        if (cc < 0) {
+            v.b = qe[e0 + 1];
+            v.d = qe[e0 + 2];
+            v.w = tw[gk];
+        }
+        return v;
+    };
+    S4 x{0, 0, 0, 0};
+    Val v{{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    int cd = 0;
+    if (kb < ke) {
+        const int c0 = code[kb];
+        x = pos[kb];
+        cd = code[min(kb + G, ke - 1)];
+        v = load(c0);
+    }
     for (int k = kb; k < ke; k += G) {
         const S4 xc = x;
-        const int cc = cd;
-        if (k + G < ke) {  // the next source, loaded under this one's work
+        const Val vc = v;
+        if (k + G < ke) {
             x = pos[k + G];
-            cd = code[k + G];
+            v = load(cd);
+            cd = code[min(k + 2 * G, ke - 1)];
         }
-        F qu, qv;
-        if (cc >= 0) {
-            const double2 e = qe[cc];
-            qu = xc.w * (F)e.x;
-            qv = xc.w * (F)e.y;
-        } else {
-            const int gk = ~cc, e0 = Tm + 3 * (gk >> 2);
-            const auto w12 = tw[gk];
-            const double2 a = qe[e0], b = qe[e0 + 1], d = qe[e0 + 2];
-            qu = xc.w * (F)a.x + w12.x * (F)b.x + w12.y * (F)d.x;
-            qv = xc.w * (F)a.y + w12.x * (F)b.y + w12.y * (F)d.y;
-        }
+        const F qu = xc.w * (F)vc.a.x + vc.w.x * (F)vc.b.x + vc.w.y * (F)vc.d.x;
+        const F qv = xc.w * (F)vc.a.y + vc.w.x * (F)vc.b.y + vc.w.y * (F)vc.d.y;
         F rx, ry, rz;
         if constexpr (REL) {
             rx = xc.x;
@@ -865,6 +879,21 @@ __global__ __launch_bounds__(64) void k_fmm_p2m(int nleaf, int Tm, const int32_t
             }
         }
     }
+}
+
+template <int P, int G, unsigned HALF_A, unsigned HALF_B, class F, class S4>
+__global__ __launch_bounds__(64, sizeof(F) == 4 && P <= 8 ? 3 : 1) void k_fmm_p2m(int nleaf, int Tm, const int32_t *__restrict__ leaf_cell,
+                                                const double4 *__restrict__ cen, const int32_t *__restrict__ sb,
+                                                const int32_t *__restrict__ se, const S4 *__restrict__ pos,
+                                                const int32_t *__restrict__ code,
+                                                const typename P2mSrc<S4>::W2 *__restrict__ tw,
+                                                const double2 *__restrict__ qe, F *__restrict__ M)
+{
+    const int grp = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7);
+    if (blockIdx.x & 8)
+        p2m_leaf<P, G, HALF_B, F, S4>(grp, nleaf, Tm, leaf_cell, cen, sb, se, pos, code, tw, qe, M);
+    else
+        p2m_leaf<P, G, HALF_A, F, S4>(grp, nleaf, Tm, leaf_cell, cen, sb, se, pos, code, tw, qe, M);
 }
 
 // The P2M source records from the sources in tree order: position (and, in FP32, relative to the
@@ -2297,23 +2326,18 @@ static void run_fmm(Ctx &c)
     {
         Prof pr(c, "fmm_p2m");
         constexpr int G = 8;  // lanes per leaf (4 measured slower: longer per-lane source loops)
-        const unsigned nb = (unsigned)((NL * G + 63) / 64);
+        const unsigned nb = (unsigned)((NL * G + 511) / 512 * 16);  // eight groups, each half of the columns
         if (NL > 0) {
-            if constexpr (std::is_same<F, float>::value) {
-                k_fmm_p2m<PP, G, p2m_acc_half_mask<PP>(0), float, float4><<<nb, 64, 0, c.stream>>>(
-                    NL, c.Tm, P.d_leaf_cell, P.d_cen, P.d_leaf_sb, P.d_leaf_se, (const float4 *)P.d_p2m_pos,
-                    P.d_p2m_code, (const float2 *)P.d_p2m_tw, c.qe, M);
-                k_fmm_p2m<PP, G, p2m_acc_half_mask<PP>(1), float, float4><<<nb, 64, 0, c.stream>>>(
-                    NL, c.Tm, P.d_leaf_cell, P.d_cen, P.d_leaf_sb, P.d_leaf_se, (const float4 *)P.d_p2m_pos,
-                    P.d_p2m_code, (const float2 *)P.d_p2m_tw, c.qe, M);
-            } else {
-                k_fmm_p2m<PP, G, p2m_half_mask<PP>(0), double, double4><<<nb, 64, 0, c.stream>>>(
-                    NL, c.Tm, P.d_leaf_cell, P.d_cen, P.d_leaf_sb, P.d_leaf_se, (const double4 *)P.d_p2m_pos,
-                    P.d_p2m_code, (const double2 *)P.d_p2m_tw, c.qe, M);
-                k_fmm_p2m<PP, G, p2m_half_mask<PP>(1), double, double4><<<nb, 64, 0, c.stream>>>(
-                    NL, c.Tm, P.d_leaf_cell, P.d_cen, P.d_leaf_sb, P.d_leaf_se, (const double4 *)P.d_p2m_pos,
-                    P.d_p2m_code, (const double2 *)P.d_p2m_tw, c.qe, M);
-            }
+            if constexpr (std::is_same<F, float>::value)
+                k_fmm_p2m<PP, G, p2m_acc_half_mask<PP>(0), p2m_acc_half_mask<PP>(1), float, float4>
+                    <<<nb, 64, 0, c.stream>>>(NL, c.Tm, P.d_leaf_cell, P.d_cen, P.d_leaf_sb, P.d_leaf_se,
+                                              (const float4 *)P.d_p2m_pos, P.d_p2m_code, (const float2 *)P.d_p2m_tw, c.qe,
+                                              M);
+            else
+                k_fmm_p2m<PP, G, p2m_half_mask<PP>(0), p2m_half_mask<PP>(1), double, double4>
+                    <<<nb, 64, 0, c.stream>>>(NL, c.Tm, P.d_leaf_cell, P.d_cen, P.d_leaf_sb, P.d_leaf_se,
+                                              (const double4 *)P.d_p2m_pos, P.d_p2m_code, (const double2 *)P.d_p2m_tw,
+                                              c.qe, M);
         }
     }
     const int fine = std::max(2, P.m2p_lmin);
