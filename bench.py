@@ -120,27 +120,24 @@ def bench_dots(args):
 
 
 # ------------------------------------------------------------------ byte / flop models
-def m2p_flops(p):
-    """FP64 (or FP32) operations of one multipole-to-target evaluation of two expansions of degree
-    p, as m2p_eval2_r performs them: setup (r^2, refined 1/r^2 and 1/r), the real m = 0 column, the
-    complex columns m >= 1 (diagonal step, first off-diagonal, three-term recurrence) with four
-    fused multiply-adds per term, and the caller's offset and scaling."""
-    f = 25                                              # setup
-    f += 2 + (5 if p >= 1 else 0) + 10 * max(0, p - 1)  # m = 0 column
-    for m in range(1, p + 1):
-        f += 18 + (15 if m < p else 0) + 17 * max(0, p - m - 1)
-    return f + 14
+def m2p_flops(p, pv=None):
+    """FP64 (or FP32) operations of one multipole-to-target evaluation of two expansions, the first
+    of degree p, the second (charges of v) of degree pv <= p, as m2p_cell performs them with both in
+    one pass: the offset, r^2, 1/r^2 and 1/r, per column the factors q_n and their fused
+    multiply-adds into the sums of the two sets, Horner's rule over the columns, the final scaling.
+    The sums over the cells of a task are on the matrix cores and not counted."""
+    pv = p if pv is None else pv
+    f = 6 + 5 + 5 + 2 + 2 + 5 + 2 * 6       # offset, r^2, 1/r^2, zeta and zeta^2, e, 1/r, the two results
+    for m in range(p + 1):
+        for n in range(m + 1, p + 1):
+            f += {1: 0, 2: 2, 3: 3}.get(n - m, 4)                       # q_n
+            f += (4 if m else 2) * (1 + (n <= pv))                      # sums of the column
+        if m:
+            f += 8 * ((m < p) + (m < pv))                               # Horner
+    return f
 
 
 V_DEGREE = 4  # degree of the far field of the charges of v in the mixed-precision mode
-
-
-def m2p_flops_v(p, pv):
-    """m2p_flops with the second expansion (charges of v) taken to degree pv <= p only: its fused
-    multiply-adds of degrees above pv (one per real m = 0 term, two per complex term) drop out."""
-    return m2p_flops(p) - sum(2 + 4 * n for n in range(pv + 1, p + 1))
-
-
 FAR_DEGREE = {4: 2, 6: 4, 8: 5, 10: 6}  # lower degree of the far list entries, per order
 
 
@@ -222,8 +219,8 @@ def kernel_model(name, n):
             "fmm_near": ("hbm", (4 if mixed else 8) * f["near_coefs"] + 4 * f["near_columns"] + 16 * (T + 3 * F)
                          + (8 + 16 + 16 + 4) * Tg + 12 * f["target_leaves"]),
             "fmm_m2p": ("valu32" if mixed else "valu64",
-                        m2p_flops_v(p, min(p, pv)) * (f["m2p_pairs"] - f["m2p_far_pairs"])
-                        + m2p_flops_v(pf, min(pf, pv)) * f["m2p_far_pairs"]),
+                        m2p_flops(p, min(p, pv)) * (f["m2p_pairs"] - f["m2p_far_pairs"])
+                        + m2p_flops(pf, min(pf, pv)) * f["m2p_far_pairs"]),
             "fmm_m2l": ("mfma32" if mixed else "mfma64", m2l_flops(p) * f["m2l_pairs"]),
             "fmm_m2m": ("mfma32" if mixed else "mfma64", m2m_flops(p) * f["m2m_cells"]),
             "fmm_p2m": ("valu32" if mixed else "valu64", p2m_flops(p) * f["sources"]),
