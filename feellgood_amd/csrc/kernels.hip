@@ -397,6 +397,14 @@ __device__ inline int vec_first(int blk, int N)
 }
 template <int FORM>
 __device__ inline int row_step() { return (int)gridDim.x * (BLOCK / form_lanes(FORM)); }
+// Whether a phase reads the control block (and k_spmv_t the norm) before its rows: in all forms but the
+// small meshes' 4, where the rows' reads beside it hide a microsecond a phase. The host queues
+// iterations before it knows that the solve has ended, and what those read, they read in vain: with
+// the rows read first everywhere, a solve that had nothing left to do took 158 us on 110,592 nodes
+// and 296 us on 262,144, against 88 and 174 (and a run's solves, of five iterations, 529 and 874
+// against 466 and 668).
+template <int FORM>
+__device__ constexpr bool decide_first() { return FORM != 4; }
 template <int FORM>
 __device__ inline int row_sub() { return (int)threadIdx.x & (form_lanes(FORM) - 1); }
 
@@ -567,8 +575,7 @@ __global__ void k_inst_rhsn(int K, const double *__restrict__ n2, KrylovCtl *ctl
 
 // The five phases of an iteration. On small meshes each is a chain of dependent memory reads (the
 // control block, the last phase's partials, the rows) of about a microsecond each, so a phase issues
-// all three together and decides afterwards; a row read by a phase that then has nothing to do is
-// read in vain.
+// all three together and decides afterwards; on larger ones it decides first (decide_first).
 
 // (C) loop head: convergence on ||r||, rho_1 = rt.r, beta, p = r + beta (p - omega v),
 // p^ = D p, w = lift(p^)  (src/algebra/bicg.h:180-199)
@@ -580,6 +587,7 @@ __global__ __launch_bounds__(BLOCK) void k_iter_p(int N, int nb, KrylovCtl *ctl,
                                                   double2 *__restrict__ p, double2 *__restrict__ ph,
                                                   double4 *__restrict__ w, const double *__restrict__ part)
 {
+    if (decide_first<FORM>() && ctl->done) return;
     int i = vec_first<FORM>(blockIdx.x, N);
     double2 ri, vi, pi, d;
     double4 e, q;
@@ -651,9 +659,9 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_v(int N, double cst, STENCIL_ARG
 {
     const int sub = row_sub<FORM>();
     const int done = ctl->done;
+    if (decide_first<FORM>() && done) return;
     double vr = 0;
     for (int i = row_first<FORM>(lblock()); i < N; i += row_step<FORM>()) {
-        if (FORM == 0 && done) return;
         double2 y = make_double2(0, 0);
         if (mag[i]) y = stencil_row<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i], sub);
         if (done) return;
@@ -678,6 +686,7 @@ __global__ __launch_bounds__(BLOCK) void k_iter_s(int N, int nb, KrylovCtl *ctl,
                                                   double2 *__restrict__ s, double2 *__restrict__ sh,
                                                   double4 *__restrict__ w, double *__restrict__ part)
 {
+    if (decide_first<FORM>() && ctl->done) return;
     int i = vec_first<FORM>(blockIdx.x, N);
     double2 ri, vi, d;
     double4 e, q;
@@ -724,7 +733,7 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STE
 {
     const int sub = row_sub<FORM>();
     int i = row_first<FORM>(lblock());
-    // the first row's product goes under the reads of the control block and the partials (but form 0)
+    // on small meshes the first row's product goes under the reads of the control block and the partials
     double2 y = make_double2(0, 0), si = make_double2(0, 0);
     auto row = [&]() {
         y = make_double2(0, 0);
@@ -732,7 +741,8 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STE
         si = s[i];
     };
     const KrylovCtl k = *ctl;
-    if (FORM != 0 && i < N) row();
+    if (decide_first<FORM>() && k.done) return;
+    if (!decide_first<FORM>() && i < N) row();
     const int slots[1] = {4};
     double red[1];
     block_load<1>(part, slots, nb, red);
@@ -769,7 +779,7 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_t(int N, int nb, double cst, STE
         return;
     }
     double ts = 0, tt = 0;
-    if (FORM == 0 && i < N) row();
+    if (decide_first<FORM>() && i < N) row();
     while (i < N) {
         if (sub == 0) {
             t[i] = y;
@@ -792,6 +802,7 @@ __global__ __launch_bounds__(BLOCK) void k_iter_x(int N, int nb, KrylovCtl *ctl,
                                                   double2 *__restrict__ x, double2 *__restrict__ r,
                                                   double *__restrict__ part)
 {
+    if (decide_first<FORM>() && ctl->done) return;
     int i = vec_first<FORM>(blockIdx.x, N);
     double2 xi, h, hs, si, ti, q;
     auto load = [&]() {
@@ -1274,6 +1285,7 @@ __global__ __launch_bounds__(BLOCK) void kf_iter_p(int N, int nb, KrylovCtl *ic,
                                                    float2 *__restrict__ p, float2 *__restrict__ ph,
                                                    float4 *__restrict__ w, const double *__restrict__ part)
 {
+    if (decide_first<FORM>() && ic->done) return;
     int i = vec_first<FORM>(blockIdx.x, N);
     float2 ri, vi, pi, d;
     float4 e, q;
@@ -1345,9 +1357,9 @@ __global__ __launch_bounds__(BLOCK) void kf_spmv_v(int N, float cst, STENCIL_ARG
 {
     const int sub = row_sub<FORM>();
     const int done = ic->done;
+    if (decide_first<FORM>() && done) return;
     double vr = 0;
     for (int i = row_first<FORM>(lblock()); i < N; i += row_step<FORM>()) {
-        if (FORM == 0 && done) return;
         float2 y = make_float2(0, 0);
         if (mag[i]) y = stencil_row_f<FORM>(i, cst, sptr, swid, scol, sval, w, ep4, eq4, Dg, ph[i], sub);
         if (done) return;
@@ -1370,6 +1382,7 @@ __global__ __launch_bounds__(BLOCK) void kf_iter_s(int N, int nb, KrylovCtl *ic,
                                                    float2 *__restrict__ s, float2 *__restrict__ sh,
                                                    float4 *__restrict__ w, double *__restrict__ part)
 {
+    if (decide_first<FORM>() && ic->done) return;
     int i = vec_first<FORM>(blockIdx.x, N);
     float2 ri, vi, d;
     float4 e, q;
@@ -1422,7 +1435,8 @@ __global__ __launch_bounds__(BLOCK) void kf_spmv_t(int N, int nb, float cst, STE
         si = s[i];
     };
     const KrylovCtl k = *ic;
-    if (FORM != 0 && i < N) row();
+    if (decide_first<FORM>() && k.done) return;
+    if (!decide_first<FORM>() && i < N) row();
     const int slots[1] = {4};
     double red[1];
     block_load<1>(part, slots, nb, red);
@@ -1459,7 +1473,7 @@ __global__ __launch_bounds__(BLOCK) void kf_spmv_t(int N, int nb, float cst, STE
         return;
     }
     double ts = 0, tt = 0;
-    if (FORM == 0 && i < N) row();
+    if (decide_first<FORM>() && i < N) row();
     while (i < N) {
         if (sub == 0) {
             t[i] = y;
@@ -1481,6 +1495,7 @@ __global__ __launch_bounds__(BLOCK) void kf_iter_x(int N, int nb, KrylovCtl *ic,
                                                    float2 *__restrict__ x, float2 *__restrict__ r,
                                                    double *__restrict__ part)
 {
+    if (decide_first<FORM>() && ic->done) return;
     int i = vec_first<FORM>(blockIdx.x, N);
     float2 xi, h, hs, si, ti, q;
     auto load = [&]() {

@@ -65,3 +65,28 @@ def test_batch_blocks(sizes, block):
     off = 2 * g.layout()[0]
     for a, b in zip(off[:-1], off[1:]):
         assert np.linalg.norm(r[a:b]) <= 2 * TOL * np.linalg.norm(rhs[a:b])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("krylov", ["fp64", "mixed"])
+@pytest.mark.parametrize("cells", [(59, 59, 59), (63, 63, 63), (64, 63, 63)])
+def test_iterations_queued_past_the_end_read_no_rows(cells, krylov):
+    """The second solve of a system starts from the first one's solution and ends at its first test, so
+    the two iterations queued behind it have nothing to do: their products take about as long as an empty
+    launch between two events (6 us, against 20 to 50 for the one that forms the first residual)."""
+    m = HostMesh.cuboid(tuple(3.0 * c for c in cells), cells, jitter=0.1, seed=5)
+    m.prepare({"volume": dict(Ms=8e5, Ae=1.3e-11, alpha=0.1)})
+    rng = np.random.default_rng(1)
+    u = np.array([1.0, 0.4, 0.0]) + rng.uniform(-0.2, 0.2, size=(m.n_nodes, 3))
+    u /= np.linalg.norm(u, axis=1, keepdims=True)
+    g = Engine(m.mesh, tol=TOL, max_iter=1000, krylov=krylov, profile=True)
+    g.set_state(nv.FG_BOTH, u=u)
+    g.base_projection(0.3)
+    g.prepare_elements(np.array([1e4, 2e4, -3e3]), 2e-14, 1.05)
+    assert not g.solve(2e-14)[0] and not g.solve(2e-14)[0]
+    g.reset_kernel_stats()
+    for _ in range(5):
+        failed, info = g.solve(2e-14)
+        assert not failed and info.iterations == 0
+    t = {k: ms / n for k, (n, ms) in g.kernel_stats().items() if n}
+    assert t["spmv"] <= 0.45 * t["spmv_r0"], t
