@@ -2185,12 +2185,18 @@ void launch_basis(Ctx &c, double r)
     k_basis<<<c.blocks_for(c.N), BLOCK, 0, c.stream>>>(c.N, cos(r), sin(r), c.rec[c.cur], c.ep4, c.eq4);
 }
 
-// Form of the solver's kernels and their blocks: four lanes per row while a row's lanes all have a
-// thread, a lane per row in one pass up to the grid's size, then passes over the rows.
+// Form of the solver's kernels and their blocks: four lanes per row up to FORM4_ROWS, a lane per row in
+// one pass up to the grid's size, then passes over the rows. With four lanes and with one, a run's
+// solves of 5 iterations (FP64 / FP32) take 263 / 384 against 264 / 386 us on 6,859 nodes, 315 / 411
+// against 311 / 410 on 24,389, 283 / 332 against 309 / 343 on 32,768, 293 / 360 against 271 / 348 on
+// 44,688, 409 / 451 against 332 / 406 on 57,456 and 360 / 422 against 352 / 412 on 65,536; the largest
+// one-pass mesh, 262,144 nodes, takes 668 / 750 in one pass and 669 / 771 with form 0.
+constexpr int FORM4_ROWS = 32768;
 template <class F>
 static void krylov_shape(const Ctx &c, F &&go)
 {
-    if (c.N <= MAX_PART * BLOCK / 4)
+    static_assert(FORM4_ROWS <= MAX_PART * BLOCK / 4, "a lane for every row's four");
+    if (c.N <= FORM4_ROWS)
         go(std::integral_constant<int, 4>(), (c.N + BLOCK / 4 - 1) / (BLOCK / 4));
     else if (c.N <= MAX_PART * BLOCK)
         go(std::integral_constant<int, 1>(), c.blocks_for(c.N));

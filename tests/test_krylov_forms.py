@@ -1,6 +1,7 @@
 """The solver's kernels in each of their forms (a whole solve in one block of 256, 512 or 1,024 threads;
 four lanes per row; a lane per row in one pass of the grid; a lane per row in several passes) at the
-edges between them: 256, 512 and 1,024 nodes, 65,536 and 262,144, and the next mesh after each. A batch's
+edges between them: 256, 512 and 1,024 nodes, 32,768 and 262,144, and the next mesh after each (and
+65,536, the most that four lanes per row could take). A batch's
 blocks with the lifted vector in LDS (up to 6,400 nodes in the largest instance) and in memory. The accepted solution's residual is recomputed in
 numpy from the assembled system; BiCGSTAB tests its recursive residual, which drifts from the true
 one by rounding only, so it is held to twice the tolerance. In FP32 iterations the accepted residual is
@@ -18,7 +19,7 @@ TOL = 1e-9
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("krylov", ["fp64", "mixed"])
-@pytest.mark.parametrize("cells", [(1, 1, 1), (2, 2, 6), (7, 7, 3), (7, 7, 7), (8, 7, 7), (15, 7, 7), (16, 7, 7), (31, 31, 63), (32, 31, 63), (63, 63, 63), (64, 63, 63)])
+@pytest.mark.parametrize("cells", [(1, 1, 1), (2, 2, 6), (7, 7, 3), (7, 7, 7), (8, 7, 7), (15, 7, 7), (16, 7, 7), (31, 31, 31), (31, 31, 32), (31, 31, 63), (32, 31, 63), (63, 63, 63), (64, 63, 63)])
 def test_solution_at_form_edges(cells, krylov):
     m = HostMesh.cuboid(tuple(3.0 * c for c in cells), cells, jitter=0.1, seed=5)
     m.prepare({"volume": dict(Ms=8e5, Ae=1.3e-11, alpha=0.1)})
@@ -69,11 +70,11 @@ def test_batch_blocks(sizes, block):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("krylov", ["fp64", "mixed"])
-@pytest.mark.parametrize("cells", [(59, 59, 59), (63, 63, 63), (64, 63, 63)])
+@pytest.mark.parametrize("cells", [(31, 31, 63), (47, 47, 47), (63, 63, 63), (64, 63, 63)])
 def test_iterations_queued_past_the_end_read_no_rows(cells, krylov):
     """The second solve of a system starts from the first one's solution and ends at its first test, so
     the two iterations queued behind it have nothing to do: their products take about as long as an empty
-    launch between two events (6 us, against 20 to 50 for the one that forms the first residual)."""
+    launch between two events (6 us, against 14 to 50 for the one that forms the first residual)."""
     m = HostMesh.cuboid(tuple(3.0 * c for c in cells), cells, jitter=0.1, seed=5)
     m.prepare({"volume": dict(Ms=8e5, Ae=1.3e-11, alpha=0.1)})
     rng = np.random.default_rng(1)
@@ -89,4 +90,5 @@ def test_iterations_queued_past_the_end_read_no_rows(cells, krylov):
         failed, info = g.solve(2e-14)
         assert not failed and info.iterations == 0
     t = {k: ms / n for k, (n, ms) in g.kernel_stats().items() if n}
-    assert t["spmv"] <= 0.45 * t["spmv_r0"], t
+    empty = min(t.values())
+    assert t["spmv"] - empty <= 0.3 * (t["spmv_r0"] - empty), t
