@@ -1532,15 +1532,25 @@ __device__ __forceinline__ void m2p_cell(const R (&cu)[2 * fcount(Q)], const R (
 // 32-bit registers of coefficients. Where both sets do not fit together (FP64 from degree 6) each
 // set has its own pass: the recurrences run twice (440 operations a pair against 355 at degree 8),
 // but every coefficient is fetched once; two passes over halves of the columns of both sets, which
-// fetch each 64-byte piece twice, took 1.02 ms against 0.84 on the 490k film.
-constexpr int M2P_REGS = 172;
+// fetch each 64-byte piece twice, took 1.02 ms against 0.84 on the 490k film. A set of more than
+// M2P_REGS (FP64, order 10: 242) is split into halves of at most M2P_HALF, columns 0 to 3 and 4 to 10:
+// unequal parts of at most 172 spilled (164 bytes a lane), and with every piece of a set fetched for
+// both parts M2P took 1.70 ms on 85,547 nodes, against 1.00 ms in the row layout and 1.08 ms now
+// (6.91, 4.50 and 4.65 ms on 353,157).
+constexpr int M2P_REGS = 172, M2P_HALF = 132;
+// registers of column m of both sets
+constexpr int m2p_col_regs(int Q, int QV, int m, int bytes)
+{
+    return (m ? 2 : 1) * ((Q + 1 - m) + (QV >= m ? QV + 1 - m : 0)) * (bytes / 4);
+}
 template <int Q, int QV, class R>
 constexpr int m2p_last_col(int ma)
 {
-    int regs = 0, m = ma;
+    int whole = 0, regs = 0, m = ma;
+    for (int q = 0; q <= Q; q++) whole += m2p_col_regs(Q, QV, q, (int)sizeof(R));
     for (; m <= Q; m++) {
-        const int c = (m ? 2 : 1) * ((Q + 1 - m) + (QV >= m ? QV + 1 - m : 0)) * (int)(sizeof(R) / 4);
-        if (m > ma && regs + c > M2P_REGS) break;
+        const int c = m2p_col_regs(Q, QV, m, (int)sizeof(R));
+        if (m > ma && regs + c > (whole > M2P_REGS ? M2P_HALF : M2P_REGS)) break;
         regs += c;
     }
     return m - 1;
@@ -1557,15 +1567,46 @@ struct M2pWave {
     int32_t toct[16];
 };
 
+// The pieces of a set (NK coefficients from element BASE of a cell's storage on) that hold coefficients
+// of columns MA..MB.
+template <int P, int NK, int BASE, int MA, int MB, class R> struct M2pPieces {
+    static constexpr int E = 16 / (int)sizeof(R);               // elements per 16-byte unit
+    static constexpr int S0 = BASE / E * E, PE = 4 * E;  // first element of the first piece; elements of a piece
+    static constexpr int all = (BASE + NK - S0 + PE - 1) / PE;
+    __host__ __device__ static constexpr bool has(int k)  // coefficient k is read
+    {
+        if (k < 0 || k >= NK) return false;
+        const int m = (k >> 1) - fidx(XL<P>::deg(k), 0);
+        return m >= MA && m <= MB && !(m == 0 && (k & 1));
+    }
+    __host__ __device__ static constexpr bool need(int q)
+    {
+        for (int e = 0; e < PE; e++)
+            if (has(S0 + q * PE + e - BASE)) return true;
+        return false;
+    }
+    __host__ __device__ static constexpr int count()
+    {
+        int n = 0;
+        for (int q = 0; q < all; q++) n += need(q);
+        return n;
+    }
+    __host__ __device__ static constexpr int at(int i)  // the i-th of them
+    {
+        int q = 0;
+        for (; !need(q) || i > 0; q++) i -= need(q);
+        return q;
+    }
+};
+
 // Coefficients k of [0, NK) of one set (base: its first element of a cell's storage) that belong to
 // columns MA..MB, of this lane's cell, into c.
 template <int P, int NK, int BASE, int MA, int MB, class R>
 __device__ __forceinline__ void m2p_load(const R *__restrict__ M, const int32_t (&cells)[4], int nload, int row,
                                          M2pWave &W, R (&c)[NK])
 {
-    constexpr int E = 16 / (int)sizeof(R);           // elements per 16-byte unit
-    constexpr int S0 = BASE / E * E, PE = 4 * E;  // first element of the first piece; elements of a piece
-    constexpr int NP = (BASE + NK - S0 + PE - 1) / PE;
+    using L = M2pPieces<P, NK, BASE, MA, MB, R>;
+    constexpr int E = L::E, S0 = L::S0, PE = L::PE, NP = L::count();
     const int lane = threadIdx.x & 63, sub = lane & 3;
     constexpr int G = 8;  // pieces in flight (their registers are the coefficients' own until then)
     static_for<0, (NP + G - 1) / G>([&](auto gc) {
@@ -1575,12 +1616,12 @@ __device__ __forceinline__ void m2p_load(const R *__restrict__ M, const int32_t 
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (i < nload)
-#pragma unroll
-                for (int q = 0; q < ng; q++)
-                    raw[q][i] = *reinterpret_cast<const u32x4 *>(M + (size_t)cells[i] * 4 * fcount(P) + S0 +
-                                                                 (g0 + q) * PE + sub * E);
+                static_for<0, ng>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value, at = S0 + L::at(g0 + q) * PE;
+                    raw[q][i] = *reinterpret_cast<const u32x4 *>(M + (size_t)cells[i] * 4 * fcount(P) + at + sub * E);
+                });
         static_for<0, ng>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
+            constexpr int q = decltype(qc)::value, at = S0 + L::at(g0 + q) * PE;
             __builtin_amdgcn_wave_barrier();  // the rows are this wavefront's own: LDS keeps its order
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -1590,15 +1631,12 @@ __device__ __forceinline__ void m2p_load(const R *__restrict__ M, const int32_t 
                 constexpr int un = decltype(uc)::value;
                 const u32x4 w = W.stage[m2p_unit(row, un)];
                 static_for<0, E>([&](auto ec) {
-                    constexpr int e = decltype(ec)::value, k = S0 + (g0 + q) * PE + un * E + e - BASE;
-                    if constexpr (k >= 0 && k < NK) {
-                        constexpr int n = XL<P>::deg(k), m = (k >> 1) - fidx(n, 0);
-                        if constexpr (m >= MA && m <= MB && !(m == 0 && (k & 1))) {
-                            if constexpr (sizeof(R) == 4) {
-                                c[k] = __uint_as_float(w[e]);
-                            } else {
-                                c[k] = __longlong_as_double(((long long)w[2 * e + 1] << 32) | w[2 * e]);
-                            }
+                    constexpr int e = decltype(ec)::value, k = at + un * E + e - BASE;
+                    if constexpr (L::has(k)) {
+                        if constexpr (sizeof(R) == 4) {
+                            c[k] = __uint_as_float(w[e]);
+                        } else {
+                            c[k] = __longlong_as_double(((long long)w[2 * e + 1] << 32) | w[2 * e]);
                         }
                     }
                 });
@@ -1637,9 +1675,10 @@ __device__ __forceinline__ double m2p_fold(const f64x4 &D)
 // with A the lanes' values and B selecting the target's column, so that the 64 lanes of a target are
 // summed in FP64 on the matrix cores beside the vector work (a cross-lane sum in the vector unit
 // takes 36 instructions a target). OUT: which sums it writes (1: u, 2: v, 3: both), added to the
-// pass before it where MA > 0.
+// pass before it where MA > 0. first: no pass of this chunk has loaded the targets yet (a single tile
+// of them stays in W).
 template <int P, int Q, int QV, int BASE, int MA, int OUT, class R>
-__device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, const R *__restrict__ M, M2pWave &W)
+__device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, const R *__restrict__ M, M2pWave &W, bool first = true)
 {
     constexpr int MB = m2p_last_col<Q, QV, R>(MA);
     const int lane = threadIdx.x & 63;
@@ -1651,7 +1690,7 @@ __device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, 
     for (int tb = T.tb; tb < T.te; tb += 16) {
         const int nt = min(16, T.te - tb);
         __builtin_amdgcn_wave_barrier();
-        if (lane < 16) {
+        if (lane < 16 && (first || T.te - T.tb > 16)) {
             const int t = tb + min(lane, nt - 1);
             const double4 y = T.pos[t];
             W.tx[lane][0] = y.x;
@@ -1683,7 +1722,7 @@ __device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, 
             if (lane < nt) *o = MA ? *o + fu : fu;
         }
     }
-    if constexpr (MB < Q) m2p_pass<P, Q, QV, BASE, MB + 1, OUT, R>(l, T, M, W);
+    if constexpr (MB < Q) m2p_pass<P, Q, QV, BASE, MB + 1, OUT, R>(l, T, M, W, false);
 }
 
 // One chunk of at most 64 list entries [b, b + n) against the task's targets, to degree Q (QV for the
@@ -1711,7 +1750,7 @@ __device__ __forceinline__ void m2p_chunk(int b, int n, const M2pTargets &T, con
         m2p_pass<P, Q, QV, 0, 0, 3, R>(l, T, M, W);
     } else {
         m2p_pass<P, Q, -1, 0, 0, 1, R>(l, T, M, W);
-        m2p_pass<P, QV, -1, 2 * fcount(P), 0, 2, R>(l, T, M, W);
+        m2p_pass<P, QV, -1, 2 * fcount(P), 0, 2, R>(l, T, M, W, false);
     }
 }
 

@@ -40,3 +40,26 @@ def test_far_field_at_task_edges(cells, leaf, low, order):
         bound = (1e-10, 1e-10) if prec == "fp64" else (1e-4, 1e-2)
         assert err[0] <= bound[0] and err[1] <= bound[1], (prec, err)
         g.close()
+
+
+@pytest.mark.gpu
+def test_order_10_costs_its_operations():
+    """In FP64 an order-10 cell takes 1.5 times the operations of an order-8 one and, its sets not
+    fitting the registers, two passes per set. Its M2P measures 1.75 times the time; with unequal parts
+    that spill, and pieces fetched that a pass does not use, 2.7 times."""
+    m = HostMesh.cuboid((180.0, 150.0, 18.0), (60, 50, 6), jitter=0.1, seed=5)
+    m.prepare({"volume": dict(Ms=8e5)})
+    rng = np.random.default_rng(1)
+    u = np.array([1.0, 0.4, 0.0]) + rng.uniform(-0.2, 0.2, size=(m.n_nodes, 3))
+    t = {}
+    for order in (8, 10):
+        g = Engine(m.mesh, demag="fmm", fmm_order=order, profile=True)
+        g.set_state(nv.FG_BOTH, u=u / np.linalg.norm(u, axis=1, keepdims=True))
+        g.calc_demag()
+        g.reset_kernel_stats()
+        for _ in range(10):
+            g.calc_demag()
+        n, ms = g.kernel_stats()["fmm_m2p"]
+        t[order] = ms / n
+        g.close()
+    assert t[10] <= 2.2 * t[8], t
