@@ -1561,6 +1561,14 @@ constexpr int m2p_last_col(int ma)
 // row r sits at 4 r + (u ^ (r / 4) % 4): sixteen lanes cover all 64 banks in the writes (four rows)
 // and in the reads (one unit of sixteen rows).
 __device__ __forceinline__ int m2p_unit(int row, int u) { return 4 * row + (u ^ ((row >> 2) & 3)); }
+// Between a lane's writes of M2pWave and other lanes' reads, and before it is written again: a wavefront's
+// LDS operations keep their order, so only the compiler has to be held to it.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
 struct M2pWave {
     u32x4 stage[64 * 4];
     double tx[16][3];  // the tile's targets and their octants
@@ -1622,11 +1630,11 @@ __device__ __forceinline__ void m2p_load(const R *__restrict__ M, const int32_t 
                 });
         static_for<0, ng>([&](auto qc) {
             constexpr int q = decltype(qc)::value, at = S0 + L::at(g0 + q) * PE;
-            __builtin_amdgcn_wave_barrier();  // the rows are this wavefront's own: LDS keeps its order
+            wave_lds_sync();
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 if (i < nload) W.stage[m2p_unit(16 * i + (lane >> 2), sub)] = raw[q][i];
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             static_for<0, 4>([&](auto uc) {
                 constexpr int un = decltype(uc)::value;
                 const u32x4 w = W.stage[m2p_unit(row, un)];
@@ -1689,7 +1697,7 @@ __device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, 
 #pragma unroll 1
     for (int tb = T.tb; tb < T.te; tb += 16) {
         const int nt = min(16, T.te - tb);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         if (lane < 16 && (first || T.te - T.tb > 16)) {
             const int t = tb + min(lane, nt - 1);
             const double4 y = T.pos[t];
@@ -1698,7 +1706,7 @@ __device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, 
             W.tx[lane][2] = y.z;
             W.toct[lane] = T.oct[t];
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         f64x4 Du = {0, 0, 0, 0}, Dv = {0, 0, 0, 0};
 #pragma unroll 1
         for (int t0 = 0; t0 < nt; t0 += l.ncopy) {
@@ -1716,7 +1724,8 @@ __device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, 
         double2 *d = T.part + (tb - T.tb) + lane;
         if constexpr (OUT == 3) {
             const double fv = m2p_fold(Dv);
-            if (lane < nt) *d = MA ? make_double2(d->x + fu, d->y + fv) : make_double2(fu, fv);
+            static_assert(MA == 0 && MB == Q, "both sets only where one pass holds them");
+            if (lane < nt) *d = make_double2(fu, fv);
         } else {
             double *o = OUT == 1 ? &d->x : &d->y;
             if (lane < nt) *o = MA ? *o + fu : fu;
