@@ -1707,23 +1707,39 @@ __device__ __forceinline__ void m2p_pass(const M2pLane &l, const M2pTargets &T, 
             W.toct[lane] = T.oct[t];
         }
         wave_lds_sync();
-        f64x4 Du = {0, 0, 0, 0}, Dv = {0, 0, 0, 0};
+        // A value that is not finite reaches the sums of the tile's other targets, as 0 times it: then the
+        // tile runs again, one target at a time. The test costs M2P 1 to 2 %.
+        double fu = 0, fv = 0;
+        unsigned mask = l.mask;
+        int t0 = 0, t1 = nt, only = -1;
 #pragma unroll 1
-        for (int t0 = 0; t0 < nt; t0 += l.ncopy) {
-            const int t = t0 + l.copy, tc = min(t, nt - 1);
-            const R x = (R)((W.tx[tc][0] - c.x) * c.w), y = (R)((W.tx[tc][1] - c.y) * c.w),
-                    z = (R)((W.tx[tc][2] - c.z) * c.w);
-            const bool on = t < nt && ((l.mask >> W.toct[tc]) & 1);
-            R su, sv;
-            m2p_cell<Q, QV, MA, MB, R>(cu, cv, x, y, z, su, sv);
-            const double sel = (lane & 15) == tc ? 1.0 : 0.0;
-            Du = Mfma<double>::mma(on ? (double)su * c.w : 0.0, sel, Du);
-            if constexpr (MA <= QV) Dv = Mfma<double>::mma(on ? (double)sv * c.w : 0.0, sel, Dv);
+        while (true) {
+            f64x4 Du = {0, 0, 0, 0}, Dv = {0, 0, 0, 0};
+#pragma unroll 1
+            for (; t0 < t1; t0 += l.ncopy) {
+                const int t = t0 + l.copy, tc = min(t, nt - 1);
+                const R x = (R)((W.tx[tc][0] - c.x) * c.w), y = (R)((W.tx[tc][1] - c.y) * c.w),
+                        z = (R)((W.tx[tc][2] - c.z) * c.w);
+                const bool on = t < nt && ((mask >> W.toct[tc]) & 1);
+                R su, sv;
+                m2p_cell<Q, QV, MA, MB, R>(cu, cv, x, y, z, su, sv);
+                const double sel = (lane & 15) == tc ? 1.0 : 0.0;
+                Du = Mfma<double>::mma(on ? (double)su * c.w : 0.0, sel, Du);
+                if constexpr (MA <= QV) Dv = Mfma<double>::mma(on ? (double)sv * c.w : 0.0, sel, Dv);
+            }
+            const double gu = m2p_fold(Du), gv = OUT == 3 ? m2p_fold(Dv) : 0.0;
+            if (only < 0 || (lane & 15) == only) {
+                fu = gu;
+                fv = gv;
+            }
+            if (only < 0 && !__any(!__builtin_isfinite(gu) || !__builtin_isfinite(gv))) break;
+            if (++only == nt) break;
+            t0 = only & ~(l.ncopy - 1);
+            t1 = t0 + 1;
+            mask = l.copy == only - t0 ? l.mask : 0u;
         }
-        const double fu = m2p_fold(Du);
         double2 *d = T.part + (tb - T.tb) + lane;
         if constexpr (OUT == 3) {
-            const double fv = m2p_fold(Dv);
             static_assert(MA == 0 && MB == Q, "both sets only where one pass holds them");
             if (lane < nt) *d = make_double2(fu, fv);
         } else {
