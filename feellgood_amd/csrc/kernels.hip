@@ -1744,7 +1744,7 @@ __global__ __launch_bounds__(BLOCK) void k_charges(int nbf, int Tm, const int4 *
 
 // 1/sqrt(x) in FP64: the hardware approximation (about 24 correct bits) and one third-order step
 // y (1 + e/2 + 3 e^2 / 8), e = 1 - x y^2, whose error 5 e^3 / 16 is below the rounding: five
-// operations against the IEEE square root and division sequences (about 30). x > 0.
+// operations against the IEEE square root and division sequences (about 30). Not a number at x = 0.
 __device__ inline double rsqrt_f64(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
@@ -1846,6 +1846,22 @@ __global__ __launch_bounds__(BLOCK) void k_p2p_direct(int N, int64_t S, int nspl
 #pragma unroll
     for (int h = 0; h < TPT; h++) {
         const int i = n0 + h * BLOCK + (int)threadIdx.x;
+        if (!(isfinite(pu[h]) && isfinite(pv[h]))) {
+            // a source at the node itself, where rsqrt_f64 gives no number: the share again with the
+            // IEEE sequences (infinite, or no number where there is no charge)
+            pu[h] = pv[h] = 0;
+#pragma unroll 1
+            for (int64_t k = k0; k < k1; k++) {
+                const int64_t s = k < la ? a0 + k : b0 + (k - la);
+                if (mixed && !((s >= r[h].x && s < r[h].y) || (s >= r[h].z && s < r[h].w))) continue;
+                const double4 y = spos[s];
+                const double2 qq = q[s];
+                const double dx = xi[h].x - y.x, dy = xi[h].y - y.y, dz = xi[h].z - y.z;
+                const double ir = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
+                pu[h] += qq.x * ir;
+                pv[h] += qq.y * ir;
+            }
+        }
         if (i < N) part[(size_t)sp * N + i] = make_double2(pu[h], pv[h]);
     }
 }

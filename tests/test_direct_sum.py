@@ -83,3 +83,46 @@ def test_direct_sum_batch(sizes):
     off, _ = g.layout()
     for k, (m, u) in enumerate(zip(ms, us)):
         check(m, u, phi[off[k]:off[k + 1]])
+
+
+def touching_tets(n_pairs):
+    """Pairs of tetrahedra whose second one has a corner at the first one's centroid, a Gauss point (both
+    exact in binary: the centroid takes a quarter of each corner), far apart from one another."""
+    pos, tets = [], []
+    for k in range(n_pairs):
+        o = np.array([0.0, 0.0, 64.0 * k])
+        tets += [np.arange(4) + 8 * k, np.arange(4) + 8 * k + 4]
+        pos += [o, o + [4, 0, 0], o + [0, 4, 0], o + [0, 0, 4], o + [1, 1, 1], o + [9, 1, 1], o + [1, 9, 1], o + [1, 1, 9]]
+    pos, tets = np.array(pos, float) * 2.0**-30, np.array(tets, np.int32)
+    treg, vol, surf = np.zeros(len(tets), np.int32), (nv.VolumeRegion * 1)(), (nv.SurfaceRegion * 1)()
+    vol[0].Ms, vol[0].Ae, vol[0].alpha = 8e5, 1e-11, 0.1
+    m = nv.Mesh()
+    m.n_nodes, m.n_tets, m.n_tris, m.n_vol_regions, m.n_surf_regions = len(pos), len(tets), 0, 1, 1
+    m.pos = pos.ctypes.data_as(C.POINTER(C.c_double))
+    m.tet_nodes, m.tet_region = (x.ctypes.data_as(C.POINTER(C.c_int32)) for x in (tets, treg))
+    m.vol, m.surf = C.cast(vol, C.POINTER(nv.VolumeRegion)), C.cast(surf, C.POINTER(nv.SurfaceRegion))
+    return m, (pos, tets, treg, vol, surf)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_pairs,batch", [(2, 1), (80, 1), (2, 3)])
+def test_source_at_a_node(n_pairs, batch):
+    """A node of a body that overlaps another one can lie on a Gauss point: its potential is infinite, as
+    the plain sum has it (no number without charge), and the other nodes' are not touched."""
+    m, own = touching_tets(n_pairs)
+    u = unit(m.n_nodes, 4)
+    v = unit(m.n_nodes, 5)
+    if n_pairs > 2:
+        v[8:16] = 0  # no charge of v at the second pair's node
+    p = oracle.Problem(m, tol=1e-10, max_iter=100)
+    p.set_state(nv.FG_BOTH, u=u, v=v)
+    p.calc_demag()
+    g = Engine.batch([m] * batch) if batch > 1 else Engine(m)
+    g.set_state(nv.FG_BOTH, u=np.tile(u, (batch, 1)), v=np.tile(v, (batch, 1)))
+    g.calc_demag()
+    at = np.arange(4, m.n_nodes, 8)
+    for out, ref in zip(g.get_state(nv.FG_NEXT)[2:], p.get_state(nv.FG_NEXT)[2:]):
+        assert not np.isfinite(ref[at]).any() and np.isfinite(np.delete(ref, at)).all()
+        for phi in out.reshape(batch, -1):
+            assert np.array_equal(phi[at], ref[at], equal_nan=True)
+            assert np.allclose(np.delete(phi, at), np.delete(ref, at), rtol=1e-11, atol=1e-12 * np.nanmax(np.abs(np.delete(ref, at))))
