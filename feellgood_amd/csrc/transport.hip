@@ -1039,7 +1039,7 @@ struct fg_spin {
     double tol = 0;
     int32_t max_iter = 0;
     int assemblies = 0;  // assemblies summed in K and L
-    int last_nit = 0;    // iterations of the last solve
+    int last_nit = -1;   // iterations of the last solve, -1 before one and after one that did not converge
     std::vector<fg_spin_volume> vol;
     hipStream_t stream = nullptr;
     DevBufs B;
@@ -1204,10 +1204,12 @@ void spin_run(fg_spin &sp, hipStream_t st, int acc, int zero_failed, fg_solve_in
     k_sp_init<<<1, 64, 0, st>>>(nbv, sp.part, sp.ctl);
     ESCHK(hipGetLastError());
     // chunks of iterations between host reads of the control block, the first one as long as the last
-    // solve took and one more (its loop test); bicg_dir ends by itself after at most max_iter + 1
-    // iterations (the overflow status breaks the one after the max_iter-th)
-    constexpr int CHUNK = 16;
-    int queued = 0, chunk = sp.last_nit > 0 ? sp.last_nit + 1 : CHUNK;
+    // solve that converged took and one more (its loop test), at most FIRST_MAX (a read costs about
+    // one iteration's time, a launch that finds the loop ended 2 us), and none where that one ended at
+    // its first test; bicg_dir ends by itself after at most max_iter + 1 iterations (the overflow
+    // status breaks the one after the max_iter-th)
+    constexpr int CHUNK = 16, FIRST_MAX = 128;
+    int queued = 0, chunk = sp.last_nit < 0 ? CHUNK : sp.last_nit > 0 ? std::min(sp.last_nit + 1, FIRST_MAX) : 0;
     while (true) {
         for (int it = 0; it < chunk; it++) {
             k_sp_p<<<nbv, ESB, 0, st>>>(n3, nbv, sp.ctl, sp.v, sp.r, sp.D, sp.p, sp.ph, sp.part);
@@ -1225,7 +1227,7 @@ void spin_run(fg_spin &sp, hipStream_t st, int acc, int zero_failed, fg_solve_in
         if (queued > sp.max_iter + 2 * CHUNK) throw std::string("spin solver: bicg_dir did not end");
         chunk = CHUNK;
     }
-    sp.last_nit = std::min(sp.h_ctl->nit, sp.max_iter);
+    sp.last_nit = sp.h_ctl->status == FG_ITER_CONVERGED ? sp.h_ctl->nit : -1;
     k_sp_finish<<<nb3, ESB, 0, st>>>(n3, sp.ctl, zero_failed, sp.Vd, sp.x);
     ESCHK(hipGetLastError());
     if (info) {

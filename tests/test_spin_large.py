@@ -1,7 +1,9 @@
 """The spin solver's phases past one pass of their grids (more than 65,536 nodes, 262,144 unknowns):
 diffusion alone on a bar against the closed form of tests/test_spin_accumulation.py, whose P1 error at
 this cell size is below 1e-3; and a second solve, whose first chunk of iterations has the length of the
-first one's, gives the same field."""
+first one's, gives the same field; and a solve after one that failed."""
+import time
+
 import numpy as np
 import pytest
 
@@ -25,3 +27,27 @@ def test_diffusion_on_a_fine_bar():
     assert np.abs(s - ref).max() <= 1e-3 * np.abs(ref).max()
     again, info2 = sp.solve(u, accumulate=False)
     assert info2.iterations == info.iterations and np.array_equal(again, s)
+
+
+@pytest.mark.gpu
+def test_solve_after_a_failed_one():
+    """A solve that ran into its iteration limit (a magnetization a thousand times too long) leaves nothing
+    behind: the next one gives the same field, and takes about as long, as one after a solve that
+    converged; with the failed one's length queued ahead it took ten times as long."""
+    m, own, pos = bar(0.0, cells=(20, 6, 6), ms=(8e5, 8e5))
+    u = np.tile([0.0, 0.0, 1.0], (m.n_nodes, 1))
+    sp = SpinSolver(m, [vol(), vol()], SURF, np.zeros(m.n_nodes), tol=1e-8, max_iter=2000)
+    ref, info = sp.solve(u, accumulate=False)
+    assert info.status == 0 and 40 <= info.iterations <= 200
+    t = {False: [], True: []}
+    for k in range(6):
+        failed = k % 2 == 1
+        if failed:
+            assert sp.solve(1e3 * u, accumulate=False)[1].iterations >= 2000
+        else:
+            sp.solve(u, accumulate=False)
+        t0 = time.perf_counter()
+        s, again = sp.solve(u, accumulate=False)
+        t[failed].append(time.perf_counter() - t0)
+        assert again.iterations == info.iterations and np.array_equal(s, ref)
+    assert min(t[True]) <= 3 * min(t[False]), t
