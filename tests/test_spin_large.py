@@ -31,23 +31,24 @@ def test_diffusion_on_a_fine_bar():
 
 @pytest.mark.gpu
 def test_solve_after_a_failed_one():
-    """A solve that ran into its iteration limit (a magnetization a thousand times too long) leaves nothing
-    behind: the next one gives the same field, and takes about as long, as one after a solve that
-    converged; with the failed one's length queued ahead it took ten times as long."""
+    """A long solve that did not converge (magnetizations far from unit length, of which the longest solve
+    is taken) leaves nothing behind: the next one gives the same field, and takes about as long, as one
+    after a solve that converged. With the failed one's iterations queued ahead of it, empty launches
+    took more than twice its own time."""
     m, own, pos = bar(0.0, cells=(20, 6, 6), ms=(8e5, 8e5))
     u = np.tile([0.0, 0.0, 1.0], (m.n_nodes, 1))
     sp = SpinSolver(m, [vol(), vol()], SURF, np.zeros(m.n_nodes), tol=1e-8, max_iter=2000)
-    ref, info = sp.solve(u, accumulate=False)
-    assert info.status == 0 and 40 <= info.iterations <= 200
+    tries = [(sp.solve(k * u, accumulate=False)[1], k) for k in (30.0, 50.0, 100.0, 200.0, 300.0, 500.0, 1000.0, 2000.0)]
+    long = max((i.iterations, k) for i, k in tries if i.status != 0)
+    assert long[0] >= 150
+    ref, info = sp.solve(0 * u, accumulate=False)
+    assert info.status == 0 and info.iterations < 60
     t = {False: [], True: []}
-    for k in range(6):
+    for k in range(10):
         failed = k % 2 == 1
-        if failed:
-            assert sp.solve(1e3 * u, accumulate=False)[1].iterations >= 2000
-        else:
-            sp.solve(u, accumulate=False)
+        sp.solve(long[1] * u if failed else 0 * u, accumulate=False)
         t0 = time.perf_counter()
-        s, again = sp.solve(u, accumulate=False)
+        s, again = sp.solve(0 * u, accumulate=False)
         t[failed].append(time.perf_counter() - t0)
         assert again.iterations == info.iterations and np.array_equal(s, ref)
-    assert min(t[True]) <= 3 * min(t[False]), t
+    assert min(t[True]) <= 1.5 * min(t[False]), t
