@@ -265,3 +265,21 @@ def test_mixed_precision_fmm_step():
     dm, dmf = np.abs(un["g"] - un["o"]).max(), np.abs(un["g"] - un["f"]).max()
     print(f"step |dm|: mixed against exact {dm:.2e}, against FP64 FMM {dmf:.2e}", flush=True)
     assert dm <= 1e-6 and dmf <= 1e-7, (dm, dmf)
+
+
+@pytest.mark.gpu
+def test_kernel_stats_count_passes():
+    """Each stage of a profiled FMM counts once per pass, also where a stage has several launches or parts
+    (rates are the work of a pass over the time of a count)."""
+    from feellgood_amd.engine import Engine
+    m = film(30, 20, 3)
+    for prec in ("fp64", "mixed"):
+        g = Engine(m.mesh, demag="fmm", fmm_order=8, fmm_leaf=16, precision=prec, profile=True)
+        assert g.fmm_info()["leaf_level"] >= 5
+        g.set_state(nv.FG_BOTH, u=np.tile([1.0, 0.0, 0.0], (m.n_nodes, 1)))
+        for _ in range(3):
+            g.calc_demag()
+        n = {k: v[0] for k, v in g.kernel_stats().items() if k.startswith("fmm_")}
+        assert set(n) == {"fmm_p2m", "fmm_m2m", "fmm_near", "fmm_m2l", "fmm_l2l", "fmm_m2p", "fmm_finish"}
+        assert set(n.values()) == {3}, n
+        g.close()
