@@ -202,7 +202,9 @@ def kernel_model(name, n):
         "node_assemble": ("hbm", 332 * N + 144 * T),
         "element": ("hbm", 284 * T + 64 * N),
         "update": ("hbm", 164 * N),
-        "charges": ("hbm", 16 * T + 96 * T + 4 * T + 80 * T + 64 * N + 16 * F + 128 * F + 64 * F + 48 * F + 96 * N),
+        # geometry, states and vertex corrections, and the charges of every source (their weights, ranks
+        # and values; an FMM context writes the element values instead)
+        "charges": ("hbm", 116 * T + 96 * N + 192 * F + 160 * T + 96 * F),
         # the tetrahedra's energies, the triangles', and the nodes' largest angle with the evolution
         "energy_angle_evolution": ("hbm", 16 * T + 136 * T + 4 * T + 64 * N + 136 * F + 4 * nnz + 128 * N),
         "p2p_direct": ("valu64", 2 * 10.0 * N * S),
@@ -214,6 +216,7 @@ def kernel_model(name, n):
         pf = far_degree(p, n.get("far_order"), n.get("precision"))
         pv = V_DEGREE if mixed else p
         models.update({
+            "charges": ("hbm", 116 * T + 96 * N + 192 * F + 16 * T + 48 * F),
             # coefficient rows (FP32 in the mixed mode) + shared columns + element values read once
             # + per-target I/O
             "fmm_near": ("hbm", (4 if mixed else 8) * f["near_coefs"] + 4 * f["near_columns"] + 16 * (T + 3 * F)

@@ -1432,8 +1432,9 @@ __global__ __launch_bounds__(256) void k_nf_apply(int ntl, const int32_t *__rest
 // parts, and the azimuthal factors are applied once per column (Horner's rule in e). Per (target,
 // cell) 228 instructions at degrees 8 / 4 in FP32 (350 with complex recurrences); in FP64 440 in two
 // passes, one per set (447 with complex recurrences and both sets at once).
-// Bound by VALU issue (FP32: 77 % of it on the 2M-tetrahedron film), in FP64 also by the latency of
-// the expansions' loads at two wavefronts per SIMD. M2P pass, with the row layout and with this one:
+// Bound by VALU issue (on the 2M-tetrahedron film the units are busy 93 % of the time in FP32, 64 % in
+// FP64), in FP64 also by the latency of the expansions' loads at two wavefronts per SIMD. M2P pass, with
+// the row layout and with this one:
 // 2M film mixed 1.90 -> 0.85 ms, 490k film FP64 0.95 -> 0.65 ms, 48k cube FP64 0.39 -> 0.09 ms,
 // 64 dots mixed 0.50 -> 0.13 ms.
 

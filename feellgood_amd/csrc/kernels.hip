@@ -380,10 +380,11 @@ __global__ __launch_bounds__(BLOCK) void k_node_assemble(
 //      would leave most CUs idle and each row one serial chain of gathers;
 //   1: a lane per row, four stencil entries in flight, while the rows fit one pass of the grid: bound
 //      by the latency of the gathers;
-//   0: a lane per row, one entry after another: with many wavefronts per SIMD to hide the latency the
-//      fewer registers and instructions win.
-// Per product, the old form (0) and the new one: 8.7 -> 5.3 us on 9,261 nodes (4), 16.1 -> 14.0 us on
-// 98,784 (1); 39.2 (0) against 41.5 (1) us on 392,784.
+//   0: a lane per row, one entry after another, with passes over the rows: many wavefronts per SIMD hide
+//      the latency, and the fewer registers cost nothing.
+// The two products of an iteration (v, t), form 0 and the form taken: 11.3, 12.2 -> 4.4, 5.1 us on 9,261
+// nodes (4), 13.6, 16.3 -> 11.8, 14.4 us on 98,784 (1); on 392,784 form 0 takes 43.7, 46.9 and form 1
+// 43.2, 45.0.
 __device__ constexpr int form_lanes(int form) { return form == 4 ? 4 : 1; }
 // The first row of this thread and the rows between its passes: stencil kernels (lane sub of the
 // row's lanes) and vector kernels (one lane per row; lanes past the block's rows have none).
